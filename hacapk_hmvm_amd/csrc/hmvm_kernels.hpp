@@ -21,6 +21,7 @@
 
 #include <type_traits>
 
+#include "hmvm_elem.hpp"
 #include "hmvm_plan.hpp"
 
 namespace hmvm {
@@ -36,23 +37,6 @@ template <typename S>
 struct AccOf { using T = float; };
 template <>
 struct AccOf<double> { using T = double; };
-
-// Element type of the slot buffers (per-tile sums): the tile's accumulation
-// type.  A lane-per-row tile's FP32 sum is stored exactly; a column-split
-// tile adds its groups' FP32 partials in FP64 and stores that sum rounded
-// once to FP32.  The segment sums that add slots into t and y accumulate in
-// FP64.  FP32 and BF16 storage thus move half the slot bytes of FP64.
-template <typename S>
-struct SlotOf { using T = float; };
-template <>
-struct SlotOf<double> { using T = double; };
-
-// Element type of the multi-RHS vectors the tiles read (the copy of X and
-// t): the MFMA operand type, i.e. FP64, FP32, and for BF16 storage the BF16
-// bits of the FP32-rounded value (round to nearest even twice, as the
-// operand conversion of the FP32 value would do).
-template <typename S>
-struct VecOf { using T = S; };
 
 // BF16 values are kept as raw uint16_t bit patterns.
 __device__ __forceinline__ double load_val(const double *p) { return *p; }
@@ -136,7 +120,7 @@ __device__ __forceinline__ float panel_scale(const PanelDesc &pd, const float *_
 struct TileOut {
   void *out;  // slots: SlotOf<S>::T of the launch's storage S
   const int32_t *tmap;
-  void *tout;  // t: double (one right-hand side), VecOf<S>::T (several)
+  void *tout;  // t: double
   const double *mscale;
 };
 
@@ -618,8 +602,8 @@ __global__ __launch_bounds__(256) HMVM_TILE_OCCUPANCY void tile_kernel_timed(con
 // both factor scales of entry i's leaf (a1 = factor_of, a2 = the next id).
 // Entries past nch reload the last slot and add nothing (unguarded loads).
 // The one-vector t sum has a descriptor per entry (int2, entry = index); the
-// multi-RHS one lists only the entries no stage-1 row map writes (int4, entry
-// = d.z).
+// multi-RHS one lists only the entries no stage-1 group writes (int4, entry =
+// d.z).
 template <bool kScaled, typename P>
 __device__ __forceinline__ double tsum_entry(int i, const int2 d, const P *__restrict__ buf,
                                              const int32_t *__restrict__ factor_of,
@@ -832,561 +816,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(S) =
       __hip_atomic_store(&ctr->xleft[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-}
-
-// ---- several right-hand sides: MFMA tiles --------------------------------
-// Y (nd x nrhs, row-major) += A X.  A tile's output is nrows x nrhs; the
-// right-hand sides go in 16-wide blocks (NB = nrhs / 16):
-//   FP64 storage: v_mfma_f64_16x16x4_f64   (K = 4, FP64 accumulate)
-//   FP32 storage: v_mfma_f32_16x16x4_f32   (K = 4, FP32 accumulate)
-//   BF16 storage: v_mfma_f32_16x16x16_bf16 (K = 16, vector entries rounded to
-//                 BF16 after the factor scale is applied, FP32 accumulate)
-// Operand layouts (wave64): A lane l holds row l%16 of K-slice l/16 (one
-// column for K = 4, four consecutive columns for K = 16), B lane l holds rhs
-// l%16 of the same K-slice; the 16x16 result gives lane l four rows of rhs
-// l%16: 4*(l/16)+v for the FP32 and BF16 instructions, l/16+4v for the FP64
-// one (Mfma<S>::row).
-// Matrix loads are the 16-byte lane loads of the one-vector path (V = 2, 4
-// or 8 consecutive rows of one column, aligned as there): lane l loads rows
-// V*(l%16) .. V*(l%16)+V-1 of a chunk of 16V rows, so one load feeds V MFMAs,
-// MFMA m taking row V*i+m of the chunk as its row i.  The wave walks the tile
-// in passes of CH chunks, and per pass the panels' columns in batches of KB
-// K-steps: all loads of a batch (matrix, and the vector entries shared by the
-// CH chunks) are issued before its MFMAs.  Loads are bounded like the
-// one-vector path's (lane groups < lanes per column, columns < ncols), so no
-// access leaves the panel; rows outside the tile only feed result rows that
-// are not stored.
-typedef double mf_d4 __attribute__((ext_vector_type(4)));
-typedef float mf_f4 __attribute__((ext_vector_type(4)));
-typedef short mf_s4 __attribute__((ext_vector_type(4)));
-
-template <typename S>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  static constexpr int K = 4;
-  using Acc = mf_d4;
-  using Op = double;
-  // result element v of lane l: row l/16 + 4v (measured on gfx950)
-  __device__ static __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
-};
-template <>
-struct Mfma<float> {
-  static constexpr int K = 4;
-  using Acc = mf_f4;
-  using Op = float;
-  // result element v of lane l: row 4(l/16) + v
-  __device__ static __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
-};
-template <>
-struct Mfma<uint16_t> {
-  static constexpr int K = 16;
-  using Acc = mf_f4;
-  using Op = mf_s4;
-  __device__ static __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
-};
-
-__device__ __forceinline__ mf_d4 mfma_step(double a, double b, mf_d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ mf_f4 mfma_step(float a, float b, mf_f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ mf_f4 mfma_step(mf_s4 a, mf_s4 b, mf_f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ short bf16_bits(float f) {
-  const uint32_t b = __float_as_uint(f);
-  return (short)(uint16_t)((b + 0x7FFFu + ((b >> 16) & 1u)) >> 16);
-}
-
-// NB consecutive elements at p (p aligned to NB elements): one 4-, 8- or
-// 16-byte access per 16 bytes.
-__device__ __forceinline__ double from_bf16(uint32_t b) { return (double)__uint_as_float(b << 16); }
-__device__ __forceinline__ uint32_t to_bf16(double v) { return (uint32_t)(uint16_t)bf16_bits((float)v); }
-
-template <int NB, typename T>
-__device__ __forceinline__ void load_n(const T *__restrict__ p, double (&v)[NB]) {
-  if constexpr (std::is_same<T, uint16_t>::value) {  // BF16 bits
-    if constexpr (NB == 1) {
-      v[0] = from_bf16(p[0]);
-    } else if constexpr (NB == 2) {
-      const uint32_t w = *reinterpret_cast<const uint32_t *>(p);
-      v[0] = from_bf16(w & 0xFFFFu);
-      v[1] = from_bf16(w >> 16);
-    } else {
-#pragma unroll
-      for (int c = 0; c < NB; c += 4) {
-        const uint2 w = *reinterpret_cast<const uint2 *>(p + c);
-        v[c] = from_bf16(w.x & 0xFFFFu);
-        v[c + 1] = from_bf16(w.x >> 16);
-        v[c + 2] = from_bf16(w.y & 0xFFFFu);
-        v[c + 3] = from_bf16(w.y >> 16);
-      }
-    }
-  } else if constexpr (NB == 1) {
-    v[0] = (double)p[0];
-  } else if constexpr (sizeof(T) == 8) {
-#pragma unroll
-    for (int c = 0; c < NB; c += 2) {
-      const double2 w = *reinterpret_cast<const double2 *>(p + c);
-      v[c] = w.x;
-      v[c + 1] = w.y;
-    }
-  } else if constexpr (NB == 2) {
-    const float2 w = *reinterpret_cast<const float2 *>(p);
-    v[0] = (double)w.x;
-    v[1] = (double)w.y;
-  } else {
-#pragma unroll
-    for (int c = 0; c < NB; c += 4) {
-      const float4 w = *reinterpret_cast<const float4 *>(p + c);
-      v[c] = (double)w.x;
-      v[c + 1] = (double)w.y;
-      v[c + 2] = (double)w.z;
-      v[c + 3] = (double)w.w;
-    }
-  }
-}
-template <int NB, typename T>
-__device__ __forceinline__ void store_n(T *__restrict__ p, const double (&v)[NB]) {
-  if constexpr (std::is_same<T, uint16_t>::value) {  // BF16 bits
-    if constexpr (NB == 1) {
-      p[0] = (uint16_t)to_bf16(v[0]);
-    } else if constexpr (NB == 2) {
-      *reinterpret_cast<uint32_t *>(p) = to_bf16(v[0]) | (to_bf16(v[1]) << 16);
-    } else {
-#pragma unroll
-      for (int c = 0; c < NB; c += 4)
-        *reinterpret_cast<uint2 *>(p + c) =
-            uint2{to_bf16(v[c]) | (to_bf16(v[c + 1]) << 16), to_bf16(v[c + 2]) | (to_bf16(v[c + 3]) << 16)};
-    }
-  } else if constexpr (NB == 1) {
-    p[0] = (T)v[0];
-  } else if constexpr (sizeof(T) == 8) {
-#pragma unroll
-    for (int c = 0; c < NB; c += 2) *reinterpret_cast<double2 *>(p + c) = double2{v[c], v[c + 1]};
-  } else if constexpr (NB == 2) {
-    *reinterpret_cast<float2 *>(p) = float2{(float)v[0], (float)v[1]};
-  } else {
-#pragma unroll
-    for (int c = 0; c < NB; c += 4)
-      *reinterpret_cast<float4 *>(p + c) = float4{(float)v[c], (float)v[c + 1], (float)v[c + 2], (float)v[c + 3]};
-  }
-}
-
-// Row `row`, right-hand sides rhs0 .. rhs0+NB-1 of a multi-RHS tile:
-// store_row with rows of nrhs entries (slots and t in the row-major
-// multi-RHS layout), one vector store.
-template <typename S, bool kScaled, int NB>
-__device__ __forceinline__ void store_rows_multi(const TileDesc &td, int row, int rhs0, int nrhs, double (&v)[NB],
-                                                 const TileOut &o, const float *__restrict__ scales) {
-  using Slot = typename SlotOf<S>::T;
-  if (td.map_off < 0) {
-    store_n<NB>(static_cast<Slot *>(o.out) + (int64_t)(td.out_off + row) * nrhs + rhs0, v);
-    return;
-  }
-  const int e = o.tmap[td.map_off + row];
-  if constexpr (kScaled) {
-    const double f = o.mscale[td.map_off + row];
-#pragma unroll
-    for (int c = 0; c < NB; ++c) v[c] *= f;
-  }
-  store_n<NB>(static_cast<typename VecOf<S>::T *>(o.tout) + (int64_t)e * nrhs + rhs0, v);
-}
-
-// Vector entries (col, rhs0 .. rhs0+NB-1) of a panel in the multi-RHS
-// layout, zero past the panel's last column.  The load address is clamped
-// into the panel so that the load is issued unconditionally: a K-step's loads
-// then sit in one basic block with the rest of the batch and are all in
-// flight before the first MFMA (a branch per load makes the compiler wait for
-// each one).  X and T panels read `src` (the caller's choice of X or T); kTP
-// panels sum stage-1 partial slots.
-template <bool kTP, int NB, typename P, typename VT>
-__device__ __forceinline__ void vec_entries_multi(const PanelDesc &pd, const VT *__restrict__ src,
-                                                  const P *__restrict__ TP, int col, int rhs0, int nrhs,
-                                                  double (&v)[NB]) {
-  const int c = col < pd.ncols ? col : pd.ncols - 1;
-  if constexpr (kTP) {
-    const int nch = pd.vec_chunks >> 16, stride = pd.vec_chunks & 0xFFFF;
-#pragma unroll
-    for (int r = 0; r < NB; ++r) v[r] = 0;
-    for (int q = 0; q < nch; ++q) {
-      double w[NB];
-      load_n<NB>(TP + (int64_t)(pd.vec_off + q * stride + c) * nrhs + rhs0, w);
-#pragma unroll
-      for (int r = 0; r < NB; ++r) v[r] += w[r];
-    }
-  } else {
-    load_n<NB>(src + (int64_t)(pd.vec_off + c) * nrhs + rhs0, v);
-  }
-  if (col >= pd.ncols)
-#pragma unroll
-    for (int r = 0; r < NB; ++r) v[r] = 0.0;
-}
-
-// Vector operands of the NB right-hand-side blocks at K-step k0 (times the
-// panel scale).  Block cb, MFMA column j is right-hand side NB*j + cb, so
-// lane l (j = l%16) loads its NB right-hand sides NB*j .. NB*j+NB-1 at once.
-// FP64 and FP32 one entry per block (column k0 + l/16), BF16 four (columns
-// k0 + 4(l/16) + q).
-template <typename S, bool kTP, int NB>
-__device__ __forceinline__ void b_operands(const PanelDesc &pd, const typename VecOf<S>::T *__restrict__ src,
-                                           const typename SlotOf<S>::T *__restrict__ TP, int nrhs, int k0,
-                                           int lane, float scale, typename Mfma<S>::Op (&b)[NB]) {
-  const int rhs0 = NB * (lane & 15);
-  if constexpr (sizeof(S) == 2 && !kTP) {
-    // X and t hold BF16 bits already: one load of NB right-hand sides per
-    // column, zero past the panel's last column, and a dense panel's
-    // power-of-two scale applied exactly (no rounding: the result equals
-    // rounding the scaled FP32 value)
-    using Raw = typename std::conditional<NB == 1, uint16_t,
-                                          typename std::conditional<NB == 2, uint32_t, uint2>::type>::type;
-    Raw raw[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int col = k0 + 4 * (lane >> 4) + q;
-      const int c = col < pd.ncols ? col : pd.ncols - 1;
-      raw[q] = *reinterpret_cast<const Raw *>(src + (int64_t)(pd.vec_off + c) * nrhs + rhs0);
-      if (col >= pd.ncols) raw[q] = Raw{};
-    }
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t h;
-        if constexpr (NB == 1)
-          h = raw[q];
-        else if constexpr (NB == 2)
-          h = cb == 0 ? (raw[q] & 0xFFFFu) : (raw[q] >> 16);
-        else
-          h = ((cb < 2 ? raw[q].x : raw[q].y) >> (16 * (cb & 1))) & 0xFFFFu;
-        if (scale != 1.0f) h = __float_as_uint(__uint_as_float(h << 16) * scale) >> 16;
-        b[cb][q] = (short)(uint16_t)h;
-      }
-  } else if constexpr (sizeof(S) == 2) {
-    double v[4][NB];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) vec_entries_multi<kTP, NB>(pd, src, TP, k0 + 4 * (lane >> 4) + q, rhs0, nrhs, v[q]);
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) b[cb][q] = bf16_bits((float)v[q][cb] * scale);
-  } else {
-    double v[NB];
-    vec_entries_multi<kTP, NB>(pd, src, TP, k0 + (lane >> 4), rhs0, nrhs, v);
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) b[cb] = (S)v[cb];
-  }
-}
-
-// Matrix words of one K-step for one chunk: FP64/FP32 one 16-byte word
-// (column k0 + l/16), BF16 four (columns k0 + 4(l/16) + q).  Columns past the
-// panel's last one read its last column (their vector entries are zero), so
-// every load stays inside the panel and none is conditional.
-template <typename S>
-struct MultiWords {
-  static constexpr int NW = sizeof(S) == 2 ? 4 : 1;
-  typename Wide<S>::T w[NW];
-};
-template <typename S>
-__device__ __forceinline__ void load_words(MultiWords<S> &mw, const S *__restrict__ base, const PanelDesc &pd, int k0,
-                                           int lane) {
-  constexpr int NW = MultiWords<S>::NW;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    const int col = NW == 1 ? k0 + (lane >> 4) : k0 + 4 * (lane >> 4) + q;
-    const int c = col < pd.ncols ? col : pd.ncols - 1;
-    mw.w[q] = load_wide<S, false>(base + (int64_t)c * pd.ld);
-  }
-}
-// A operand of MFMA m (row V*i+m of the chunk as row i) from a chunk's words.
-template <typename S>
-__device__ __forceinline__ typename Mfma<S>::Op a_of(const MultiWords<S> &mw, int m) {
-  if constexpr (sizeof(S) == 2) {
-    mf_s4 a;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const unsigned int u = mw.w[q][m >> 1];
-      a[q] = (short)(unsigned short)((m & 1) ? (u >> 16) : (u & 0xFFFFu));
-    }
-    return a;
-  } else {
-    return mw.w[0][m];
-  }
-}
-
-// Chunks per pass and K-steps per batch, measured at N=101,250 for 16, 32
-// and 64 right-hand sides (chunks and K-steps halved and doubled): FP64 four
-// chunks up to 32 right-hand sides and two for 64 (fewer passes, fewer
-// re-reads of X); FP32 and BF16 two chunks when the accumulators fit 32
-// VGPRs (one for BF16 with 16 right-hand sides); FP64 batches 8 K-steps for
-// 16 right-hand sides and 4 otherwise; FP32 4 for 16 and 32 right-hand
-// sides, 2 for 64 (8 for 32: launch A 0.32 -> 0.42 ms); BF16 2 (32
-// columns; with X and t as BF16 bits, 2 beat 1 by 8% in launch A at 32).
-template <typename S, int NB>
-struct MultiShape {
-  static constexpr int V = Wide<S>::V;
-  static constexpr int ACCW = sizeof(typename Mfma<S>::Acc) / 4;  // VGPRs per accumulator
-  static constexpr int CH = sizeof(S) == 8                ? (NB <= 2 ? 4 : 2)
-                            : (sizeof(S) == 2 && NB == 1) ? 1
-                                                          : (V * NB * ACCW <= 32 ? 2 : 1);
-  static constexpr int KB = sizeof(S) == 8 ? (NB == 1 ? 8 : 4) : sizeof(S) == 4 ? (NB <= 2 ? 4 : 2) : 2;
-};
-
-// One panel of one pass: nl (wave-uniform) live chunks; chunks past the
-// tile's last row run no loads and no MFMAs.  A batch of KB K-steps issues
-// all its loads, then its MFMAs.
-template <typename S, int NB, bool kTP, int CH>
-__device__ __forceinline__ void multi_panel(const PanelDesc &pd, const S *const *base, int nl,
-                                            const typename VecOf<S>::T *__restrict__ src,
-                                            const typename SlotOf<S>::T *__restrict__ TP, float scale, int lane,
-                                            typename Mfma<S>::Acc (&acc)[CH][Wide<S>::V][NB]) {
-  using M = Mfma<S>;
-  constexpr int V = Wide<S>::V, K = M::K, KB = MultiShape<S, NB>::KB, nrhs = 16 * NB;
-  for (int k0 = 0; k0 < pd.ncols; k0 += KB * K) {
-    MultiWords<S> a[KB][CH];
-    typename M::Op b[KB][NB];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-      for (int ch = 0; ch < CH; ++ch)
-        if (ch < nl) load_words<S>(a[kb][ch], base[ch], pd, k0 + kb * K, lane);
-      b_operands<S, kTP, NB>(pd, src, TP, nrhs, k0 + kb * K, lane, scale, b[kb]);
-    }
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int ch = 0; ch < CH; ++ch)
-        if (ch < nl)
-#pragma unroll
-        for (int m = 0; m < V; ++m) {
-          const typename M::Op am = a_of<S>(a[kb][ch], m);
-#pragma unroll
-          for (int cb = 0; cb < NB; ++cb) acc[ch][m][cb] = mfma_step(am, b[kb][cb], acc[ch][m][cb]);
-        }
-  }
-}
-
-// A operand of one K-step for a short tile: row `row` of the tile as MFMA
-// row l%16, one element of column k0 + l/16 (FP32 only).  Rows past the tile
-// and columns past the panel read the tile's last row / the panel's last
-// column: such rows are not stored, and such columns meet zero vector entries.
-template <typename S>
-__device__ __forceinline__ S a_narrow(const S *__restrict__ vals, const PanelDesc &pd, int row, int nrows, int k0,
-                                      int lane) {
-  const int col = k0 + (lane >> 4);
-  const int c = col < pd.ncols ? col : pd.ncols - 1;
-  const int r = row < nrows ? row : nrows - 1;
-  return vals[pd.val_off + r + (int64_t)c * pd.ld];
-}
-
-template <typename S, int NB, int NL, bool kTP, int CH>
-__device__ __forceinline__ void multi_panel_narrow(const PanelDesc &pd, const S *__restrict__ vals, int nrows,
-                                                   const typename VecOf<S>::T *__restrict__ src,
-                                                   const typename SlotOf<S>::T *__restrict__ TP, float scale, int lane,
-                                                   typename Mfma<S>::Acc (&acc)[CH][NB]) {
-  using M = Mfma<S>;
-  constexpr int K = M::K, KB = MultiShape<S, NB>::KB, nrhs = 16 * NB;
-  for (int k0 = 0; k0 < pd.ncols; k0 += KB * K) {
-    typename M::Op a[KB][NL], b[KB][NB];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-      for (int ch = 0; ch < NL; ++ch) a[kb][ch] = a_narrow<S>(vals, pd, 16 * ch + (lane & 15), nrows, k0 + kb * K, lane);
-      b_operands<S, kTP, NB>(pd, src, TP, nrhs, k0 + kb * K, lane, scale, b[kb]);
-    }
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int ch = 0; ch < NL; ++ch)
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) acc[ch][cb] = mfma_step(a[kb][ch], b[kb][cb], acc[ch][cb]);
-  }
-}
-
-// Short FP32 tiles (at most 32 rows): MFMA row i is tile row 16*ch + i, so a
-// tile of r rows runs ceil(r/16) MFMAs per K-step and right-hand-side block
-// instead of 4, with 4-byte element loads.  Measured at N=101,250 with 32
-// right-hand sides: faster for FP32; slower for FP64 (8-byte loads, only
-// two MFMAs saved) and BF16 (four strided 2-byte loads per lane), which keep
-// the 16-byte path.
-template <typename S, bool kScaled, int NB, bool kHasTP>
-__device__ __forceinline__ void multi_tile_narrow(const TileDesc &td, const PanelDesc *__restrict__ panels,
-                                                  const S *__restrict__ vals,
-                                                  const typename VecOf<S>::T *__restrict__ X,
-                                                  const typename VecOf<S>::T *__restrict__ T,
-                                                  const typename SlotOf<S>::T *__restrict__ TP,
-                                                  const float *__restrict__ scales, const TileOut &o,
-                                                  int lane) {
-  static_assert(sizeof(S) == 4, "the narrow path is FP32 only");
-  using M = Mfma<S>;
-  using Acc = typename M::Acc;
-  constexpr int CH = 2;  // 32 rows
-  constexpr int nrhs = 16 * NB;
-  const int nlive = td.nrows > 16 ? 2 : 1;
-  Acc acc[CH][NB];
-#pragma unroll
-  for (int ch = 0; ch < CH; ++ch)
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) acc[ch][cb] = Acc{0, 0, 0, 0};
-  for (int p = 0; p < td.npanel; ++p) {
-    const PanelDesc pd = panels[td.panel0 + p];
-    float scale = 1.0f;
-    if constexpr (kScaled) scale = panel_scale(pd, scales);
-    const typename VecOf<S>::T *src = pd.vec_sel == kVecX ? X : T;
-    if (kHasTP && pd.vec_sel == kVecTP) {
-      if (nlive == 2) multi_panel_narrow<S, NB, 2, kHasTP>(pd, vals, td.nrows, src, TP, scale, lane, acc);
-      else multi_panel_narrow<S, NB, 1, kHasTP>(pd, vals, td.nrows, src, TP, scale, lane, acc);
-    } else {
-      if (nlive == 2) multi_panel_narrow<S, NB, 2, false>(pd, vals, td.nrows, src, TP, scale, lane, acc);
-      else multi_panel_narrow<S, NB, 1, false>(pd, vals, td.nrows, src, TP, scale, lane, acc);
-    }
-  }
-#pragma unroll
-  for (int ch = 0; ch < CH; ++ch)
-    if (ch < nlive)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * ch + M::row(lane, v);
-        double r[NB];
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[ch][cb][v];
-        if (row < td.nrows) store_rows_multi<S, kScaled, NB>(td, row, NB * (lane & 15), nrhs, r, o, scales);
-      }
-}
-
-// nrhs = 16*NB; one wave per tile.  kHasTP: the plan has panels that sum
-// stage-1 partial slots (the loop for those is compiled only then).
-template <typename S, bool kScaled, int NB, bool kHasTP>
-__global__ __launch_bounds__(256) void tile_multi_kernel(const TileDesc *__restrict__ tiles, int ntiles,
-                                                         const PanelDesc *__restrict__ panels,
-                                                         const S *__restrict__ vals,
-                                                         const typename VecOf<S>::T *__restrict__ X,
-                                                         const typename VecOf<S>::T *__restrict__ T,
-                                                         const typename SlotOf<S>::T *__restrict__ TP,
-                                                         const float *__restrict__ scales, TileOut o) {
-  using M = Mfma<S>;
-  using Acc = typename M::Acc;
-  using Sh = MultiShape<S, NB>;
-  constexpr int V = Sh::V, CH = Sh::CH;
-  constexpr int nrhs = 16 * NB;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int lane = (int)(threadIdx.x & 63);
-  const int tid = (int)blockIdx.x * (int)(blockDim.x >> 6) + wave;
-  if (tid >= ntiles) return;
-  const TileDesc td = tiles[tid];
-  if constexpr (sizeof(S) == 4) {
-    if (td.nrows <= 8 * V) {
-      multi_tile_narrow<S, kScaled, NB, kHasTP>(td, panels, vals, X, T, TP, scales, o, lane);
-      return;
-    }
-  }
-  const int shift = (int)(td.first.val_off % V);
-  const int lpc = (td.nrows + shift + V - 1) / V;  // lane groups (V rows each) of the tile
-  for (int g0 = 0; g0 < lpc; g0 += 16 * CH) {      // pass: CH chunks of 16 lane groups
-    Acc acc[CH][V][NB];
-#pragma unroll
-    for (int ch = 0; ch < CH; ++ch)
-#pragma unroll
-      for (int m = 0; m < V; ++m)
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) acc[ch][m][cb] = Acc{0, 0, 0, 0};
-    // chunks of this pass that hold rows of the tile (wave-uniform)
-    const int nlive = (lpc - g0 + 15) / 16 < CH ? (lpc - g0 + 15) / 16 : CH;
-    int grp[CH];  // lane group each lane loads; lanes past the tile load group 0
-#pragma unroll
-    for (int ch = 0; ch < CH; ++ch) grp[ch] = g0 + 16 * ch + (lane & 15) < lpc ? g0 + 16 * ch + (lane & 15) : 0;
-    for (int p = 0; p < td.npanel; ++p) {
-      const PanelDesc pd = panels[td.panel0 + p];
-      float scale = 1.0f;
-      if constexpr (kScaled) scale = panel_scale(pd, scales);
-      const S *base[CH];
-#pragma unroll
-      for (int ch = 0; ch < CH; ++ch) base[ch] = vals + (pd.val_off - shift) + (int64_t)V * grp[ch];
-      const typename VecOf<S>::T *src = pd.vec_sel == kVecX ? X : T;
-      if (kHasTP && pd.vec_sel == kVecTP)
-        multi_panel<S, NB, kHasTP, CH>(pd, base, nlive, src, TP, scale, lane, acc);
-      else
-        multi_panel<S, NB, false, CH>(pd, base, nlive, src, TP, scale, lane, acc);
-    }
-#pragma unroll
-    for (int ch = 0; ch < CH; ++ch)
-      if (ch < nlive)
-#pragma unroll
-      for (int m = 0; m < V; ++m)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          // result row i of MFMA m: row V*i+m of the chunk, minus the shift;
-          // block cb holds right-hand side NB*(lane%16) + cb
-          const int row = V * (16 * ch + g0 + M::row(lane, v)) + m - shift;
-          double r[NB];
-#pragma unroll
-          for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[ch][m][cb][v];
-          if (row >= 0 && row < td.nrows)
-            store_rows_multi<S, kScaled, NB>(td, row, NB * (lane & 15), nrhs, r, o, scales);
-        }
-  }
-}
-
-// y sum for nrhs right-hand sides: out[i*nrhs+c] = (accumulate ? out : 0) +
-// sum_e buf[(list[e]+i)*nrhs + c], e over entry i's list range in list order
-// (segsum_kernel's sums).  A thread sums W consecutive right-hand sides: W =
-// 16 / sizeof(P) (16-byte slot loads) when out is 16-byte aligned, else 1.
-// Up to U list entries and their slots are in flight at once (the y lists
-// hold 11 to 19 FP64 and 14 to 23 FP32 slots at N=101,250; measured: U = 24
-// for FP64, 16 for FP32).  The slots stay in their own type until summed, so
-// that the guarded loads are all issued before the first wait.
-template <int W, typename P>
-__global__ __launch_bounds__(256) void ysum_multi_kernel(int n, int nrhs, const int2 *__restrict__ rng,
-                                                         const int64_t *__restrict__ list,
-                                                         const P *__restrict__ buf, double *__restrict__ out,
-                                                         int accumulate) {
-  constexpr int U = sizeof(P) == 8 ? 24 : 16;
-  const int nw = nrhs / W;
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)n * nw) return;
-  const int i = (int)(g / nw), c = (int)(g - (int64_t)i * nw) * W;
-  const int2 r = rng[i];
-  const int e1 = r.y;
-  double a[W];
-#pragma unroll
-  for (int w = 0; w < W; ++w) a[w] = 0;
-  using Raw = typename std::conditional<
-      W == 1, P, typename std::conditional<sizeof(P) == 8, double2, float4>::type>::type;
-  static_assert(W == 1 || sizeof(Raw) == 16, "16-byte slot loads");
-  for (int e = r.x; e < e1; e += U) {
-    int64_t l[U];
-    Raw v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) l[u] = e + u < e1 ? list[e + u] : 0;
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = e + u < e1 ? *reinterpret_cast<const Raw *>(buf + (l[u] + i) * nrhs + c) : Raw{};
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool on = e + u < e1;
-      if constexpr (W == 1) {
-        a[0] += on ? (double)v[u] : 0.0;
-      } else if constexpr (W == 2) {
-        a[0] += on ? (double)v[u].x : 0.0;
-        a[1] += on ? (double)v[u].y : 0.0;
-      } else {
-        a[0] += on ? (double)v[u].x : 0.0;
-        a[1] += on ? (double)v[u].y : 0.0;
-        a[2] += on ? (double)v[u].z : 0.0;
-        a[3] += on ? (double)v[u].w : 0.0;
-      }
-    }
-  }
-  double *o = out + (int64_t)i * nrhs + c;
-  if (accumulate) {
-    double prev[W];
-    load_n<W>(o, prev);
-#pragma unroll
-    for (int w = 0; w < W; ++w) a[w] = prev[w] + a[w];
-  }
-  store_n<W>(o, a);
 }
 
 // Achievable-bandwidth probes: a read-only stream (sum) and a copy, each

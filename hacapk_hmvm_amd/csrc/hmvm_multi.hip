@@ -1,0 +1,47 @@
+// hmvm_multi.hip -- launches of the multi-RHS group kernels (hmvm_multi.hpp).
+#include "hmvm_multi.hpp"
+
+namespace hmvm {
+
+namespace {
+template <typename S, int NB>
+void launch(const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
+  constexpr size_t lds = multi_lds_wave<S, NB>();
+  hipLaunchKernelGGL((multi_kernel<S, NB>), dim3(ngroups), dim3(64 * waves), lds * waves, st, a);
+}
+template <typename S>
+void launch_nb(int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
+  if (nrhs == 16)
+    launch<S, 1>(a, ngroups, waves, st);
+  else if (nrhs == 32)
+    launch<S, 2>(a, ngroups, waves, st);
+  else
+    launch<S, 4>(a, ngroups, waves, st);
+}
+}  // namespace
+
+void launch_multi_groups(int storage, int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
+  if (ngroups == 0) return;
+  if (storage == kF64)
+    launch_nb<double>(nrhs, a, ngroups, waves, st);
+  else if (storage == kF32)
+    launch_nb<float>(nrhs, a, ngroups, waves, st);
+  else
+    launch_nb<uint16_t>(nrhs, a, ngroups, waves, st);
+}
+
+void launch_multi_pack(int storage, int n, const MultiPack *recs, const void *vals, const float *scales, void *out,
+                       hipStream_t st) {
+  if (n == 0) return;
+  if (storage == kF64)
+    hipLaunchKernelGGL((multi_pack_kernel<double>), dim3(n), dim3(256), 0, st, recs, (const double *)vals, scales,
+                       (double *)out);
+  else if (storage == kF32)
+    hipLaunchKernelGGL((multi_pack_kernel<float>), dim3(n), dim3(256), 0, st, recs, (const float *)vals, scales,
+                       (float *)out);
+  else
+    hipLaunchKernelGGL((multi_pack_kernel<uint16_t>), dim3(n), dim3(256), 0, st, recs, (const uint16_t *)vals, scales,
+                       (uint16_t *)out);
+}
+
+}  // namespace hmvm

@@ -1,0 +1,474 @@
+// hmvm_multi.hpp -- gfx950 kernels of the products with several right-hand
+// sides (schedule and packed values: hmvm_multi_plan.hpp).
+//
+// Y (nd x nrhs, row-major) (+)= A X, nrhs = 16*NB right-hand sides.
+//   FP64 storage: v_mfma_f64_16x16x4_f64   (K = 4, FP64 accumulate)
+//   FP32 storage: v_mfma_f32_16x16x4_f32   (K = 4, FP32 accumulate)
+//   BF16 storage: v_mfma_f32_16x16x32_bf16 (K = 32, vector entries in BF16,
+//                 FP32 accumulate)
+// Operand layouts (wave64): A lane l holds row l%16 of K-slice l/16, B lane l
+// right-hand side l%16 of the same K-slice (one column for K = 4, eight for
+// K = 32); the 16x16 result gives lane l four rows of column l%16:
+// 4*(l/16)+v for the FP32 and BF16 instructions, l/16+4v for the FP64 one.
+// Which column stands at which k is free as long as both operands agree: the
+// 16 lanes of K-slice g take the KS consecutive columns of slice g of a
+// batch, so a batch is four MFMA steps (FP64, FP32) or one (BF16), and a
+// lane's matrix words are its A operands as loaded.  Block cb, MFMA column j
+// is right-hand side NB*j + cb, so a lane's NB right-hand sides are one
+// vector load.
+#pragma once
+
+#include "hmvm_elem.hpp"
+#include "hmvm_multi_args.hpp"
+
+namespace hmvm {
+
+typedef double mf_d2 __attribute__((ext_vector_type(2)));
+typedef double mf_d4 __attribute__((ext_vector_type(4)));
+typedef float mf_f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 mf_b8 __attribute__((ext_vector_type(8)));
+// X may be 8-byte aligned only; global loads need no more than 4.
+typedef double mf_d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <typename S>
+struct Mfma;
+template <>
+struct Mfma<double> {
+  static constexpr int KS = 4, E = 2, H = 2;
+  using Acc = mf_d4;
+  using Word = mf_d2;  // 16 bytes of a row: E columns
+  __device__ static __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }  // (measured on gfx950)
+};
+template <>
+struct Mfma<float> {
+  static constexpr int KS = 4, E = 4, H = 1;
+  using Acc = mf_f4;
+  using Word = mf_f4;
+  __device__ static __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+template <>
+struct Mfma<uint16_t> {
+  static constexpr int KS = 8, E = 8, H = 1;
+  using Acc = mf_f4;
+  using Word = mf_b8;
+  __device__ static __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+
+__device__ __forceinline__ mf_d4 mfma_step(double a, double b, mf_d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ mf_f4 mfma_step(float a, float b, mf_f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ mf_f4 mfma_step(mf_b8 a, mf_b8 b, mf_f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Halves h (0 low, 1 high) of words a and b as one word {a, b}.
+__device__ __forceinline__ uint32_t pack_half(uint32_t a, uint32_t b, int h) {
+  return __builtin_amdgcn_perm(b, a, h ? 0x07060302u : 0x05040100u);
+}
+union Bf16x8 {
+  uint32_t u[4];
+  mf_b8 v;
+};
+
+// NB consecutive right-hand sides of a vector row, as loaded.
+template <typename V, int NB>
+struct RhsWord;
+template <int NB>
+struct RhsWord<double, NB> {
+  double v[NB];
+};
+template <int NB>
+struct RhsWord<float, NB> {
+  float v[NB];
+};
+template <>
+struct RhsWord<uint16_t, 1> {
+  uint32_t u[1];
+};
+template <int NB>
+struct RhsWord<uint16_t, NB> {
+  uint32_t u[NB / 2];
+};
+// X may be 8-byte aligned only: element-aligned loads.
+template <int NB>
+__device__ __forceinline__ void load_rhs(const double *__restrict__ p, RhsWord<double, NB> &w) {
+  if constexpr (NB == 1) {
+    w.v[0] = p[0];
+  } else {
+#pragma unroll
+    for (int c = 0; c < NB; c += 2) {
+      const mf_d2u d = *reinterpret_cast<const mf_d2u *>(p + c);
+      w.v[c] = d[0];
+      w.v[c + 1] = d[1];
+    }
+  }
+}
+template <int NB>
+__device__ __forceinline__ void load_rhs(const float *__restrict__ p, RhsWord<float, NB> &w) {
+  if constexpr (NB == 1) {
+    w.v[0] = p[0];
+  } else if constexpr (NB == 2) {
+    const float2 d = *reinterpret_cast<const float2 *>(p);
+    w.v[0] = d.x;
+    w.v[1] = d.y;
+  } else {
+    const float4 d = *reinterpret_cast<const float4 *>(p);
+    w.v[0] = d.x;
+    w.v[1] = d.y;
+    w.v[2] = d.z;
+    w.v[3] = d.w;
+  }
+}
+template <int NB>
+__device__ __forceinline__ void load_rhs(const uint16_t *__restrict__ p, RhsWord<uint16_t, NB> &w) {
+  if constexpr (NB == 1) {
+    w.u[0] = p[0];
+  } else if constexpr (NB == 2) {
+    w.u[0] = *reinterpret_cast<const uint32_t *>(p);
+  } else {
+    const uint2 d = *reinterpret_cast<const uint2 *>(p);
+    w.u[0] = d.x;
+    w.u[1] = d.y;
+  }
+}
+
+// What one batch loads: NT row tiles of 16 rows, KS columns a lane.
+template <typename S, int NB, int NT>
+struct MultiLoads {
+  typename Mfma<S>::Word a[NT][Mfma<S>::H];
+  RhsWord<typename VecOf<S>::T, NB> x[Mfma<S>::KS];
+};
+
+// Batches whose loads are in flight at once: two (three and four cost
+// registers and instruction cache and were slower, FP64 0.56 -> 0.65 and BF16
+// 0.188 -> 0.217 ms at N=101,250 with 32 right-hand sides), one where the sums
+// leave no registers for a second.
+template <typename S, int NB>
+constexpr int multi_depth() {
+  return sizeof(S) >= 4 && NB == 4 ? 1 : 2;
+}
+// How a column loop ends when its batches are not a multiple of the depth:
+// with a tail (more code), or with batches of zeros read from the zero page
+// (more products); N=101,250, 32 right-hand sides, tail / zeros: FP64 0.557 /
+// 0.545, FP32 0.331 / 0.354, BF16 0.195 / 0.177 ms; BF16 with 64 at N=50,021
+// 0.122 / 0.130.
+template <typename S, int NB>
+constexpr bool multi_tail() {
+  return sizeof(S) == 4 || (sizeof(S) == 2 && NB == 4);
+}
+
+// Whether the MFMA sums of a few batches are folded into sums of their own:
+// FP32 storage (FP64 sums up to 32 right-hand sides, FP32 for 64: no registers
+// for more), and FP64 storage with 16 right-hand sides, the only case with
+// registers for it.
+// An even share of a group's columns is a longer chain of roundings than a
+// tile of the one-vector launches: without, the error against 64 bits was
+// 2.6e-7 instead of 1.1e-7 at N=4,096 and 5.1e-7 instead of 3.4e-7 at
+// N=101,250; with, FP64 1.1e-7 and 1.3e-7, at 3% of the time.
+template <typename S, int NB>
+constexpr bool multi_fold() {
+  return sizeof(S) == 4 || (sizeof(S) == 8 && NB == 1);
+}
+template <typename S, int NB>
+using MultiSum = typename std::conditional<sizeof(S) == 4 && NB <= 2, mf_d4, typename Mfma<S>::Acc>::type;
+
+// out += the item's columns: D batches of loads in flight, and the slices of
+// the D after those.
+template <typename S, int NB, int NT>
+__device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiItem &it, int lane,
+                                              MultiSum<S, NB> (&out)[NT][NB]) {
+  using M = Mfma<S>;
+  using V = typename VecOf<S>::T;
+  constexpr int KS = M::KS, E = M::E, H = M::H, nrhs = 16 * NB;
+  const int i = lane & 15, g = lane >> 4, nr = it.nrows, nb = it.nbatch;
+  if (nb == 0) return;
+  const MultiSlice *sl = a.slices + it.slice0 + g;
+  // this lane's rows; lanes past the item's rows load its first rows
+  const S *ap = (const S *)a.vals + it.a0 + (int64_t)g * nr * KS;
+  int off[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) off[t] = (16 * t + i < nr ? 16 * t + i : i < nr ? i : 0) * E;
+  const V *X = (const V *)a.X + NB * i, *T = (const V *)a.T + NB * i, *Z = (const V *)a.zero + NB * i;
+  auto load = [&](MultiLoads<S, NB, NT> &l, const MultiSlice s, bool on) {
+    const S *av = on ? ap : (const S *)a.zero;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        l.a[t][h] = __builtin_nontemporal_load(reinterpret_cast<const typename M::Word *>(av + h * nr * E + off[t]));
+    ap += kMultiBatch * KS * nr;
+    const V *xr = ((s.info & kSliceT) ? T : X) + (int64_t)s.v * nrhs;
+    const int n = on ? s.info & 15 : 0;
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
+      load_rhs<NB>(q < n ? xr : Z, l.x[q]);  // the zero columns of a slice meet zeros
+      xr += nrhs;
+    }
+  };
+  typename M::Acc part[multi_fold<S, NB>() ? NT : 1][NB];
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) part[t][cb] = typename M::Acc{0, 0, 0, 0};
+  };
+  auto fold = [&]() {
+    if constexpr (multi_fold<S, NB>()) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) out[t][cb][v] += part[t][cb][v];
+      clear();
+    }
+  };
+  if constexpr (multi_fold<S, NB>()) clear();
+  auto products = [&](const MultiLoads<S, NB, NT> &l) {
+    if constexpr (sizeof(S) == 2) {
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) {
+        Bf16x8 b;
+#pragma unroll
+        for (int q = 0; q < KS; q += 2) b.u[q / 2] = pack_half(l.x[q].u[cb / 2], l.x[q + 1].u[cb / 2], cb & 1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) out[t][cb] = mfma_step(l.a[t][0], b.v, out[t][cb]);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < KS; ++q)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int cb = 0; cb < NB; ++cb)
+            if constexpr (multi_fold<S, NB>())
+              part[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], part[t][cb]);
+            else
+              out[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], out[t][cb]);
+    }
+  };
+  constexpr int D = multi_depth<S, NB>();
+  MultiLoads<S, NB, NT> l[D];
+  MultiSlice s[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) s[d] = sl[kMultiBatch * (d < nb ? d : 0)];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load(l[d], s[d], d < nb);
+    s[d] = sl[kMultiBatch * (D + d < nb ? D + d : 0)];
+  }
+  // No load in these loops is conditional: a branch around one makes the
+  // compiler wait for all loads in flight where its paths meet.
+  if constexpr (multi_tail<S, NB>()) {
+    int b = 0;
+    for (; b + 2 * D <= nb; b += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        products(l[d]);
+        load(l[d], s[d], true);
+        s[d] = sl[kMultiBatch * (b + d + 2 * D < nb ? b + d + 2 * D : 0)];
+      }
+      fold();
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (b + d < nb) products(l[d]);
+      if (b + d + D < nb) load(l[d], s[d], true);
+    }
+    fold();
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (b + d + D < nb) products(l[d]);
+    fold();
+  } else {
+    for (int b = 0; b < nb; b += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        products(l[d]);
+        load(l[d], s[d], b + d + D < nb);
+        s[d] = sl[kMultiBatch * (b + d + 2 * D < nb ? b + d + 2 * D : 0)];
+      }
+      fold();
+    }
+  }
+}
+
+// MFMA tiles whose sums of all waves are added at once: 8 KiB of LDS a wave.
+template <typename S, int NB>
+constexpr int multi_piece() {
+  constexpr int n = 8192 / (256 * NB * (int)sizeof(typename SlotOf<S>::T));
+  return n < 1 ? 1 : n;
+}
+template <typename S, int NB>
+constexpr int multi_lds_wave() {
+  return multi_piece<S, NB>() * 256 * NB * (int)sizeof(typename SlotOf<S>::T);
+}
+
+// W right-hand sides c.. of the t row that entry m of the row map names
+// (BF16: times both factor scales of its leaf).
+template <typename S, int NB, int W>
+__device__ __forceinline__ void store_t(const MultiArgs &a, int m, int c, double (&r)[W]) {
+  const int e = a.tmap[m];
+  if constexpr (sizeof(S) == 2) {
+    const double f = a.mscale[m];
+#pragma unroll
+    for (int k = 0; k < W; ++k) r[k] *= f;
+  }
+  store_n<W>((typename VecOf<S>::T *)a.t_out + (int64_t)e * (16 * NB) + c, r);
+}
+
+// One item of NT row tiles: a partial one's rows go to its slots; the kept
+// one's are added over the waves (in wave order, FP64) and go to y, t or a
+// t slot.
+template <typename S, int NB, int NT>
+__device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it, int lane,
+                                           typename SlotOf<S>::T *lds) {
+  using M = Mfma<S>;
+  using Slot = typename SlotOf<S>::T;
+  constexpr int nrhs = 16 * NB;
+  constexpr int PT = multi_piece<S, NB>() < NT ? multi_piece<S, NB>() : NT;
+  constexpr int W = 16 / (int)sizeof(Slot);  // right-hand sides a thread adds (16 bytes)
+  using Sum = MultiSum<S, NB>;
+  Sum acc[NT][NB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb) acc[t][cb] = Sum{0, 0, 0, 0};
+  multi_columns<S, NB, NT>(a, it, lane, acc);
+  if (it.kind != kItemKept) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = 16 * t + M::row(lane, v);
+        if (row >= it.nrows) continue;
+        double r[NB];
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[t][cb][v];
+        if (it.kind == kItemSlot)
+          store_n<NB>((Slot *)a.slots + ((int64_t)it.out + row) * nrhs + NB * (lane & 15), r);
+        else
+          store_t<S, NB>(a, it.out + row, NB * (lane & 15), r);
+      }
+    return;
+  }
+  const int nthreads = (int)blockDim.x, nw = nthreads >> 6, w = (int)(threadIdx.x >> 6);
+  Slot *mine = lds + w * PT * 256 * NB;
+#pragma unroll
+  for (int t0 = 0; t0 < NT; t0 += PT) {
+    __syncthreads();  // the previous piece is read, and this workgroup's slots are written
+#pragma unroll
+    for (int t = t0; t < t0 + PT && t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double r[NB];
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[t][cb][v];
+        store_n<NB>(mine + ((t - t0) * 16 + M::row(lane, v)) * nrhs + NB * (lane & 15), r);
+      }
+    __syncthreads();
+    const int nt = NT - t0 < PT ? NT - t0 : PT;
+    for (int e = (int)threadIdx.x; e < nt * 16 * nrhs / W; e += nthreads) {
+      const int c = e * W % nrhs, ri = e * W / nrhs;  // right-hand sides c.., tile row ri
+      const int row = 16 * t0 + ri;
+      if (row >= grp.nrows) continue;
+      double s[W];
+#pragma unroll
+      for (int k = 0; k < W; ++k) s[k] = 0;
+      for (int q = 0; q < nw; ++q) {
+        double r[W];
+        load_n<W>(lds + (q * PT * 16 + ri) * nrhs + c, r);
+#pragma unroll
+        for (int k = 0; k < W; ++k) s[k] += r[k];
+      }
+      if (grp.kind == kMultiY) {
+        const int64_t y = (int64_t)grp.out + row;
+        const int2 rg = a.yrng[y];
+        for (int l = rg.x; l < rg.y; ++l) {
+          double r[W];
+          load_n<W>((const Slot *)a.slots + (a.ylist[l] + y) * nrhs + c, r);
+#pragma unroll
+          for (int k = 0; k < W; ++k) s[k] += r[k];
+        }
+        double *o = a.Y + y * nrhs + c;
+        if (a.y16) {
+          if (a.accumulate) {
+            double r[W];
+            load_n<W>(o, r);
+#pragma unroll
+            for (int k = 0; k < W; ++k) s[k] = r[k] + s[k];
+          }
+          store_n<W>(o, s);
+        } else {
+#pragma unroll
+          for (int k = 0; k < W; ++k) o[k] = a.accumulate ? o[k] + s[k] : s[k];
+        }
+      } else if (grp.kind == kMultiT) {
+        store_t<S, NB>(a, grp.out + row, c, s);
+      } else {
+        store_n<W>((Slot *)a.slots + ((int64_t)grp.out + row) * nrhs + c, s);
+      }
+    }
+  }
+}
+
+// multi_item for the row tiles that `rows` rows take.
+template <typename S, int NB>
+__device__ __forceinline__ void multi_item_rows(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it,
+                                                int lane, typename SlotOf<S>::T *lds) {
+  static_assert(kMultiRows <= 64, "row tiles");
+  if (it.nrows <= 16)
+    multi_item<S, NB, 1>(a, grp, it, lane, lds);
+  else if (it.nrows <= 32)
+    multi_item<S, NB, 2>(a, grp, it, lane, lds);
+  else if (it.nrows <= 48)
+    multi_item<S, NB, 3>(a, grp, it, lane, lds);
+  else
+    multi_item<S, NB, 4>(a, grp, it, lane, lds);
+}
+
+template <typename S, int NB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void multi_kernel(MultiArgs a) {
+  extern __shared__ double multi_lds[];
+  using Slot = typename SlotOf<S>::T;
+  const int lane = (int)(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const MultiGroup grp = a.groups[blockIdx.x];
+  const MultiWave wv = a.waves[(int)blockIdx.x * (int)(blockDim.x >> 6) + w];
+  for (int i = 0; i < wv.nitems; ++i)
+    multi_item_rows<S, NB>(a, grp, a.items[wv.item0 + i], lane, (Slot *)multi_lds);
+}
+
+// Packs the values of one record per workgroup (MultiPack); one thread a row
+// of a slice, rows across the lanes on both sides.
+template <typename S>
+__global__ __launch_bounds__(256) void multi_pack_kernel(const MultiPack *__restrict__ recs, const S *__restrict__ vals,
+                                                         const float *__restrict__ scales, S *__restrict__ out) {
+  using M = Mfma<S>;
+  constexpr int KS = M::KS, E = M::E, H = M::H;
+  const MultiPack r = recs[blockIdx.x];
+  const int nsl = (r.cols + KS - 1) / KS + r.pad;
+  float scale = 1.0f;
+  if constexpr (sizeof(S) == 2)
+    if (r.factor >= 0) scale = scales[r.factor];
+  for (int k = (int)threadIdx.x; k < nsl * r.rows; k += (int)blockDim.x) {
+    const int s = k / r.rows, row = k - s * r.rows;
+    const S *src = vals + r.src + row + (int64_t)s * KS * r.ld;
+    S v[KS];
+#pragma unroll
+    for (int q = 0; q < KS; ++q) v[q] = s * KS + q < r.cols ? src[(int64_t)q * r.ld] : S(0);
+    if constexpr (sizeof(S) == 2)  // a power of two: exact
+#pragma unroll
+      for (int q = 0; q < KS; ++q) v[q] = (S)(__float_as_uint(__uint_as_float((uint32_t)v[q] << 16) * scale) >> 16);
+    S *dst = out + r.dst + (int64_t)s * r.nrows * KS + (int64_t)(r.row0 + row) * E;
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int e = 0; e < E; ++e) dst[(int64_t)h * r.nrows * E + e] = v[h * E + e];
+  }
+}
+
+}  // namespace hmvm

@@ -353,12 +353,10 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
     P.tsum.n = (int)P.n_t;
     P.tsum.seg.assign((size_t)P.n_t, -1);
     // A row group of one column chunk whose leaves all read a materialised t
-    // has one partial slot per t entry: in the multi-RHS launches its tile
-    // writes t itself, through a row map (scaled like the t sum under BF16),
-    // and the multi-RHS t sum leaves those entries out.  The one-vector
-    // launches keep the slots and the full t sum (there the map load at the
-    // end of the tile costs launch A more than the t sum saves: measured on
-    // a batch of 64 matrices, FP32 1.108 -> 1.135 ms).
+    // has one partial slot per t entry: its rows get a map to t
+    // (map_off_multi).  The launches keep the slots and the full t sum (the
+    // map load at the end of the tile costs launch A more than the t sum
+    // saves: measured on a batch of 64 matrices, FP32 1.108 -> 1.135 ms).
     std::map<int64_t, bool> direct;  // first slot -> every piece of the group materialised
     for (const PieceRec &pc : pieces)
       if (single.count(pc.slot0)) {
@@ -604,7 +602,7 @@ std::string verify_plan(const Plan &P, const LeafArrays &la) {
   const int64_t npan = (int64_t)P.panels.size();
   std::vector<int64_t> seen2(P.nlf, 0);
   int64_t seen1 = 0;
-  std::vector<char> t_written((size_t)P.n_t, 0);  // t entries a stage-1 tile writes (multi-RHS launches)
+  std::vector<char> t_written((size_t)P.n_t, 0);  // t entries a stage-1 row map names
   for (int list = 0; list < 2; list++) {
     const std::vector<TileDesc> &tl = list == 0 ? P.tiles_a : P.tiles_b;
     for (const TileDesc &t : tl) {
@@ -729,8 +727,7 @@ std::string verify_plan(const Plan &P, const LeafArrays &la) {
   const int64_t ntseg = (int64_t)P.tsum.ptr.size() - 1, nyseg = (int64_t)P.ysum.ptr.size() - 1;
   for (int i = 0; i < P.tsum.n; i++) {
     const int s = P.tsum.seg[i];
-    // every t entry has a t sum segment (the one-vector launches sum them all;
-    // the multi-RHS t sum skips the entries a row map writes)
+    // every t entry has a t sum segment (the launches sum them all)
     if (s < 0 || s >= ntseg) return "t segment id out of range";
     const int e0 = P.tsum.ptr[s], e1 = P.tsum.ptr[s + 1];
     for (int e = e0; e < e1; e++) {

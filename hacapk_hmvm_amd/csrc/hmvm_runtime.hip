@@ -19,6 +19,7 @@
 #include "hacapk.h"
 #include "hmvm_hip.h"
 #include "hmvm_kernels.hpp"
+#include "hmvm_multi_args.hpp"
 #include "hmvm_plan.hpp"
 #include "hmvm_status.hpp"
 #include "io_records.hpp"
@@ -106,14 +107,13 @@ std::vector<int2> seg_ranges(const SegSum &g) {
 // {first slot, (nch << 16) | stride, t entry, 0} of every summed t entry, in
 // entry order: every segment lists its slots at one stride (a rank row's
 // partial slots in the column chunks of its row group are one row group
-// apart).  Entries marked in `skip` (written through a stage-1 row map) get
-// no descriptor.  False when a segment is not at one stride, or its fields do
-// not fit.
-bool t_descs(const SegSum &g, const std::vector<char> &skip, std::vector<int4> *out) {
+// apart).  False when a segment is not at one stride, or its fields do not
+// fit.
+bool t_descs(const SegSum &g, std::vector<int4> *out) {
   out->clear();
   for (size_t i = 0; i < g.seg.size(); i++) {
     const int s = g.seg[i];
-    if (s < 0 || (!skip.empty() && skip[i])) continue;
+    if (s < 0) continue;
     const int e0 = g.ptr[s], e1 = g.ptr[s + 1], nch = e1 - e0;
     const int64_t first = nch > 0 ? g.list[e0] + (int64_t)i : 0;
     const int64_t stride = nch > 1 ? g.list[e0 + 1] - g.list[e0] : 0;
@@ -161,7 +161,6 @@ struct hmvm_plan {
   hipStream_t stream2 = nullptr;       // dense tiles, concurrent with stage 1 / t sum / stage 2
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool a_mixed = false;  // launch A order is not "stage-1 tiles, then dense" (modes 1 and 2 need that)
-  bool has_tp = false;   // some panel sums stage-1 partial slots (kVecTP)
   int persist_key = -1, persist_blocks = 0;  // persistent launch: its shape (kernel variant, block size) and grid
   int tiles_version = 0, persist_version = -1;  // tile lists changed / the dealt lists are of this version
   TileDesc *d_ptiles_a = nullptr, *d_ptiles_b = nullptr;  // persistent launch: tiles dealt to the waves
@@ -171,8 +170,22 @@ struct hmvm_plan {
   void *d_mslots = nullptr;  // slot_bytes(storage) per slot
   void *d_mt = nullptr;      // t: vec_bytes(storage) per entry
   void *d_mXc = nullptr;     // X in the operand type (FP32 and BF16 storage)
-  TileDesc *d_mtiles_a = nullptr, *d_mtiles_b = nullptr;  // XCD-aware tile layouts of launches A and B
-  int mtiles_wpb = 0;                                     // waves per workgroup they were laid out for
+  std::vector<int> nstrtl, nstrtt;  // first row and column of every leaf, for the schedule below
+  bool multi_ready = false;         // the multi-RHS schedule is built (hmvm_multi_plan.hpp)
+  int multi_waves = 0, n_mgroups_a = 0, n_mgroups_b = 0, n_mtsum = 0;
+  int64_t n_mt = 0, n_mslots = 0;
+  MultiGroup *d_mgroups_a = nullptr, *d_mgroups_b = nullptr;  // in dispatch order
+  MultiWave *d_mwaves_a = nullptr, *d_mwaves_b = nullptr;
+  int32_t *d_mtmap = nullptr, *d_mtfac = nullptr, *d_mylist = nullptr;
+  MultiItem *d_mitems = nullptr;
+  MultiSlice *d_mslices = nullptr;
+  void *d_mvals = nullptr;      // values packed for the multi-RHS kernels, or one window of them
+  int64_t multi_elems = 0;      // packed values
+  std::vector<MultiWindow> multi_windows;  // empty: all values are packed
+  MultiPack *d_mpack = nullptr;
+  int4 *d_mtsum = nullptr;      // {first, (nch << 16) | stride, entry, 0}
+  int2 *d_myrng = nullptr;
+  double *d_mscale_m = nullptr, *d_mzero = nullptr;
   double *d_mX = nullptr, *d_mY = nullptr;
   PersistCounters *d_ctr = nullptr;
   int ncu = 0;     // compute units of the device
@@ -190,8 +203,6 @@ struct hmvm_plan {
   int2 *d_yrng = nullptr;   // per-entry list ranges of the y sum
   int2 *d_tdesc = nullptr;    // t sum: {first slot, (nch << 16) | stride} per entry
   int n_tsum = 0;             // t entries summed by the one-vector launches
-  int4 *d_tdesc_m = nullptr;  // multi-RHS t sum: {first, (nch << 16) | stride, entry, 0} of the
-  int n_tsum_m = 0;           // entries no stage-1 row map writes
   float *d_scales = nullptr;
   double *d_x = nullptr, *d_y = nullptr;  // staging for host-pointer calls
   size_t device_bytes = 0;
@@ -199,8 +210,10 @@ struct hmvm_plan {
   ~hmvm_plan() {
     void *ptrs[] = {d_vals,  d_tiles_a, d_tiles_b, d_panels, d_t,      d_slots,
                     d_tfac,  d_tmap,    d_ylist,  d_scales, d_x,      d_y,
-                    d_yrng,  d_tdesc,   d_tdesc_m, d_mtiles_a, d_mtiles_b, d_ptiles_a, d_ptiles_b, d_pptr_a, d_pptr_b,
-                    d_ctr,   d_mslots,  d_mt,      d_mX,     d_mY,     d_mXc,    d_mscale};
+                    d_yrng,  d_tdesc,   d_ptiles_a, d_ptiles_b, d_pptr_a, d_pptr_b,
+                    d_ctr,   d_mslots,  d_mt,      d_mX,     d_mY,     d_mXc,    d_mscale,
+                    d_mgroups_a, d_mgroups_b, d_mwaves_a, d_mwaves_b, d_mtmap, d_mtfac, d_mylist, d_mitems, d_mslices,
+                    d_mtsum, d_myrng, d_mscale_m, d_mzero, d_mvals, d_mpack};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
@@ -770,7 +783,6 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
   err = verify_plan(p->plan, src.la);
   if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "schedule check failed: %s", err.c_str());
   Plan &P = p->plan;
-  for (const PanelDesc &pd : P.panels) p->has_tp = p->has_tp || pd.vec_sel == kVecTP;
   p->a_mixed = order_mixed(P);
   HIP_TRY(hipGetDevice(&p->device));
   HIP_TRY(hipStreamCreate(&p->stream));
@@ -793,26 +805,17 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
       (rc = upload(&p->d_ylist, P.ysum.list)) || (rc = upload(&p->d_yrng, seg_ranges(P.ysum))))
     return rc;
   {
-    std::vector<int4> all, multi;
-    if (!t_descs(P.tsum, {}, &all))
+    std::vector<int4> all;
+    if (!t_descs(P.tsum, &all))
       return set_error(HMVM_ERR_UNSUPPORTED, "t sum segment with more than 65535 chunks or an irregular stride");
     if (all.size() != (size_t)P.tsum.n) return set_error(HMVM_ERR_UNSUPPORTED, "t entry without a t sum segment");
     std::vector<int2> one(all.size());  // every entry, in entry order
     for (size_t i = 0; i < all.size(); i++) one[i] = make_int2(all[i].x, all[i].y);
     if ((rc = upload(&p->d_tdesc, one))) return rc;
     p->n_tsum = (int)one.size();
-    if (!P.t_direct && !P.tmap.empty()) {  // multi-RHS: the entries the row maps write are not summed
-      std::vector<char> mapped((size_t)P.n_t, 0);
-      for (int32_t e : P.tmap) mapped[(size_t)e] = 1;
-      (void)t_descs(P.tsum, mapped, &multi);  // a subset of `all`, which passed
-    } else {
-      multi.swap(all);
-    }
-    if ((rc = upload(&p->d_tdesc_m, multi))) return rc;
-    p->n_tsum_m = (int)multi.size();
   }
   if (p->mode != 0 && (rc = partition_a(p.get()))) return rc;
-  if (!P.tmap.empty() && (rc = upload(&p->d_tmap, P.tmap))) return rc;
+  if (P.t_direct && (rc = upload(&p->d_tmap, P.tmap))) return rc;
   if (p->storage == kBF16) {
     if ((rc = upload(&p->d_tfac, P.factor_of_trow))) return rc;
     if ((rc = dalloc(&p->d_scales, (size_t)P.nfactors))) return rc;
@@ -826,10 +829,12 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
   HIP_TRY(hipMalloc(&p->d_vals, eb * (size_t)std::max<int64_t>(P.nvals, 1)));
   // column padding is read (and discarded) by the 16-byte lane loads: keep it zero
   HIP_TRY(hipMemsetAsync(p->d_vals, 0, eb * (size_t)std::max<int64_t>(P.nvals, 1), p->stream));
+  p->nstrtl.assign(src.la.nstrtl, src.la.nstrtl + src.la.nlf);
+  p->nstrtt.assign(src.la.nstrtt, src.la.nstrtt + src.la.nlf);
 
   // values: streamed to the GPU in windows and repacked there
   if ((rc = upload_values(p.get(), src))) return rc;
-  if (p->storage == kBF16 && !P.tmap.empty()) {
+  if (p->storage == kBF16 && P.t_direct && !P.tmap.empty()) {
     if ((rc = dalloc(&p->d_mscale, P.tmap.size()))) return rc;
     hipLaunchKernelGGL(map_scale_kernel, dim3((unsigned)((P.tmap.size() + 255) / 256)), dim3(256), 0, p->stream,
                        (int)P.tmap.size(), p->d_tmap, p->d_tfac, (const float *)p->d_scales, p->d_mscale);
@@ -841,8 +846,8 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
   p->device_bytes = eb * (size_t)P.nvals + sizeof(TileDesc) * (P.tiles_a.size() + P.tiles_b.size()) +
                     sizeof(PanelDesc) * P.panels.size() + 8 * (size_t)(P.n_t + 2 * P.nd) +
                     slot_bytes(p->storage) * (size_t)(P.n_tp + P.n_z) +
-                    4 * (size_t)P.n_t + (p->d_mscale ? 12 : 4) * P.tmap.size() +
-                    sizeof(int2) * (size_t)p->n_tsum + sizeof(int4) * (size_t)p->n_tsum_m +
+                    4 * (size_t)P.n_t + (P.t_direct ? (p->d_mscale ? 12 : 4) * P.tmap.size() : 0) +
+                    sizeof(int2) * (size_t)p->n_tsum +
                     8 * (P.ysum.list.size() + P.ysum.seg.size());
   if (verbose())
     std::fprintf(stderr,
@@ -855,7 +860,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
 }
 
 // Where the tiles of one launch store their rows: the slots, and for
-// stage-1 tiles with a row map the plan's t (or the multi-RHS T).
+// stage-1 tiles with a row map the plan's t.
 TileOut tile_out(const hmvm_plan *p, void *out, void *tout) {
   return TileOut{out, p->d_tmap, tout, p->d_mscale};
 }
@@ -1012,77 +1017,101 @@ void launch_phase(hmvm_plan *p, int phase, const double *x, double *y, int accum
 }
 
 // ---- several right-hand sides -------------------------------------------------
-// Workgroup w of a launch runs on XCD w % kXcds: MI355X hands the workgroups
-// of a grid to its 8 XCDs round robin, and each XCD has its own L2.  A
-// multi-RHS tile reads a slice of X (launch A) or t (launch B) of nrhs
-// entries per column, which other tiles over the same columns read again.
-// Sorted by the start of that slice, the tiles are cut into kXcds runs of
-// equal work (elements), and laid out so that the workgroups of XCD k take
-// run k's tiles, largest first: each XCD then reads about one kXcds-th of the
-// vector, which its L2 holds, instead of all of it.  A workgroup whose run is
-// used up takes tiles of the run with the most left.
-std::vector<TileDesc> xcd_layout(const std::vector<TileDesc> &tiles, int wpb) {
-  const size_t n = tiles.size();
-  std::vector<size_t> idx(n);
-  for (size_t i = 0; i < n; i++) idx[i] = i;
-  std::stable_sort(idx.begin(), idx.end(),
-                   [&](size_t a, size_t b) { return tiles[a].first.vec_off < tiles[b].first.vec_off; });
-  auto work = [&](size_t i) { return (double)tiles[i].nrows * (double)tiles[i].ncols; };
-  double total = 0;
-  for (size_t i = 0; i < n; i++) total += work(i);
-  std::vector<std::vector<size_t>> run(kXcds);
-  double cum = 0;
-  for (size_t i : idx) {
-    const int r = total > 0 ? std::min(kXcds - 1, (int)((cum + 0.5 * work(i)) * kXcds / total)) : 0;
-    run[r].push_back(i);
-    cum += work(i);
-  }
-  for (auto &r : run)
-    std::stable_sort(r.begin(), r.end(), [&](size_t a, size_t b) { return work(a) > work(b); });
-  std::vector<TileDesc> out;
-  out.reserve(n);
-  std::vector<size_t> pos(kXcds, 0);
-  for (int w = 0; out.size() < n; w++) {
-    for (int k = 0; k < wpb && out.size() < n; k++) {
-      int r = w % kXcds;
-      if (pos[r] == run[r].size()) {  // run used up: the run with the most tiles left
-        for (int q = 0; q < kXcds; q++)
-          if (run[q].size() - pos[q] > run[r].size() - pos[r]) r = q;
-      }
-      out.push_back(tiles[run[r][pos[r]++]]);
-    }
-  }
-  return out;
+// Elements of the multi-RHS value window: the value of HMVM_MULTI_WINDOW when
+// set (>= 1), else 0 (all values packed once, in windows only if memory lacks).
+int64_t multi_window_elems() {
+  const char *e = std::getenv("HMVM_MULTI_WINDOW");
+  return e && *e ? std::max(0LL, std::atoll(e)) : 0;
 }
 
-// Uploads the XCD-aware layouts of both launches for the plan's current
-// workgroup size (again when that changes).
-int multi_layout(hmvm_plan *p) {
-  const int wpb = p->block_threads / 64;
-  if (p->mtiles_wpb == wpb && p->d_mtiles_a) return HMVM_OK;
-  for (TileDesc **d : {&p->d_mtiles_a, &p->d_mtiles_b})
-    if (*d) {
-      (void)hipFree(*d);
-      *d = nullptr;
-    }
-  p->mtiles_wpb = 0;
-  // the multi-RHS launches send the rows of stage-1 tiles with a
-  // multi-RHS row map to t
-  std::vector<TileDesc> ta = p->plan.tiles_a;
-  for (TileDesc &t : ta) t.map_off = t.map_off_multi;
+void multi_free(hmvm_plan *p) {
+  void *bufs[] = {p->d_mgroups_a, p->d_mgroups_b, p->d_mwaves_a, p->d_mwaves_b, p->d_mitems, p->d_mslices,
+                  p->d_mtmap,     p->d_mtsum,     p->d_myrng,    p->d_mylist,   p->d_mzero,  p->d_mtfac,
+                  p->d_mscale_m,  p->d_mpack,     p->d_mvals};
+  for (void *b : bufs)
+    if (b) (void)hipFree(b);
+  p->d_mgroups_a = p->d_mgroups_b = nullptr;
+  p->d_mwaves_a = p->d_mwaves_b = nullptr;
+  p->d_mitems = nullptr;
+  p->d_mslices = nullptr;
+  p->d_mtmap = p->d_mylist = p->d_mtfac = nullptr;
+  p->d_mtsum = nullptr;
+  p->d_myrng = nullptr;
+  p->d_mzero = p->d_mscale_m = nullptr;
+  p->d_mpack = nullptr;
+  p->d_mvals = nullptr;
+  p->multi_ready = false;
+  p->multi_windows.clear();
+}
+
+// Builds, checks and uploads the multi-RHS schedule and packs its values.
+// window: 0 packs all values into a copy of their own; else a buffer of so
+// many elements, which every apply fills and uses window by window.
+int multi_schedule(hmvm_plan *p, int64_t window) {
+  MultiPlan M;
+  MultiOptions opt = multi_options(p->plan);
+  if (window > 0) opt.wave_cols = 0;
+  std::string err = build_multi_plan(p->plan, p->storage, p->nstrtl.data(), p->nstrtt.data(), opt, &M);
+  if (err.empty()) err = verify_multi_plan(p->plan, p->storage, M);
+  if (err.empty() && window > 0) err = window_multi_plan(p->storage, window, &M, &p->multi_windows);
+  if (!err.empty()) return set_error(HMVM_ERR_UNSUPPORTED, "multi-RHS schedule: %s", err.c_str());
+  std::vector<int4> ts;
+  for (const MultiPlan::TSum &t : M.tsum)
+    ts.push_back(make_int4(t.first, (int)(((unsigned)t.nch << 16) | (unsigned)t.stride), t.entry, 0));
+  std::vector<int2> rng((size_t)p->plan.nd);
+  for (size_t i = 0; i < rng.size(); i++) rng[i] = make_int2(M.yptr[2 * i], M.yptr[2 * i + 1]);
   int rc;
-  if ((rc = upload(&p->d_mtiles_a, xcd_layout(ta, wpb))) ||
-      (rc = upload(&p->d_mtiles_b, xcd_layout(p->plan.tiles_b, wpb))))
+  if ((rc = upload(&p->d_mgroups_a, M.groups_a)) || (rc = upload(&p->d_mgroups_b, M.groups_b)) ||
+      (rc = upload(&p->d_mwaves_a, M.waves_a)) || (rc = upload(&p->d_mwaves_b, M.waves_b)) ||
+      (rc = upload(&p->d_mitems, M.items)) || (rc = upload(&p->d_mslices, M.slices)) ||
+      (rc = upload(&p->d_mtmap, M.tmap)) || (rc = upload(&p->d_mtsum, ts)) || (rc = upload(&p->d_myrng, rng)) ||
+      (rc = upload(&p->d_mylist, M.ylist)) || (rc = upload(&p->d_mpack, M.pack)) ||
+      (rc = upload(&p->d_mzero, std::vector<double>(kMultiZeroBytes / 8, 0.0))))
     return rc;
-  p->mtiles_wpb = wpb;
+  if (p->storage == kBF16) {
+    if ((rc = upload(&p->d_mtfac, M.t_factor)) || (rc = dalloc(&p->d_mscale_m, M.tmap.size()))) return rc;
+    if (!M.tmap.empty())
+      hipLaunchKernelGGL(map_scale_kernel, dim3((unsigned)((M.tmap.size() + 255) / 256)), dim3(256), 0, p->stream,
+                         (int)M.tmap.size(), p->d_mtmap, p->d_mtfac, (const float *)p->d_scales, p->d_mscale_m);
+  }
+  if ((rc = dalloc_bytes(&p->d_mvals, (size_t)elem_bytes(p->storage) * (size_t)(window > 0 ? window : M.nvals))))
+    return rc;
+  if (window == 0) {
+    launch_multi_pack(p->storage, (int)M.pack.size(), p->d_mpack, p->d_vals, p->d_scales, p->d_mvals, p->stream);
+    HIP_TRY(hipStreamSynchronize(p->stream));
+    (void)hipFree(p->d_mpack);
+    p->d_mpack = nullptr;
+  }
+  HIP_TRY(hipStreamSynchronize(p->stream));
+  HIP_TRY(hipGetLastError());
+  p->multi_waves = M.waves;
+  p->n_mgroups_a = (int)M.groups_a.size();
+  p->n_mgroups_b = (int)M.groups_b.size();
+  p->n_mtsum = (int)ts.size();
+  p->n_mt = M.n_t;
+  p->n_mslots = M.n_slots;
+  p->multi_elems = M.nvals;
+  p->multi_ready = true;
   return HMVM_OK;
 }
 
-int reserve_multi(hmvm_plan *p, int nrhs) {
-  if (nrhs != 16 && nrhs != 32 && nrhs != 64) return set_error(HMVM_ERR_ARG, "nrhs must be 16, 32 or 64");
-  int rc = multi_layout(p);
-  if (rc) return rc;
-  if (p->multi_cap >= nrhs) return HMVM_OK;
+// The schedule with all values packed, or, where the device has no memory for
+// that, with a window of half, a quarter, ... of them.
+int multi_schedule_fit(hmvm_plan *p, bool whole) {
+  int64_t window = multi_window_elems();
+  if (window == 0 && !whole) window = std::max<int64_t>(1, p->plan.nvals / 2);
+  for (;;) {
+    multi_free(p);
+    const int rc = multi_schedule(p, window);
+    if (rc == HMVM_OK) return rc;
+    (void)hipGetLastError();
+    multi_free(p);
+    if (rc != HMVM_ERR_HIP || window == 1) return rc;
+    window = window > 0 ? (window + 1) / 2 : std::max<int64_t>(1, p->plan.nvals / 2);
+  }
+}
+
+int multi_buffers(hmvm_plan *p, int nrhs) {
   const Plan &P = p->plan;
   void *bufs[5] = {p->d_mslots, p->d_mt, p->d_mX, p->d_mY, p->d_mXc};
   for (void *b : bufs)
@@ -1091,8 +1120,9 @@ int reserve_multi(hmvm_plan *p, int nrhs) {
   p->d_mX = p->d_mY = nullptr;
   p->d_mXc = nullptr;
   p->multi_cap = 0;
-  if ((rc = dalloc_bytes(&p->d_mslots, slot_bytes(p->storage) * (size_t)(P.n_tp + P.n_z) * nrhs)) ||
-      (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)P.n_t * nrhs)) ||
+  int rc;
+  if ((rc = dalloc_bytes(&p->d_mslots, slot_bytes(p->storage) * (size_t)p->n_mslots * nrhs)) ||
+      (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)p->n_mt * nrhs)) ||
       (rc = dalloc(&p->d_mX, (size_t)P.nd * nrhs)) || (rc = dalloc(&p->d_mY, (size_t)P.nd * nrhs)))
     return rc;
   if (p->storage != kF64 && (rc = dalloc_bytes(&p->d_mXc, vec_bytes(p->storage) * (size_t)P.nd * nrhs))) return rc;
@@ -1100,122 +1130,113 @@ int reserve_multi(hmvm_plan *p, int nrhs) {
   return HMVM_OK;
 }
 
-// T: the t read by stage-2 panels (launch B; NULL in launch A, whose
-// stage-1 tiles with a row map write it instead)
-template <typename S, bool kScaled, int NB>
-void launch_multi_tiles(hmvm_plan *p, const TileDesc *d_tiles, int ntiles, const void *Xv, const void *Tv,
-                        hipStream_t st) {
-  if (ntiles == 0) return;
-  const int wpb = p->block_threads / 64;
-  const TileOut o = tile_out(p, p->d_mslots, p->d_mt);
-  const auto *TP = (const typename SlotOf<S>::T *)p->d_mslots;
-  const auto *X = (const typename VecOf<S>::T *)Xv;
-  const auto *T = (const typename VecOf<S>::T *)Tv;
-  if (p->has_tp)
-    hipLaunchKernelGGL((tile_multi_kernel<S, kScaled, NB, true>), dim3((ntiles + wpb - 1) / wpb),
-                       dim3(p->block_threads), 0, st, d_tiles, ntiles, p->d_panels, (const S *)p->d_vals, X, T,
-                       TP, (const float *)p->d_scales, o);
-  else
-    hipLaunchKernelGGL((tile_multi_kernel<S, kScaled, NB, false>), dim3((ntiles + wpb - 1) / wpb),
-                       dim3(p->block_threads), 0, st, d_tiles, ntiles, p->d_panels, (const S *)p->d_vals, X, T,
-                       TP, (const float *)p->d_scales, o);
+int reserve_multi(hmvm_plan *p, int nrhs) {
+  if (nrhs != 16 && nrhs != 32 && nrhs != 64) return set_error(HMVM_ERR_ARG, "nrhs must be 16, 32 or 64");
+  int rc;
+  if (!p->multi_ready && (rc = multi_schedule_fit(p, true))) return rc;
+  if (p->multi_cap >= nrhs) return HMVM_OK;
+  rc = multi_buffers(p, nrhs);
+  if (rc == HMVM_ERR_HIP && p->multi_windows.empty()) {
+    // the packed values took the memory of the work buffers: pack them in windows
+    (void)hipGetLastError();
+    if ((rc = multi_schedule_fit(p, false))) return rc;
+    rc = multi_buffers(p, nrhs);
+  }
+  return rc;
 }
 
-template <typename S, bool kScaled>
-void launch_multi_nb(hmvm_plan *p, const TileDesc *d_tiles, int ntiles, const void *X, const void *T, int nrhs,
-                     hipStream_t st) {
-  if (nrhs == 16)
-    launch_multi_tiles<S, kScaled, 1>(p, d_tiles, ntiles, X, T, st);
-  else if (nrhs == 32)
-    launch_multi_tiles<S, kScaled, 2>(p, d_tiles, ntiles, X, T, st);
-  else
-    launch_multi_tiles<S, kScaled, 4>(p, d_tiles, ntiles, X, T, st);
-}
-
-// Multi-RHS t (phase 1) or y (phase 3) segment sum over slots of type P.
-template <typename P>
-void launch_segsum_multi(hmvm_plan *p, int phase, double *Y, int nrhs, int accumulate, hipStream_t st) {
-  const Plan &P_ = p->plan;
-  const P *slots = (const P *)p->d_mslots;
-  if (phase == 1) {
-    // 16-byte loads and stores (slots and t are the plan's own allocations)
-    const int4 *desc = p->d_tdesc_m;
-    const int n = p->n_tsum_m;
-    if (P_.t_fused || n == 0) return;
-    // t in the multi-RHS operand type (VecOf: FP64, FP32 or BF16 bits)
-    const int64_t tw = (int64_t)n * (nrhs / (16 / (int)sizeof(P)));
-    const dim3 grid((unsigned)((tw + 255) / 256));
-    P *T = (P *)p->d_mt;
-    if (p->storage == kBF16)
-      hipLaunchKernelGGL((tsum_multi_kernel<true, P, uint16_t>), grid, dim3(256), 0, st, n, nrhs, desc, slots,
-                         p->d_tfac, p->d_scales, (uint16_t *)p->d_mt);
-    else
-      hipLaunchKernelGGL((tsum_multi_kernel<false, P, P>), grid, dim3(256), 0, st, n, nrhs, desc,
-                         slots, (const int32_t *)nullptr, (const float *)nullptr, T);
-  } else if (((uintptr_t)Y & 15) == 0) {  // 16-byte slot loads where the caller's Y is 16-byte aligned
-    constexpr int W = 16 / sizeof(P);
-    const int64_t tot = (int64_t)P_.ysum.n * (nrhs / W);
-    hipLaunchKernelGGL((ysum_multi_kernel<W, P>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, P_.ysum.n,
-                       nrhs, p->d_yrng, p->d_ylist, slots, Y, accumulate);
-  } else {
-    const int64_t tot = (int64_t)P_.ysum.n * nrhs;
-    hipLaunchKernelGGL((ysum_multi_kernel<1, P>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, P_.ysum.n,
-                       nrhs, p->d_yrng, p->d_ylist, slots, Y, accumulate);
+// which: 0 launch A (stage 1 to t and t slots), 1 launch B (rows of y); X in
+// the operand type
+void launch_multi_part(hmvm_plan *p, int which, const void *X, double *Y, int nrhs, int accumulate, hipStream_t st) {
+  MultiArgs a;
+  const MultiGroup *groups = which ? p->d_mgroups_b : p->d_mgroups_a;
+  const MultiWave *waves = which ? p->d_mwaves_b : p->d_mwaves_a;
+  a.groups = groups;
+  a.waves = waves;
+  a.items = p->d_mitems;
+  a.slices = p->d_mslices;
+  a.vals = p->d_mvals;
+  a.X = X;
+  a.T = p->d_mt;
+  a.zero = p->d_mzero;
+  a.slots = p->d_mslots;
+  a.t_out = p->d_mt;
+  a.tmap = p->d_mtmap;
+  a.mscale = p->d_mscale_m;
+  a.Y = Y;
+  a.yrng = p->d_myrng;
+  a.ylist = p->d_mylist;
+  a.accumulate = accumulate;
+  a.y16 = ((uintptr_t)Y & 15) == 0;
+  if (p->multi_windows.empty()) {
+    launch_multi_groups(p->storage, nrhs, a, which ? p->n_mgroups_b : p->n_mgroups_a, p->multi_waves, st);
+    return;
+  }
+  for (const MultiWindow &w : p->multi_windows) {
+    if (w.launch != which) continue;
+    // element e of the packed values stands at e - w.a0 of the window
+    void *vals = (void *)((uintptr_t)p->d_mvals - (uintptr_t)w.a0 * (uintptr_t)elem_bytes(p->storage));
+    launch_multi_pack(p->storage, w.npack, p->d_mpack + w.pack0, p->d_vals, p->d_scales, vals, st);
+    a.vals = vals;
+    a.groups = groups + w.group0;
+    a.waves = waves + (size_t)w.group0 * p->multi_waves;
+    launch_multi_groups(p->storage, nrhs, a, w.ngroups, p->multi_waves, st);
   }
 }
 
+// Multi-RHS t sum over slots of type P.
+template <typename P>
+void launch_tsum_multi(hmvm_plan *p, int nrhs, hipStream_t st) {
+  const int n = p->n_mtsum;
+  if (n == 0) return;
+  const P *slots = (const P *)p->d_mslots;
+  // 16-byte loads and stores (slots and t are the plan's own allocations); t
+  // in the multi-RHS operand type (VecOf: FP64, FP32 or BF16 bits)
+  const int64_t tw = (int64_t)n * (nrhs / (16 / (int)sizeof(P)));
+  const dim3 grid((unsigned)((tw + 255) / 256));
+  if (p->storage == kBF16)
+    hipLaunchKernelGGL((tsum_multi_kernel<true, P, uint16_t>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, slots,
+                       p->d_mtfac, p->d_scales, (uint16_t *)p->d_mt);
+  else
+    hipLaunchKernelGGL((tsum_multi_kernel<false, P, P>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, slots,
+                       (const int32_t *)nullptr, (const float *)nullptr, (P *)p->d_mt);
+}
+
+// Phase 0: the operand copy of X (FP32 and BF16 storage) and launch A, 1: the
+// t sum, 2: launch B.
 void launch_multi_phase(hmvm_plan *p, int phase, const double *X, double *Y, int nrhs, int accumulate,
                         hipStream_t st) {
   const Plan &P = p->plan;
-  if (phase == 0 || phase == 2) {
-    const TileDesc *tl = phase == 0 ? p->d_mtiles_a : p->d_mtiles_b;
-    const int nt = (int)(phase == 0 ? P.tiles_a.size() : P.tiles_b.size());
-    const void *T = phase == 0 ? nullptr : p->d_mt;
-    if (p->storage != kF64) {
-      // the tiles read X and t in the operand type: a copy of X made here,
-      // before launch A, and a t the t sum writes so
-      if (phase == 0) {
-        const size_t n = (size_t)P.nd * nrhs;
-        const unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 8192);
-        const bool a16 = ((uintptr_t)X & 15) == 0;
-        if (p->storage == kF32 && a16)
-          hipLaunchKernelGGL((to_vec_kernel<2, float>), dim3(blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
-        else if (p->storage == kF32)
-          hipLaunchKernelGGL((to_vec_kernel<1, float>), dim3(2 * blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
-        else if (a16)
-          hipLaunchKernelGGL((to_vec_kernel<2, uint16_t>), dim3(blocks), dim3(256), 0, st, X, (uint16_t *)p->d_mXc,
-                             n);
-        else
-          hipLaunchKernelGGL((to_vec_kernel<1, uint16_t>), dim3(2 * blocks), dim3(256), 0, st, X,
-                             (uint16_t *)p->d_mXc, n);
-      }
-    }
-    if (p->storage == kF64 && nrhs > 16 && ((uintptr_t)X & 15) != 0) {
-      // the tiles load two or four right-hand sides at once (16-byte loads):
-      // an X that is not 16-byte aligned is first copied to the plan's own
-      if (phase == 0)
-        (void)hipMemcpyAsync(p->d_mX, X, sizeof(double) * (size_t)P.nd * nrhs, hipMemcpyDeviceToDevice, st);
-      X = p->d_mX;
-    }
-    const void *Xv = p->storage == kF64 ? (const void *)X : (const void *)p->d_mXc;
+  if (phase == 1) {
     if (p->storage == kF64)
-      launch_multi_nb<double, false>(p, tl, nt, Xv, T, nrhs, st);
-    else if (p->storage == kF32)
-      launch_multi_nb<float, false>(p, tl, nt, Xv, T, nrhs, st);
+      launch_tsum_multi<double>(p, nrhs, st);
     else
-      launch_multi_nb<uint16_t, true>(p, tl, nt, Xv, T, nrhs, st);
-  } else if (p->storage == kF64) {
-    launch_segsum_multi<double>(p, phase, Y, nrhs, accumulate, st);
-  } else {
-    launch_segsum_multi<float>(p, phase, Y, nrhs, accumulate, st);
+      launch_tsum_multi<float>(p, nrhs, st);
+    return;
   }
+  if (phase == 3) return;
+  if (phase == 0 && p->storage != kF64) {
+    // the groups read X and t in the operand type
+    const size_t n = (size_t)P.nd * nrhs;
+    const unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 8192);
+    const bool a16 = ((uintptr_t)X & 15) == 0;
+    if (p->storage == kF32 && a16)
+      hipLaunchKernelGGL((to_vec_kernel<2, float>), dim3(blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
+    else if (p->storage == kF32)
+      hipLaunchKernelGGL((to_vec_kernel<1, float>), dim3(2 * blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
+    else if (a16)
+      hipLaunchKernelGGL((to_vec_kernel<2, uint16_t>), dim3(blocks), dim3(256), 0, st, X, (uint16_t *)p->d_mXc, n);
+    else
+      hipLaunchKernelGGL((to_vec_kernel<1, uint16_t>), dim3(2 * blocks), dim3(256), 0, st, X, (uint16_t *)p->d_mXc,
+                         n);
+  }
+  launch_multi_part(p, phase == 2, p->storage == kF64 ? (const void *)X : (const void *)p->d_mXc, Y, nrhs, accumulate,
+                    st);
 }
 
 int apply_multi(hmvm_plan *p, const double *X, double *Y, int nrhs, int accumulate, hipStream_t st) {
   if (p->multi_cap < nrhs) return set_error(HMVM_ERR_ARG, "call hmvm_plan_reserve_multi(plan, %d) first", nrhs);
-  int rc = multi_layout(p);  // no-op unless the workgroup size changed since hmvm_plan_reserve_multi
-  if (rc) return rc;
-  for (int ph = 0; ph < 4; ph++) launch_multi_phase(p, ph, X, Y, nrhs, accumulate, st);
+  for (int ph = 0; ph < 3; ph++) launch_multi_phase(p, ph, X, Y, nrhs, accumulate, st);
   HIP_TRY(hipGetLastError());
   return HMVM_OK;
 }
@@ -1876,6 +1897,10 @@ int hmvm_plan_check(const matrix2 *mat2, const hmvm_options *opt, hmvm_plan_info
   if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "%s", err.c_str());
   err = verify_plan(P, s.la);
   if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "schedule check failed: %s", err.c_str());
+  MultiPlan M;  // the schedule of several right-hand sides (a matrix too large for it keeps the other)
+  if (build_multi_plan(P, po.storage, s.la.nstrtl, s.la.nstrtt, multi_options(P), &M).empty())
+    err = verify_multi_plan(P, po.storage, M);
+  if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "multi-RHS schedule check failed: %s", err.c_str());
   if (info) fill_info(nullptr, P, po.storage, info);
   return HMVM_OK;
 }

@@ -115,13 +115,11 @@ typedef struct hmvm_options {
                          /* stage 1/2                                           */
   int t_mode;            /* stage-2 vector entries: 0 sum the stage-1 partial   */
                          /* slots on the fly, 1 read a materialised t (one more */
-                         /* launch; with several right-hand sides the stage-1   */
-                         /* tiles of a row group of one column chunk write      */
-                         /* their t rows themselves and the t sum adds the      */
-                         /* rest), 2 choose per leaf (likewise),                */
+                         /* launch), 2 choose per leaf,                         */
                          /* 3 t written directly by the stage-1 tiles (bands of */
                          /* rank rows over all of a column cluster's columns;   */
-                         /* no extra launch), -1 default (1)                    */
+                         /* no extra launch), -1 default (1); products with     */
+                         /* several right-hand sides always materialise t       */
   int max_rows;          /* rows per tile (0: by storage); at most 192*V-V+1,  */
                          /* V = 16 bytes / element size; when set, also for the */
                          /* stage-2 tiles unless max_rows_b is set              */
@@ -204,18 +202,17 @@ int hmvm_plan_reset_launch(hmvm_plan *plan);
 
 /* Several right-hand sides on the matrix cores: Y (+)= A X with X, Y of
  * nd x nrhs doubles, row-major (X[i*nrhs + c]); nrhs = 16, 32 or 64.  FP64
- * storage runs v_mfma_f64_16x16x4, FP32 v_mfma_f32_16x16x4 (FP32 accumulate
- * in a tile, FP64 across tiles), BF16 v_mfma_f32_16x16x16_bf16 with the
- * vector entries rounded to BF16 (FP32 and BF16 storage read an FP32 copy
- * of X that the apply makes on the device).  hmvm_plan_reserve_multi
- * allocates the per-plan work buffers for up to nrhs columns and lays the
- * tiles out for the 8 XCDs (workgroups over the same columns of X share an
- * L2); the apply itself allocates nothing unless the plan's workgroup size
- * changed since (it then lays the tiles out again, a synchronous upload:
- * call hmvm_plan_reserve_multi again before capturing the apply in a graph).
- * The host form reserves by itself.  d_X and d_Y need 8-byte alignment; a
- * 16-byte-aligned d_Y gets 16-byte stores, and an FP64 plan copies a d_X
- * that is not 16-byte aligned to its own buffer first (same values). */
+ * storage runs v_mfma_f64_16x16x4, FP32 v_mfma_f32_16x16x4 (FP32 sums of a
+ * few columns, folded into FP64 sums, FP32 ones for 64 right-hand sides; FP64
+ * across waves), BF16 v_mfma_f32_16x16x32_bf16 with the vector entries rounded
+ * to BF16 (FP32 and BF16 storage read a copy of X in their own type that the
+ * apply makes on the device).  hmvm_plan_reserve_multi builds the multi-RHS
+ * schedule, packs a copy of the plan's values in its order (about the size of
+ * the plan's own; where the device lacks that memory, a smaller window that
+ * every apply fills part by part) and allocates the work buffers for up to
+ * nrhs columns; the apply itself allocates nothing.  The host form reserves by
+ * itself.  d_X and d_Y need 8-byte alignment; a 16-byte-aligned d_Y gets
+ * 16-byte stores. */
 int hmvm_plan_reserve_multi(hmvm_plan *plan, int nrhs);
 int hmvm_plan_apply_multi(hmvm_plan *plan, const double *d_X, double *d_Y, int nrhs, int accumulate, void *stream);
 int hmvm_plan_apply_multi_host(hmvm_plan *plan, const double *X, double *Y, int nrhs, int accumulate);
@@ -393,9 +390,10 @@ int hmvm_bicgstab_static(hmvm_plan *plan, const double *d_b, double *d_u, int ma
  * The schedule a plan runs, as plain arrays: the autotuner's features, and
  * the CPU tests that replay it.  Element (r, j) of a tile's panel p is
  * values[val_off + r + j*ld]; row r of a tile goes to slot out_off + r, or to
- * t[tmap[map_off + r]] when map_off >= 0 (in the multi-RHS launches: when
- * map_off_multi >= 0, and their t sum leaves the entries so written alone);
- * the panel's vector entry j is
+ * t[tmap[map_off + r]] when map_off >= 0 (map_off_multi: the same for an
+ * execution that sends the rows of one-chunk row groups straight to t and
+ * whose t sum leaves the entries so written alone; the library's multi-RHS
+ * launches do so in a schedule of their own); the panel's vector entry j is
  * x[vec_off + j] (vec_sel 0), t[vec_off + j] (1) or
  * sum_{c<nch} slots[vec_off + c*stride + j] (2, vec_chunks = nch<<16 | stride).  Repack record: values[dst_off + r +
  * c*dst_cs] = source[src_off + r*src_rs + c*src_cs].  Segment sums:
@@ -405,7 +403,7 @@ typedef struct hmvm_panel {
   int ld, ncols, vec_off, vec_sel, factor, vec_chunks;
 } hmvm_panel;
 /* first: a copy of panel panel0; ncols: the columns of all its panels;
- * map_off_multi: the row map the multi-RHS launches use in place of map_off */
+ * map_off_multi: a row map to use in place of map_off */
 typedef struct hmvm_tile {
   int nrows, panel0, npanel, out_off, map_off, flags, ncols, map_off_multi;
   hmvm_panel first;
