@@ -13,14 +13,18 @@ namespace hmvm {
 namespace {
 
 // The value layout by factor, from the repack records.
-struct Piece {  // rows of a stage-1 stack
+struct Piece {  // rows of a stage-1 stack: ranks k0.. of a leaf
   int leaf, k0, n;
 };
-struct Stack {
+struct Band {  // rows of a stage-1 stack stored together: all of it, or one band
   int64_t base;
-  int ld, ncols, col0;
+  int ld, row0, rows;
+};
+struct Stack {  // the stacked a1 factors of a column cluster
+  int ncols, col0;
   int rows = 0;
   std::vector<Piece> pieces;
+  std::vector<Band> bands;
 };
 struct Factor {  // dense leaf or a2 factor: columns of a row cluster
   int64_t base;
@@ -176,11 +180,14 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
     const int leaf = r.factor / 2;
     if (r.factor % 2 == 0) {
       const int col0 = nstrtt[leaf] - 1;
-      if (stacks.empty() || stacks.back().ld != r.dst_cs || stacks.back().ncols != r.cols ||
-          stacks.back().col0 != col0 || stacks.back().base + stacks.back().rows != r.dst_off)
-        stacks.push_back({r.dst_off, r.dst_cs, r.cols, col0, 0, {}});
-      stacks.back().pieces.push_back({leaf, kdone[leaf], r.rows});
-      stacks.back().rows += r.rows;
+      if (stacks.empty() || stacks.back().ncols != r.cols || stacks.back().col0 != col0)
+        stacks.push_back({r.cols, col0, 0, {}, {}});
+      Stack &s = stacks.back();
+      if (s.bands.empty() || s.bands.back().ld != r.dst_cs || s.bands.back().base + s.bands.back().rows != r.dst_off)
+        s.bands.push_back({r.dst_off, r.dst_cs, s.rows, 0});
+      s.bands.back().rows += r.rows;
+      s.pieces.push_back({leaf, kdone[leaf], r.rows});
+      s.rows += r.rows;
       kdone[leaf] += r.rows;
     } else {
       const int row0 = nstrtl[leaf] - 1;
@@ -273,7 +280,11 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
         const int nc = std::min(s.ncols - c0, step);
         col.slices.clear();
         col.pack.clear();
-        col.pack.push_back({s.base + r0 + (int64_t)c0 * s.ld, 0, s.ld, nr, nc, 0, 0, 0, -1, 0});
+        for (const Band &q : s.bands) {
+          const int a = std::max(q.row0, r0), e = std::min(q.row0 + q.rows, r0 + nr);
+          if (a < e)
+            col.pack.push_back({q.base + (a - q.row0) + (int64_t)c0 * q.ld, 0, q.ld, e - a, nc, a - r0, 0, 0, -1, 0});
+        }
         B.add_slices(col, nc, s.col0 + c0, false);
         const Builder::Place b = B.place(col, nr);
         if (direct && s.ncols <= opt.wave_cols)

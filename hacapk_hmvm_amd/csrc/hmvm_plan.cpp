@@ -124,8 +124,9 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
   std::vector<TileDesc> t1, td, t2;        // stage-1, dense, stage-2 tiles
 
   std::vector<char> mat(nlf, 0);  // stage 2 of this leaf reads the materialised t
-  if (opt.t_mode == 3) {
-    // ---- stage 1 in bands, t written directly (t_mode 3) -----------------------------
+  const bool bands = opt.t_mode == 1 && opt.bands;
+  if (opt.t_mode == 3 || bands) {
+    // ---- stage 1 in bands, t written directly (t_mode 3) or from one slot per entry ----
     // t in row-cluster order, ranks contiguous (so that consecutive a2 factors
     // of a row cluster multiply one contiguous slice of t and merge)
     int64_t tp = 0;
@@ -141,6 +142,11 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
     P.factor_of_trow.assign((size_t)P.n_t, 0);
     for (int i = 0; i < nlf; i++)
       for (int k = 0; mat[i] && k < la.kt[i]; k++) P.factor_of_trow[t_idx[i] + k] = 2 * i;
+    P.tsum.ptr.assign(1, 0);
+    if (bands) {
+      P.tsum.n = (int)P.n_t;
+      P.tsum.seg.assign((size_t)P.n_t, -1);
+    }
     // A column cluster's stacked a1 factors (K rank rows x ndt columns) are
     // cut into bands of near-equal height r (a multiple of V, about w1/ndt
     // rows, at most MR): band b is stored on its own, column-major with
@@ -190,6 +196,12 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
           r.dst_cs = rp;
           r.factor = 2 * i;
           P.repack.push_back(r);
+          if (bands) {  // t sum: one slot of the band per entry
+            const int64_t t0 = t_idx[i] + (a - kofs);
+            for (int k = 0; k < b - a; k++) P.tsum.seg[(size_t)t0 + k] = (int)P.tsum.ptr.size() - 1;
+            P.tsum.list.push_back(P.n_tp + (a - kb0) - t0);
+            P.tsum.ptr.push_back((int)P.tsum.list.size());
+          }
         }
         PanelDesc pd;
         pd.val_off = base;
@@ -203,9 +215,10 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
         tdsc.nrows = nr;
         tdsc.panel0 = (int)P.panels.size();
         tdsc.npanel = 1;
-        tdsc.out_off = 0;
-        tdsc.map_off = (int)P.tmap.size();
-        tdsc.map_off_multi = tdsc.map_off;
+        tdsc.out_off = bands ? (int)P.n_tp : 0;
+        tdsc.map_off_multi = (int)P.tmap.size();
+        tdsc.map_off = bands ? -1 : tdsc.map_off_multi;
+        if (bands) P.n_tp += nr;
         for (int r = 0; r < nr; r++)
           P.tmap.push_back((int32_t)(t_idx[row_leaf[(size_t)kb0 + r]] + row_k[(size_t)kb0 + r]));
         P.panels.push_back(pd);
@@ -215,10 +228,10 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
       }
     }
     if (P.tmap.size() > (size_t)INT32_MAX) return "t map exceeds int32";
-    P.tsum.n = 0;
-    P.tsum.ptr.assign(1, 0);
-    P.t_fused = false;
-    P.t_direct = true;
+    if (P.n_tp > INT32_MAX) return "stage-1 slots exceed int32";
+    P.t_fused = bands && P.n_t == 0;
+    P.t_direct = !bands;
+    P.t_bands = bands && P.n_t > 0;
   } else {
   // ---- stage 1 layout + tiles -----------------------------------------------------
   int64_t tpos = 0;
@@ -354,7 +367,7 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
     P.tsum.seg.assign((size_t)P.n_t, -1);
     // A row group of one column chunk whose leaves all read a materialised t
     // has one partial slot per t entry: its rows get a map to t
-    // (map_off_multi).  The launches keep the slots and the full t sum (the
+    // (map_off_multi).  With other groups beside them the launches keep the slots and the full t sum (the
     // map load at the end of the tile costs launch A more than the t sum
     // saves: measured on a batch of 64 matrices, FP32 1.108 -> 1.135 ms).
     std::map<int64_t, bool> direct;  // first slot -> every piece of the group materialised
@@ -666,6 +679,12 @@ std::string verify_plan(const Plan &P, const LeafArrays &la) {
               const int32_t e = P.tmap[(size_t)t.map_off_multi + r];
               if (e < 0 || e >= P.n_t) return "t map entry out of range";
               if (t_written[(size_t)e]++) return "t entry written twice";
+              if (!P.t_bands) continue;
+              // written to t or to its slot: the t sum of the entry is that slot alone
+              const int sg = (size_t)e < P.tsum.seg.size() ? P.tsum.seg[(size_t)e] : -1;
+              if (sg < 0 || (size_t)sg + 1 >= P.tsum.ptr.size() || P.tsum.ptr[sg + 1] != P.tsum.ptr[sg] + 1 ||
+                  P.tsum.list[(size_t)P.tsum.ptr[sg]] + e != t.out_off + r)
+                return "band row and its t sum disagree";
             }
           }
           if (!P.t_direct && (int64_t)t.out_off + t.nrows > P.n_tp) return "stage-1 slot out of range";
@@ -713,7 +732,7 @@ std::string verify_plan(const Plan &P, const LeafArrays &la) {
     if (la.ltmtx[i] == 1) want1 += (int64_t)la.kt[i] * la.ndt[i];
   }
   if (seen1 != want1) return "stage-1 coverage wrong";
-  if (P.t_direct)
+  if (P.t_direct || P.t_bands)
     for (char w : t_written)
       if (!w) return "t entry never written";
 

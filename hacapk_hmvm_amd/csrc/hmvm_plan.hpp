@@ -83,7 +83,8 @@ struct TileDesc {         // 64 bytes (one scalar load)
   int32_t ncols = 0;      // columns of all the tile's panels together
   // >= 0: row r may go straight to t[tmap[map_off_multi + r]] (a stage-1 tile
   // of a row group of one column chunk; the launches write its slots, which
-  // the t sum adds); map_off under t_mode 3
+  // the t sum adds, or t if all stage-1 tiles are such, Plan::t_bands);
+  // map_off under t_mode 3
   int32_t map_off_multi = -1;
   // a copy of panels[panel0]: the tile's first matrix loads need nothing but
   // this descriptor
@@ -125,6 +126,7 @@ struct PlanOptions {
   int order = 0;          // 0: memory order, 1: largest tiles first
   int t_mode = 0;         // stage-2 vector: 0 partial sums on the fly, 1 materialised t, 2 per leaf,
                           // 3 t written directly by banded stage-1 tiles
+  bool bands = false;     // t_mode 1 with the stage-1 tiles of t_mode 3: one slot per t entry
   int max_rows = kMaxTileRows;  // rows per tile (rank rows per stage-1 group, leaf rows per chunk)
   int max_rows_b = 0;           // rows per stage-2 tile (0: max_rows)
 };
@@ -151,6 +153,8 @@ struct Plan {
   int nfactors = 0;
   bool t_fused = true;               // no stage-2 panel reads the materialised t (no t sum launch)
   bool t_direct = false;             // t_mode 3: stage-1 tiles write t themselves (no t sum launch)
+  bool t_bands = false;              // PlanOptions::bands: every t entry has one slot, and every stage-1
+                                     // tile a map_off_multi
   std::vector<int32_t> tmap;         // t index of every row of the stage-1 tiles with a row map (all of them
                                      // under t_mode 3; otherwise those of one-chunk row groups)
   std::vector<RepackDesc> repack;

@@ -482,6 +482,7 @@ const LaunchDefaults &launch_defaults(int storage) {
 // cube FP64 0.186 -> 0.165 and FP32 0.113 -> 0.094, N=60,013 (leaf 64) BF16
 // 0.087 -> 0.075.
 constexpr int64_t kKneeA[3] = {8192, 8192, 20480};  // FP64, FP32, BF16
+constexpr int64_t kBandLen[3] = {200000000, 64000000, 64000000};  // see plan_options
 struct FitWidths {
   int64_t a, b;  // stage-1 and dense tiles, stage-2 tiles
   int rows_b;    // rows of a stage-2 tile
@@ -504,7 +505,8 @@ PlanOptions plan_options(const hmvm_options *o, int64_t len) {
   PlanOptions po;
   po.storage = o->storage;
   const LaunchDefaults &ld = launch_defaults(po.storage);
-  const FitWidths fit = fit_widths(po.storage >= kF64 && po.storage <= kBF16 ? po.storage : kF64, len, ld.max_rows_b);
+  const int storage = po.storage >= kF64 && po.storage <= kBF16 ? po.storage : kF64;  // (others are refused later)
+  const FitWidths fit = fit_widths(storage, len, ld.max_rows_b);
   po.w1 = o->w1 > 0 ? o->w1 : (int)std::min<int64_t>(ld.w1, fit.a);
   po.w2 = o->w2 > 0 ? o->w2 : (int)std::min<int64_t>(ld.w2, fit.a);
   po.w3 = o->w3 > 0 ? o->w3 : o->w2 > 0 ? o->w2 : (int)std::min<int64_t>(ld.w3, fit.b);
@@ -516,10 +518,26 @@ PlanOptions plan_options(const hmvm_options *o, int64_t len) {
   // t_mode < 0: materialise t for every leaf.  With t in row-cluster order
   // the stage-2 factors of a cluster merge into one panel, which beats summing
   // the stage-1 partials on the fly in all three storages (measured at
-  // N = 101,250) despite the extra launch, and beats t_mode 3 (stage-1 bands
-  // writing t directly: thin bands over large clusters re-read x), also in
-  // the persistent mode, which runs the t sum as one of its stages.
+  // N = 101,250) despite the extra launch, also in the persistent mode, which
+  // runs the t sum as one of its stages.
+  // Below kBandLen elements the stage-1 tiles are bands over all columns of
+  // their cluster, so the launches write t from them and need no t sum: one
+  // launch of about 4.5 us less (enqueueing it takes the host 2.7 us).  Above,
+  // chunks of columns are faster: thin bands over large clusters read x
+  // again and again, which the wide loads of short elements hide least.
+  // Chunks -> bands, us per product: N=1,000 FP64 16.3 -> 13.9, N=4,096 FP64
+  // 23.4 -> 18.8 / FP32 22.1 -> 18.8 / BF16 24.4 -> 20.8, N=10,007 cube FP64
+  // 41.5 -> 36.0, N=20,011 (52 million elements) 89.7 -> 82.0 / 56.1 -> 53.1 /
+  // 44.7 -> 40.6, N=35,003 (83 million) 138 -> 129 / 75.5 -> 77.0 / 51.9 ->
+  // 59.9, N=60,013 (141 million) 208 -> 204 / 113 -> 116 / 74 -> 83, N=101,250
+  // 327 -> 329 / 177 -> 196 / 117 -> 147.  (Summing t inside launch B instead
+  // repeats the sums in every row tile: N=4,096 FP64 23.2 -> 30.8.)
   po.t_mode = o->t_mode >= 0 ? o->t_mode : 1;
+  po.bands = o->t_mode < 0 && len < kBandLen[storage];
+  // bands of at most 64 rows (the column-split path) balance FP64's launch A
+  // once its tiles are wide: N=20,000 57.3 -> 54.9, N=30,011 124 -> 121, N=60,013
+  // 204 -> 201; below, the width keeps them short already
+  if (po.bands && po.storage == kF64 && len >= 24000000 && o->max_rows <= 0) po.max_rows = 64;
   return po;
 }
 
@@ -738,6 +756,16 @@ int upload_values(hmvm_plan *p, const Source &src) {
   return rc;
 }
 
+// The tiles of launch `which` as its launches take them: in a plan with bands
+// the stage-1 tiles write t through their maps (the persistent launch takes
+// the plan's own, which write the slots that its t sum stage reads).
+std::vector<TileDesc> launch_list(const Plan &P, const std::vector<TileDesc> &tiles) {
+  std::vector<TileDesc> l = tiles;
+  if (P.t_bands)
+    for (TileDesc &t : l) t.map_off = t.map_off_multi;
+  return l;
+}
+
 // Whether launch A's order puts a dense tile before a stage-1 tile.
 bool order_mixed(const Plan &P) {
   for (int i = 0; i < P.n_stage1_tiles; i++)
@@ -766,7 +794,7 @@ int partition_a(hmvm_plan *p) {
         ns.push_back((uint8_t)part);
       }
   HIP_TRY(hipStreamSynchronize(p->stream));
-  HIP_TRY(hipMemcpy(p->d_tiles_a, nt.data(), sizeof(TileDesc) * nt.size(), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(p->d_tiles_a, launch_list(P, nt).data(), sizeof(TileDesc) * nt.size(), hipMemcpyHostToDevice));
   P.tiles_a.swap(nt);
   P.a_stage1.swap(ns);
   p->a_mixed = false;
@@ -828,7 +856,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
   int rc;
   const size_t eb = (size_t)elem_bytes(p->storage);
   // schedule
-  if ((rc = upload(&p->d_tiles_a, P.tiles_a)) || (rc = upload(&p->d_tiles_b, P.tiles_b)) ||
+  if ((rc = upload(&p->d_tiles_a, launch_list(P, P.tiles_a))) || (rc = upload(&p->d_tiles_b, P.tiles_b)) ||
       (rc = upload(&p->d_panels, P.panels)) ||
       (rc = upload(&p->d_ylist, P.ysum.list)) || (rc = upload(&p->d_yrng, seg_ranges(P.ysum))))
     return rc;
@@ -843,7 +871,8 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
     p->n_tsum = (int)one.size();
   }
   if (p->mode != 0 && (rc = partition_a(p.get()))) return rc;
-  if (P.t_direct && (rc = upload(&p->d_tmap, P.tmap))) return rc;
+  const bool mapped = P.t_direct || P.t_bands;  // the launches write t through the maps
+  if (mapped && (rc = upload(&p->d_tmap, P.tmap))) return rc;
   if (p->storage == kBF16) {
     if ((rc = upload(&p->d_tfac, P.factor_of_trow))) return rc;
     if ((rc = dalloc(&p->d_scales, (size_t)P.nfactors))) return rc;
@@ -862,7 +891,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
 
   // values: streamed to the GPU in windows and repacked there
   if ((rc = upload_values(p.get(), src))) return rc;
-  if (p->storage == kBF16 && P.t_direct && !P.tmap.empty()) {
+  if (p->storage == kBF16 && mapped && !P.tmap.empty()) {
     if ((rc = dalloc(&p->d_mscale, P.tmap.size()))) return rc;
     hipLaunchKernelGGL(map_scale_kernel, dim3((unsigned)((P.tmap.size() + 255) / 256)), dim3(256), 0, p->stream,
                        (int)P.tmap.size(), p->d_tmap, p->d_tfac, (const float *)p->d_scales, p->d_mscale);
@@ -874,7 +903,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
   p->device_bytes = eb * (size_t)P.nvals + sizeof(TileDesc) * (P.tiles_a.size() + P.tiles_b.size()) +
                     sizeof(PanelDesc) * P.panels.size() + 8 * (size_t)(P.n_t + 2 * P.nd) +
                     slot_bytes(p->storage) * (size_t)(P.n_tp + P.n_z) +
-                    4 * (size_t)P.n_t + (P.t_direct ? (p->d_mscale ? 12 : 4) * P.tmap.size() : 0) +
+                    4 * (size_t)P.n_t + (mapped ? (p->d_mscale ? 12 : 4) * P.tmap.size() : 0) +
                     sizeof(int2) * (size_t)p->n_tsum +
                     8 * (P.ysum.list.size() + P.ysum.seg.size());
   if (verbose())
@@ -890,7 +919,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
 // Where the tiles of one launch store their rows: the slots, and for
 // stage-1 tiles with a row map the plan's t.
 TileOut tile_out(const hmvm_plan *p, void *out, void *tout) {
-  return TileOut{out, p->d_tmap, tout, p->d_mscale};
+  return TileOut{out, p->d_tmap, tout, p->d_mscale, p->plan.t_bands ? 1 : 0};
 }
 
 // kind: unused by the one-wave-per-tile launch (kept so every launch names
@@ -1011,7 +1040,7 @@ void launch_segsum(hmvm_plan *p, int phase, double *y, int accumulate, hipStream
   const Plan &P_ = p->plan;
   const P *slots = (const P *)p->d_slots;
   if (phase == 1) {
-    if (P_.t_fused || p->n_tsum == 0) return;
+    if (P_.t_fused || P_.t_bands || p->n_tsum == 0) return;
     const dim3 grid((p->n_tsum + 255) / 256);
     if (p->storage == kBF16)
       hipLaunchKernelGGL((tsum_kernel<true, P>), grid, dim3(256), 0, st, p->n_tsum, p->d_tdesc, slots, p->d_tfac,
@@ -2464,7 +2493,7 @@ int hmvm_plan_set_tile_flags(hmvm_plan *plan, int which, const int *flags) {
   }
   TileDesc *d = which == 0 ? plan->d_tiles_a : plan->d_tiles_b;
   HIP_TRY(hipStreamSynchronize(plan->stream));
-  HIP_TRY(hipMemcpy(d, nt.data(), sizeof(TileDesc) * nt.size(), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(d, launch_list(P, nt).data(), sizeof(TileDesc) * nt.size(), hipMemcpyHostToDevice));
   tl.swap(nt);
   plan->tiles_version++;
   return plan->mode == 1 ? persist_prepare(plan) : HMVM_OK;
@@ -2491,7 +2520,7 @@ int hmvm_plan_set_tile_order(hmvm_plan *plan, int which, const int *perm) {
   for (int i = 0; i < n; i++) nt[i] = tl[perm[i]];
   TileDesc *d = which == 0 ? plan->d_tiles_a : plan->d_tiles_b;
   HIP_TRY(hipStreamSynchronize(plan->stream));
-  HIP_TRY(hipMemcpy(d, nt.data(), sizeof(TileDesc) * (size_t)n, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(d, launch_list(P, nt).data(), sizeof(TileDesc) * (size_t)n, hipMemcpyHostToDevice));
   tl.swap(nt);
   if (which == 0) {
     std::vector<uint8_t> ns((size_t)n);

@@ -118,8 +118,10 @@ typedef struct hmvm_options {
                          /* launch), 2 choose per leaf,                         */
                          /* 3 t written directly by the stage-1 tiles (bands of */
                          /* rank rows over all of a column cluster's columns;   */
-                         /* no extra launch), -1 default (1); products with     */
-                         /* several right-hand sides always materialise t       */
+                         /* no extra launch), -1 default (1; small matrices with */
+                         /* the tiles of 3, whose launches write t and need no  */
+                         /* extra one); products with several right-hand sides  */
+                         /* always materialise t                                */
   int max_rows;          /* rows per tile (0: by storage); at most 192*V-V+1,  */
                          /* V = 16 bytes / element size; when set, also for the */
                          /* stage-2 tiles unless max_rows_b is set              */
