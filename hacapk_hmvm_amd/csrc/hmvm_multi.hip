@@ -4,30 +4,32 @@
 namespace hmvm {
 
 namespace {
-template <typename S, int NB>
+template <typename S, int NB, bool kOrdered>
 void launch(const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
-  constexpr size_t lds = multi_lds_wave<S, NB>();
-  hipLaunchKernelGGL((multi_kernel<S, NB>), dim3(ngroups), dim3(64 * waves), lds * waves, st, a);
+  constexpr size_t lds = multi_lds_wave<S, NB, kOrdered>();
+  hipLaunchKernelGGL((multi_kernel<S, NB, kOrdered>), dim3(ngroups), dim3(64 * waves), lds * waves, st, a);
 }
-template <typename S>
+template <typename S, bool kOrdered>
 void launch_nb(int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
   if (nrhs == 16)
-    launch<S, 1>(a, ngroups, waves, st);
+    launch<S, 1, kOrdered>(a, ngroups, waves, st);
   else if (nrhs == 32)
-    launch<S, 2>(a, ngroups, waves, st);
+    launch<S, 2, kOrdered>(a, ngroups, waves, st);
   else
-    launch<S, 4>(a, ngroups, waves, st);
+    launch<S, 4, kOrdered>(a, ngroups, waves, st);
 }
 }  // namespace
 
-void launch_multi_groups(int storage, int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
+void launch_multi_groups(int storage, int nrhs, int which, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
   if (ngroups == 0) return;
   if (storage == kF64)
-    launch_nb<double>(nrhs, a, ngroups, waves, st);
+    launch_nb<double, false>(nrhs, a, ngroups, waves, st);
   else if (storage == kF32)
-    launch_nb<float>(nrhs, a, ngroups, waves, st);
+    launch_nb<float, false>(nrhs, a, ngroups, waves, st);
+  else if (which == 0)
+    launch_nb<uint16_t, true>(nrhs, a, ngroups, waves, st);
   else
-    launch_nb<uint16_t>(nrhs, a, ngroups, waves, st);
+    launch_nb<uint16_t, false>(nrhs, a, ngroups, waves, st);
 }
 
 void launch_multi_pack(int storage, int n, const MultiPack *recs, const void *vals, const float *scales, void *out,

@@ -5,7 +5,7 @@
 //   FP64 storage: v_mfma_f64_16x16x4_f64   (K = 4, FP64 accumulate)
 //   FP32 storage: v_mfma_f32_16x16x4_f32   (K = 4, FP32 accumulate)
 //   BF16 storage: v_mfma_f32_16x16x32_bf16 (K = 32, vector entries in BF16,
-//                 FP32 accumulate)
+//                 FP32 accumulate; stage 1 v_mfma_f32_16x16x16_bf16)
 // Operand layouts (wave64): A lane l holds row l%16 of K-slice l/16, B lane l
 // right-hand side l%16 of the same K-slice (one column for K = 4, eight for
 // K = 32); the 16x16 result gives lane l four rows of column l%16:
@@ -64,6 +64,11 @@ __device__ __forceinline__ mf_f4 mfma_step(mf_b8 a, mf_b8 b, mf_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+typedef short mf_s4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ mf_f4 mfma_step16(mf_s4 a, mf_s4 b, mf_f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
 // Halves h (0 low, 1 high) of words a and b as one word {a, b}.
 __device__ __forceinline__ uint32_t pack_half(uint32_t a, uint32_t b, int h) {
   return __builtin_amdgcn_perm(b, a, h ? 0x07060302u : 0x05040100u);
@@ -71,6 +76,7 @@ __device__ __forceinline__ uint32_t pack_half(uint32_t a, uint32_t b, int h) {
 union Bf16x8 {
   uint32_t u[4];
   mf_b8 v;
+  mf_s4 h[2];
 };
 
 // NB consecutive right-hand sides of a vector row, as loaded.
@@ -140,6 +146,7 @@ template <typename S, int NB, int NT>
 struct MultiLoads {
   typename Mfma<S>::Word a[NT][Mfma<S>::H];
   RhsWord<typename VecOf<S>::T, NB> x[Mfma<S>::KS];
+  int end;  // kOrdered: the batch ends a chunk
 };
 
 // Batches whose loads are in flight at once: two (three and four cost
@@ -168,18 +175,21 @@ constexpr bool multi_tail() {
 // tile of the one-vector launches: without, the error against 64 bits was
 // 2.6e-7 instead of 1.1e-7 at N=4,096 and 5.1e-7 instead of 3.4e-7 at
 // N=101,250; with, FP64 1.1e-7 and 1.3e-7, at 3% of the time.
-template <typename S, int NB>
+// BF16 stage 1 (kOrdered) folds a chunk at its end, into FP64 sums.
+template <typename S, int NB, bool kOrdered>
 constexpr bool multi_fold() {
-  return sizeof(S) == 4 || (sizeof(S) == 8 && NB == 1);
+  return kOrdered || sizeof(S) == 4 || (sizeof(S) == 8 && NB == 1);
 }
-template <typename S, int NB>
-using MultiSum = typename std::conditional<sizeof(S) == 4 && NB <= 2, mf_d4, typename Mfma<S>::Acc>::type;
+template <typename S, int NB, bool kOrdered>
+using MultiSum =
+    typename std::conditional<kOrdered || (sizeof(S) == 4 && NB <= 2), mf_d4, typename Mfma<S>::Acc>::type;
 
 // out += the item's columns: D batches of loads in flight, and the slices of
-// the D after those.
-template <typename S, int NB, int NT>
+// the D after those.  kOrdered (BF16 stage 1): a batch is two steps of 16
+// columns, one after the other (ordered_column).
+template <typename S, int NB, int NT, bool kOrdered>
 __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiItem &it, int lane,
-                                              MultiSum<S, NB> (&out)[NT][NB]) {
+                                              MultiSum<S, NB, kOrdered> (&out)[NT][NB]) {
   using M = Mfma<S>;
   using V = typename VecOf<S>::T;
   constexpr int KS = M::KS, E = M::E, H = M::H, nrhs = 16 * NB;
@@ -201,14 +211,17 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         l.a[t][h] = __builtin_nontemporal_load(reinterpret_cast<const typename M::Word *>(av + h * nr * E + off[t]));
     ap += kMultiBatch * KS * nr;
     const V *xr = ((s.info & kSliceT) ? T : X) + (int64_t)s.v * nrhs;
-    const int n = on ? s.info & 15 : 0;
+    l.end = on ? s.info & kSliceEnd : 0;
+    const int n = on ? s.info & 15 : 0, n2 = on ? (s.info >> 4) & 15 : 0;
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
-      load_rhs<NB>(q < n ? xr : Z, l.x[q]);  // the zero columns of a slice meet zeros
+      if (kOrdered && q == kHalf) xr += (kStep - kHalf) * nrhs;
+      const bool in_use = kOrdered && q >= kHalf ? q - kHalf < n2 : q < n;
+      load_rhs<NB>(in_use ? xr : Z, l.x[q]);  // the zero columns of a slice meet zeros
       xr += nrhs;
     }
   };
-  typename M::Acc part[multi_fold<S, NB>() ? NT : 1][NB];
+  typename M::Acc part[multi_fold<S, NB, kOrdered>() ? NT : 1][NB];
   auto clear = [&]() {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -216,7 +229,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       for (int cb = 0; cb < NB; ++cb) part[t][cb] = typename M::Acc{0, 0, 0, 0};
   };
   auto fold = [&]() {
-    if constexpr (multi_fold<S, NB>()) {
+    if constexpr (multi_fold<S, NB, kOrdered>()) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -226,7 +239,10 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       clear();
     }
   };
-  if constexpr (multi_fold<S, NB>()) clear();
+  if constexpr (multi_fold<S, NB, kOrdered>()) clear();
+  auto fold_all = [&]() {  // after D batches, where chunks do not say
+    if constexpr (!kOrdered) fold();
+  };
   auto products = [&](const MultiLoads<S, NB, NT> &l) {
     if constexpr (sizeof(S) == 2) {
 #pragma unroll
@@ -234,9 +250,22 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         Bf16x8 b;
 #pragma unroll
         for (int q = 0; q < KS; q += 2) b.u[q / 2] = pack_half(l.x[q].u[cb / 2], l.x[q + 1].u[cb / 2], cb & 1);
+        if constexpr (kOrdered) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) out[t][cb] = mfma_step(l.a[t][0], b.v, out[t][cb]);
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              Bf16x8 w;
+              w.v = l.a[t][0];
+              part[t][cb] = mfma_step16(w.h[h], b.h[h], part[t][cb]);
+            }
+        } else {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) out[t][cb] = mfma_step(l.a[t][0], b.v, out[t][cb]);
+        }
       }
+      if constexpr (kOrdered)
+        if (__builtin_amdgcn_readfirstlane(l.end)) fold();
     } else {
 #pragma unroll
       for (int q = 0; q < KS; ++q)
@@ -244,7 +273,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int cb = 0; cb < NB; ++cb)
-            if constexpr (multi_fold<S, NB>())
+            if constexpr (multi_fold<S, NB, kOrdered>())
               part[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], part[t][cb]);
             else
               out[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], out[t][cb]);
@@ -271,18 +300,18 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         load(l[d], s[d], true);
         s[d] = sl[kMultiBatch * (b + d + 2 * D < nb ? b + d + 2 * D : 0)];
       }
-      fold();
+      fold_all();
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       if (b + d < nb) products(l[d]);
       if (b + d + D < nb) load(l[d], s[d], true);
     }
-    fold();
+    fold_all();
 #pragma unroll
     for (int d = 0; d < D; ++d)
       if (b + d + D < nb) products(l[d]);
-    fold();
+    fold_all();
   } else {
     for (int b = 0; b < nb; b += D) {
 #pragma unroll
@@ -291,20 +320,22 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         load(l[d], s[d], b + d + D < nb);
         s[d] = sl[kMultiBatch * (b + d + 2 * D < nb ? b + d + 2 * D : 0)];
       }
-      fold();
+      fold_all();
     }
   }
 }
 
 // MFMA tiles whose sums of all waves are added at once: 8 KiB of LDS a wave.
-template <typename S, int NB>
+template <typename S, bool kOrdered>
+using LdsOf = typename std::conditional<kOrdered, double, typename SlotOf<S>::T>::type;
+template <typename S, int NB, bool kOrdered>
 constexpr int multi_piece() {
-  constexpr int n = 8192 / (256 * NB * (int)sizeof(typename SlotOf<S>::T));
+  constexpr int n = 8192 / (256 * NB * (int)sizeof(LdsOf<S, kOrdered>));
   return n < 1 ? 1 : n;
 }
-template <typename S, int NB>
+template <typename S, int NB, bool kOrdered>
 constexpr int multi_lds_wave() {
-  return multi_piece<S, NB>() * 256 * NB * (int)sizeof(typename SlotOf<S>::T);
+  return multi_piece<S, NB, kOrdered>() * 256 * NB * (int)sizeof(LdsOf<S, kOrdered>);
 }
 
 // W right-hand sides c.. of the t row that entry m of the row map names
@@ -323,21 +354,21 @@ __device__ __forceinline__ void store_t(const MultiArgs &a, int m, int c, double
 // One item of NT row tiles: a partial one's rows go to its slots; the kept
 // one's are added over the waves (in wave order, FP64) and go to y, t or a
 // t slot.
-template <typename S, int NB, int NT>
+template <typename S, int NB, int NT, bool kOrdered>
 __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it, int lane,
-                                           typename SlotOf<S>::T *lds) {
+                                           LdsOf<S, kOrdered> *lds) {
   using M = Mfma<S>;
   using Slot = typename SlotOf<S>::T;
   constexpr int nrhs = 16 * NB;
-  constexpr int PT = multi_piece<S, NB>() < NT ? multi_piece<S, NB>() : NT;
-  constexpr int W = 16 / (int)sizeof(Slot);  // right-hand sides a thread adds (16 bytes)
-  using Sum = MultiSum<S, NB>;
+  constexpr int PT = multi_piece<S, NB, kOrdered>() < NT ? multi_piece<S, NB, kOrdered>() : NT;
+  constexpr int W = 16 / (int)sizeof(*lds);  // right-hand sides a thread adds (16 bytes)
+  using Sum = MultiSum<S, NB, kOrdered>;
   Sum acc[NT][NB];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) acc[t][cb] = Sum{0, 0, 0, 0};
-  multi_columns<S, NB, NT>(a, it, lane, acc);
+  multi_columns<S, NB, NT, kOrdered>(a, it, lane, acc);
   if (it.kind != kItemKept) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -356,7 +387,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
     return;
   }
   const int nthreads = (int)blockDim.x, nw = nthreads >> 6, w = (int)(threadIdx.x >> 6);
-  Slot *mine = lds + w * PT * 256 * NB;
+  LdsOf<S, kOrdered> *mine = lds + w * PT * 256 * NB;
 #pragma unroll
   for (int t0 = 0; t0 < NT; t0 += PT) {
     __syncthreads();  // the previous piece is read, and this workgroup's slots are written
@@ -410,36 +441,40 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
         store_t<S, NB>(a, grp.out + row, c, s);
       } else {
         store_n<W>((Slot *)a.slots + ((int64_t)grp.out + row) * nrhs + c, s);
+        if constexpr (kOrdered) {
+#pragma unroll
+          for (int k = 0; k < W; ++k) s[k] -= (double)(Slot)s[k];
+          store_n<W>((Slot *)a.slots + ((int64_t)grp.out + grp.nrows + row) * nrhs + c, s);
+        }
       }
     }
   }
 }
 
 // multi_item for the row tiles that `rows` rows take.
-template <typename S, int NB>
+template <typename S, int NB, bool kOrdered>
 __device__ __forceinline__ void multi_item_rows(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it,
-                                                int lane, typename SlotOf<S>::T *lds) {
-  static_assert(kMultiRows <= 64, "row tiles");
+                                                int lane, LdsOf<S, kOrdered> *lds) {
+  static_assert(kMultiRows <= 64 && kOrderedRows <= 32, "row tiles");
   if (it.nrows <= 16)
-    multi_item<S, NB, 1>(a, grp, it, lane, lds);
-  else if (it.nrows <= 32)
-    multi_item<S, NB, 2>(a, grp, it, lane, lds);
+    multi_item<S, NB, 1, kOrdered>(a, grp, it, lane, lds);
+  else if (kOrdered || it.nrows <= 32)
+    multi_item<S, NB, 2, kOrdered>(a, grp, it, lane, lds);
   else if (it.nrows <= 48)
-    multi_item<S, NB, 3>(a, grp, it, lane, lds);
+    multi_item<S, NB, 3, kOrdered>(a, grp, it, lane, lds);
   else
-    multi_item<S, NB, 4>(a, grp, it, lane, lds);
+    multi_item<S, NB, 4, kOrdered>(a, grp, it, lane, lds);
 }
 
-template <typename S, int NB>
+template <typename S, int NB, bool kOrdered>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void multi_kernel(MultiArgs a) {
   extern __shared__ double multi_lds[];
-  using Slot = typename SlotOf<S>::T;
   const int lane = (int)(threadIdx.x & 63);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const MultiGroup grp = a.groups[blockIdx.x];
   const MultiWave wv = a.waves[(int)blockIdx.x * (int)(blockDim.x >> 6) + w];
   for (int i = 0; i < wv.nitems; ++i)
-    multi_item_rows<S, NB>(a, grp, a.items[wv.item0 + i], lane, (Slot *)multi_lds);
+    multi_item_rows<S, NB, kOrdered>(a, grp, a.items[wv.item0 + i], lane, (LdsOf<S, kOrdered> *)multi_lds);
 }
 
 // Packs the values of one record per workgroup (MultiPack); one thread a row
@@ -456,10 +491,13 @@ __global__ __launch_bounds__(256) void multi_pack_kernel(const MultiPack *__rest
     if (r.factor >= 0) scale = scales[r.factor];
   for (int k = (int)threadIdx.x; k < nsl * r.rows; k += (int)blockDim.x) {
     const int s = k / r.rows, row = k - s * r.rows;
-    const S *src = vals + r.src + row + (int64_t)s * KS * r.ld;
+    const S *src = vals + r.src + row;
     S v[KS];
 #pragma unroll
-    for (int q = 0; q < KS; ++q) v[q] = s * KS + q < r.cols ? src[(int64_t)q * r.ld] : S(0);
+    for (int q = 0; q < KS; ++q) {
+      const int c = r.ordered ? ordered_column(s, q) : s * KS + q;
+      v[q] = c < r.cols ? src[(int64_t)c * r.ld] : S(0);
+    }
     if constexpr (sizeof(S) == 2)  // a power of two: exact
 #pragma unroll
       for (int q = 0; q < KS; ++q) v[q] = (S)(__float_as_uint(__uint_as_float((uint32_t)v[q] << 16) * scale) >> 16);

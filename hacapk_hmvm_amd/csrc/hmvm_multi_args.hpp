@@ -31,8 +31,9 @@ struct MultiArgs {
   int y16;  // Y is 16-byte aligned
 };
 
-// One workgroup of `waves` waves per group; nrhs 16, 32 or 64.
-void launch_multi_groups(int storage, int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st);
+// One workgroup of `waves` waves per group; nrhs 16, 32 or 64; which: 0 the
+// stage-1 groups, 1 the rows of y.
+void launch_multi_groups(int storage, int nrhs, int which, const MultiArgs &a, int ngroups, int waves, hipStream_t st);
 // Packs n records' values (out: MultiPlan::nvals elements of the storage type).
 void launch_multi_pack(int storage, int n, const MultiPack *recs, const void *vals, const float *scales, void *out,
                        hipStream_t st);

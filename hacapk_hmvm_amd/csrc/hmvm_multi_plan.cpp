@@ -53,6 +53,17 @@ struct Builder {
     for (int k = 0; k < n; k += KS)
       c.slices.push_back({v + k, std::min(KS, n - k) | (t ? kSliceT : 0)});
   }
+  // The slices of a chunk of n columns of BF16 stage 1 (ordered_column).
+  void add_ordered(Columns &c, int n, int v) const {
+    for (int k = 0; k < n; k += 2 * kStep)
+      for (int s = 0; s < kMultiBatch; s++) {
+        auto in_use = [&](int first) { return std::max(0, std::min(kHalf, n - first)); };
+        const int first = k + s * kHalf;
+        // (a slice without columns stays inside the vector)
+        c.slices.push_back({first < n ? v + first : v,
+                            in_use(first) | in_use(first + kStep) << 4 | (k + 2 * kStep >= n ? kSliceEnd : 0)});
+      }
+  }
   // Places the columns of an item of nrows rows: {a0, slice0, batches}.
   struct Place {
     int64_t a0;
@@ -68,7 +79,7 @@ struct Builder {
     M.slices.insert(M.slices.end(), pad, MultiSlice{0, 0});
     for (MultiPack &r : c.pack) {
       const int last = (int)r.dst + (r.cols + KS - 1) / KS;
-      r.pad = last == n ? pad : 0;  // the records of the last columns also write the item's padding
+      if (!r.ordered) r.pad = last == n ? pad : 0;  // the records of the last columns also write the item's padding
       r.dst = p.a0 + r.dst * nrows * KS;
       r.nrows = nrows;
       M.pack.push_back(r);
@@ -215,34 +226,35 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
 
   GroupList A, Bl;
   // Adds a workgroup: each wave's own items, then its share of the kept
-  // batches, which go to the waves so that all end together.
-  auto add_group = [&](GroupList &L, MultiKind kind, int64_t out_row, int key, const Builder::Place &kept, int nrows, const std::vector<std::vector<MultiItem>> &own,
-                       const std::vector<double> &load) {
-    std::vector<int> take(nw, 0);
+  // batches, which go to the waves, `unit` at a time, so that all end together.
+  auto add_group = [&](GroupList &L, MultiKind kind, int64_t out_row, int key, const Builder::Place &kept, int nrows,
+                       const std::vector<std::vector<MultiItem>> &own, const std::vector<double> &load, int unit = 1) {
+    std::vector<int> take(nw, 0);  // in units, the last of which may be shorter
     std::vector<double> l = load;
     const double c = batch_cost(nrows);
     double total = kept.nbatch * c;
     for (double v : l) total += v;
-    int left = kept.nbatch;
+    int left = (kept.nbatch + unit - 1) / unit;
     for (int w = 0; w < nw && left > 0; w++) {
-      const int n = std::min(left, std::max(0, (int)((total / nw - l[w]) / c)));
+      const int n = std::min(left, std::max(0, (int)((total / nw - l[w]) / (c * unit))));
       take[w] = n;
-      l[w] += n * c;
+      l[w] += n * c * unit;
       left -= n;
     }
     while (left > 0) {
       const int w = (int)(std::min_element(l.begin(), l.end()) - l.begin());
       take[w]++;
-      l[w] += c;
+      l[w] += c * unit;
       left--;
     }
     int b = 0;
     for (int w = 0; w < nw; w++) {
       L.waves.push_back({(int32_t)M.items.size(), (int32_t)own[w].size() + 1});
       M.items.insert(M.items.end(), own[w].begin(), own[w].end());
-      M.items.push_back({kept.a0 + (int64_t)b * kMultiBatch * nrows * B.KS, kept.slice0 + b * kMultiBatch, take[w],
-                         nrows, -1, kItemKept, 0});
-      b += take[w];
+      const int n = std::min(take[w] * unit, kept.nbatch - b);
+      M.items.push_back({kept.a0 + (int64_t)b * kMultiBatch * nrows * B.KS, kept.slice0 + b * kMultiBatch, n, nrows, -1,
+                         kItemKept, 0});
+      b += n;
     }
     L.groups.push_back({nrows, kind, (int32_t)out_row, 0});
     L.key.push_back(key);
@@ -258,6 +270,16 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
     int key;
   };
   std::vector<Single> single;  // stacks that one wave takes
+  // rows r0.. and columns c0.. of a stack from an item's slice `first` on, a
+  // record per band; pad >= 0: ordered
+  auto pack_stack = [&](const Stack &s, int r0, int nr, int c0, int nc, int first, int pad) {
+    for (const Band &q : s.bands) {
+      const int a = std::max(q.row0, r0), e = std::min(q.row0 + q.rows, r0 + nr);
+      if (a < e)
+        col.pack.push_back({q.base + (a - q.row0) + (int64_t)c0 * q.ld, first, q.ld, e - a, nc, a - r0, 0,
+                            std::max(pad, 0), -1, pad >= 0 ? 1 : 0});
+    }
+  };
   for (const Stack &s : stacks) {
     std::vector<int32_t> trow((size_t)s.rows);
     {
@@ -267,6 +289,62 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
           if (t_idx[p.leaf] < 0) return "stage-1 rows of a leaf without a2";
           trow[(size_t)r++] = t_idx[p.leaf] + p.k0 + k;
         }
+    }
+    if (bf16) {
+      // row groups as Plan::chunk_rows has them: a leaf that fits starts a
+      // group where it would straddle two
+      std::vector<int> size(1, 0);
+      for (size_t i = 0; i < s.pieces.size();) {
+        int kt = 0;
+        for (const int leaf = s.pieces[i].leaf; i < s.pieces.size() && s.pieces[i].leaf == leaf; i++) kt += s.pieces[i].n;
+        for (int done = 0; done < kt;) {
+          const int full = size.back();
+          if (full == P.chunk_rows ||
+              (done == 0 && full > 0 && full + kt > P.chunk_rows && kt <= P.chunk_rows))
+            size.push_back(0);
+          const int take = std::min(kt - done, P.chunk_rows - size.back());
+          size.back() += take;
+          done += take;
+        }
+      }
+      const int rows = std::min(opt.rows_a, kOrderedRows);
+      int g0 = 0;
+      for (const int n : size) {
+        const int C = std::min(s.ncols, chunk_cols(n, P.chunk_w));
+        const int unit = (C + 2 * kStep - 1) / (2 * kStep);  // batches of a chunk
+        const int step = std::max({opt.cols1, s.ncols / 32768, C}) / C * C;  // (at most 32768 groups)
+        const bool direct = step >= s.ncols;
+        for (int r0 = g0; r0 < g0 + n; r0 += rows) {
+          const int nr = std::min(rows, g0 + n - r0);
+          const int64_t slot0 = M.n_slots;
+          int groups = 0;
+          for (int c0 = 0; c0 < s.ncols; c0 += step, groups++) {
+            const int end = std::min(s.ncols, c0 + step);
+            col.slices.clear();
+            col.pack.clear();
+            for (int c = c0; c < end; c += C) {
+              const int nc = std::min(C, end - c), first = (int)col.slices.size();
+              B.add_ordered(col, nc, s.col0 + c);
+              pack_stack(s, r0, nr, c, nc, first, (int)col.slices.size() - first - (nc + B.KS - 1) / B.KS);
+            }
+            const Builder::Place b = B.place(col, nr);
+            const int64_t map = (int64_t)M.tmap.size();
+            if (direct && s.ncols <= opt.wave_cols)
+              single.push_back({{b.a0, b.slice0, b.nbatch, nr, (int32_t)map, kItemT, 0}, s.col0});
+            else
+              add_group(A, direct ? kMultiT : kMultiTSlot, direct ? map : M.n_slots, s.col0 + c0, b, nr, none, idle,
+                        unit);
+            if (!direct) M.n_slots += 2 * nr;
+            if (M.n_slots > INT32_MAX) return "slots exceed int32";
+          }
+          if (direct)
+            M.tmap.insert(M.tmap.end(), trow.begin() + r0, trow.begin() + r0 + nr);
+          else
+            for (int r = 0; r < nr; r++) M.tsum.push_back({(int32_t)(slot0 + r), 2 * groups, nr, trow[(size_t)r0 + r]});
+        }
+        g0 += n;
+      }
+      continue;
     }
     const int cols1 = std::max(opt.cols1, s.ncols / 32768);  // (at most 65535 chunks)
     const int nch = (s.ncols + cols1 - 1) / cols1;
@@ -280,11 +358,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
         const int nc = std::min(s.ncols - c0, step);
         col.slices.clear();
         col.pack.clear();
-        for (const Band &q : s.bands) {
-          const int a = std::max(q.row0, r0), e = std::min(q.row0 + q.rows, r0 + nr);
-          if (a < e)
-            col.pack.push_back({q.base + (a - q.row0) + (int64_t)c0 * q.ld, 0, q.ld, e - a, nc, a - r0, 0, 0, -1, 0});
-        }
+        pack_stack(s, r0, nr, c0, nc, 0, -1);
         B.add_slices(col, nc, s.col0 + c0, false);
         const Builder::Place b = B.place(col, nr);
         if (direct && s.ncols <= opt.wave_cols)
@@ -560,7 +634,7 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
           return "wave items out of range";
         for (int i = wv.item0; i < wv.item0 + wv.nitems; i++) {
           const MultiItem &it = M.items[(size_t)i];
-          if (it.nrows < 1 || it.nrows > kMultiRows) return "item rows";
+          if (it.nrows < 1 || it.nrows > (storage == kBF16 && list == 0 ? kOrderedRows : kMultiRows)) return "item rows";
           if (it.slice0 < 0 || it.nbatch < 0 || (int64_t)it.slice0 + (int64_t)it.nbatch * kMultiBatch > nslice)
             return "item slices";
           if (it.a0 < 0 || it.a0 + (int64_t)it.nbatch * kMultiBatch * it.nrows * KS > M.nvals)
@@ -581,10 +655,16 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
           }
           for (int64_t s = it.slice0; s < it.slice0 + (int64_t)it.nbatch * kMultiBatch; s++) {
             const MultiSlice &q = M.slices[(size_t)s];
-            const int n = q.info & 15;
-            const bool t = (q.info & kSliceT) != 0;
-            if (n > KS || (t && list == 0)) return "slice";
-            if (q.v < 0 || (int64_t)q.v + n > (t ? M.n_t : (int64_t)P.nd)) return "slice outside its vector";
+            const bool t = (q.info & kSliceT) != 0, ordered = storage == kBF16 && list == 0;
+            const int n1 = q.info & 15, n2 = ordered ? (q.info >> 4) & 15 : 0, n = n1 + n2;
+            if (n > KS || (ordered && (n1 > kHalf || n2 > kHalf)) || (t && list == 0)) return "slice";
+            // a wave's columns end with a chunk, and a batch's slices agree
+            if (ordered && (q.info & kSliceEnd) != (M.slices[(size_t)((s / kMultiBatch) * kMultiBatch)].info & kSliceEnd))
+              return "chunk end";
+            if (ordered && s == it.slice0 + (int64_t)it.nbatch * kMultiBatch - 1 && !(q.info & kSliceEnd))
+              return "columns end inside a chunk";
+            if (q.v < 0 || (int64_t)q.v + (n2 > 0 ? kStep + n2 : n1) > (t ? M.n_t : (int64_t)P.nd))
+              return "slice outside its vector";
             covered += (int64_t)n * it.nrows;
           }
         }
@@ -596,6 +676,9 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
           if (e < 0 || e >= M.n_t || t_seen[(size_t)e]++) return "t row out of range or written twice";
         } else if (g.kind == kMultiTSlot && list == 0) {
           if ((int64_t)g.out + r >= M.n_slots || slot_seen[(size_t)g.out + r]++) return "t slot";
+          if (storage != kBF16) continue;
+          const int64_t low = (int64_t)g.out + g.nrows + r;  // what the FP32 slot leaves
+          if (low >= M.n_slots || slot_seen[(size_t)low]++) return "t slot";
         } else if (g.kind == kMultiY && list == 1) {
           if ((int64_t)g.out + r >= P.nd || y_seen[(size_t)g.out + r]++) return "y row out of range or written twice";
         } else {

@@ -57,9 +57,34 @@ inline int multi_word(int storage) { return storage == kF64 ? 2 : storage == kF3
 
 struct MultiSlice {
   int32_t v;     // row of X or t of the first column
-  int32_t info;  // columns in use (0..KS), bit 8: rows of t (else X)
+  int32_t info;  // columns in use (0..KS), bit 8: rows of t (else X); BF16 stage 1: see below
 };
 constexpr int kSliceT = 1 << 8;
+
+// Stage 1 of BF16 storage, whose t is rounded to BF16: a sum that lies next to
+// a rounding boundary decides an element of t, so the order of its additions
+// is part of the result (with one FP32 sum per wave, the elements of t rounded
+// the other way moved elements of y by up to 1.5e-3 of their size).  The order
+// is that of a tile of the one-vector launches at its default size: rank rows
+// in groups of at most Plan::chunk_rows that end with a leaf, a group's columns
+// in chunks (chunk_cols), a chunk one FP32 sum in steps of 16 columns
+// (v_mfma_f32_16x16x16_bf16), and the chunks added in FP64, in registers, over
+// the waves, and over a stack's groups (a group's slots are the FP32 rounding
+// of its rows, then of what that leaves).  A batch is two steps of 16 columns:
+// its slice s takes columns 4s + 0..3 and, as its second half, those + 16; info
+// holds the columns in use of each half (bits 0..3, 4..7) and whether the batch
+// ends a chunk.
+// Rows: 32, as a chunk's FP32 and FP64 sums of 64 rows and 64 right-hand sides
+// would spill.  Product at N=50,021 (cube), 16 / 32 / 64 right-hand sides: the
+// tile launches 122 / 145 / 371 us, one FP32 sum per wave 78 / 94 / 124, this
+// 85 / 106 / 138 (one wave a chunk, all chunks through FP32 slots: 91 / 115 /
+// 140, and N=4,096 29 / 40 / 46 instead of 16 / 16 / 21).
+constexpr int kSliceEnd = 1 << 9;
+constexpr int kOrderedRows = 32;
+constexpr int kHalf = 4, kStep = 16;
+constexpr int ordered_column(int slice, int q) {
+  return slice / kMultiBatch * 2 * kStep + slice % kMultiBatch * kHalf + q % kHalf + q / kHalf * kStep;
+}
 
 // nbatch batches of slices from slice0, values from a0, over nrows rows.
 // out: first slot (kItemSlot), offset in tmap (kItemT); a kept item's sum is
@@ -90,7 +115,7 @@ struct MultiPack {
   int64_t src, dst;
   int32_t ld, rows, cols, row0, nrows, pad;
   int32_t factor;  // BF16: the factor's scale goes into the values (-1: none)
-  int32_t reserved;
+  int32_t ordered; // column q of slice s is ordered_column(s, q), else s*KS + q
 };
 
 struct MultiOptions {

@@ -28,6 +28,8 @@ std::vector<std::pair<int, int>> row_chunks(int n, int mr) {
   return out;
 }
 
+}  // namespace
+
 // Columns per tile for a tile of nr rows and a target of w elements; for
 // nr <= 32 a multiple of the 64/nr lane groups.
 int chunk_cols(int nr, int w) {
@@ -38,8 +40,6 @@ int chunk_cols(int nr, int w) {
   }
   return c;
 }
-
-}  // namespace
 
 int lane_elems(int storage) { return storage == kF64 ? 2 : storage == kF32 ? 4 : 8; }
 
@@ -110,6 +110,8 @@ std::string build_plan(const LeafArrays &la, const PlanOptions &opt, Plan *plan)
   // bases are multiples of V.
   const int V = lane_elems(opt.storage);
   P.lane_elems = V;
+  P.chunk_w = opt.chunk_w;
+  P.chunk_rows = opt.chunk_rows;
   if (opt.align % V) return "alignment must be a multiple of the lane width";
   std::vector<int64_t> t_idx(nlf, -1);     // index of t_b[0] in the materialised t
   // stage-1 rows of every piece of a leaf (a leaf of more than max_rows

@@ -129,6 +129,8 @@ struct PlanOptions {
   bool bands = false;     // t_mode 1 with the stage-1 tiles of t_mode 3: one slot per t entry
   int max_rows = kMaxTileRows;  // rows per tile (rank rows per stage-1 group, leaf rows per chunk)
   int max_rows_b = 0;           // rows per stage-2 tile (0: max_rows)
+  int chunk_w = 32768;          // multi-RHS BF16 stage-1 sums: see Plan
+  int chunk_rows = kMaxTileRows;
 };
 
 struct LeafArrays {       // the caller's descriptors (matrix2 or matrix)
@@ -141,6 +143,9 @@ struct LeafArrays {       // the caller's descriptors (matrix2 or matrix)
   int64_t src_len = 0;              // length of the source buffer
 };
 
+// Columns of a chunk of nr stage-1 rows of about w elements.
+int chunk_cols(int nr, int w);
+
 // Elements a lane loads at once (16 bytes): 2 FP64, 4 FP32, 8 BF16.
 int lane_elems(int storage);
 
@@ -148,6 +153,10 @@ struct Plan {
   int nd = 0, nlf = 0;
   int lane_elems = 2;                // column strides and factor bases are multiples of this
   int max_rows = kMaxTileRows;       // rows per tile
+  // BF16 products with several right-hand sides: rank rows of a column cluster
+  // in groups of at most chunk_rows, a group's columns in chunks of chunk_cols(
+  // rows, chunk_w); a chunk is one FP32 sum (see hmvm_multi_plan.hpp)
+  int chunk_w = 0, chunk_rows = 0;
   int64_t nvals = 0;                 // device value buffer (elements)
   int64_t len = 0;                   // reference element count
   int nfactors = 0;

@@ -534,6 +534,13 @@ PlanOptions plan_options(const hmvm_options *o, int64_t len) {
   // repeats the sums in every row tile: N=4,096 FP64 23.2 -> 30.8.)
   po.t_mode = o->t_mode >= 0 ? o->t_mode : 1;
   po.bands = o->t_mode < 0 && len < kBandLen[storage];
+  // A BF16 product with several right-hand sides rounds t to BF16, so its
+  // stage-1 sums keep their order: that of tiles of len / 4096 elements (of
+  // the caller's, where set), whatever the one-vector launches take.
+  po.chunk_w = po.t_mode == 3 ? 1 << 30
+               : o->w1 > 0    ? o->w1
+                              : (int)std::min<int64_t>(ld.w1, std::max<int64_t>(1024, len / 4096));
+  po.chunk_rows = po.max_rows;
   // bands of at most 64 rows (the column-split path) balance FP64's launch A
   // once its tiles are wide: N=20,000 57.3 -> 54.9, N=30,011 124 -> 121, N=60,013
   // 204 -> 201; below, the width keeps them short already
@@ -1226,7 +1233,7 @@ void launch_multi_part(hmvm_plan *p, int which, const void *X, double *Y, int nr
   a.accumulate = accumulate;
   a.y16 = ((uintptr_t)Y & 15) == 0;
   if (p->multi_windows.empty()) {
-    launch_multi_groups(p->storage, nrhs, a, which ? p->n_mgroups_b : p->n_mgroups_a, p->multi_waves, st);
+    launch_multi_groups(p->storage, nrhs, which, a, which ? p->n_mgroups_b : p->n_mgroups_a, p->multi_waves, st);
     return;
   }
   for (const MultiWindow &w : p->multi_windows) {
@@ -1237,7 +1244,7 @@ void launch_multi_part(hmvm_plan *p, int which, const void *X, double *Y, int nr
     a.vals = vals;
     a.groups = groups + w.group0;
     a.waves = waves + (size_t)w.group0 * p->multi_waves;
-    launch_multi_groups(p->storage, nrhs, a, w.ngroups, p->multi_waves, st);
+    launch_multi_groups(p->storage, nrhs, which, a, w.ngroups, p->multi_waves, st);
   }
 }
 
