@@ -44,28 +44,28 @@ int hip_fail(const char *what, hipError_t e) {
 
 constexpr int kBlock = 256;
 constexpr int kDotBlocks = 512;
+constexpr size_t kScalarDoubles = 4 * kDotBlocks + 16;  // two arrays of partials, the scalars
 
-// device scalars
+// Device scalars.  A kernel's block 0 writes what later kernels need, in
+// words of that kernel alone: every block of a kernel reads the words of the
+// kernels before it and computes the same values from them, so no block waits
+// for another.
 enum {
-  kAlpha = 0, kBeta, kZeta, kZnomOld, kRnorm, kBnorm,
-  kStop,   // 0 running, 1 converged, 2 breakdown
-  kIters,  // iterations that updated u
+  kBnorm = 0, kRho, kRnorm, kStopP, kItersP,  // bicg_p (kBnorm: the first one)
+  kAlpha, kRhoOld, kStopT,                    // bicg_t
+  kZeta, kStopU, kItersU,                     // bicg_update
+  kOutStop, kOutIters, kOutRnorm, kOutBnorm,  // bicg_state, for the host
   kNumScalars
 };
+static_assert(4 * kDotBlocks + kNumScalars <= kScalarDoubles, "work space of the scalars");
+// stop words: 0 running, 1 converged, 2 breakdown; iterations counted once
+// they have updated u
 
-// partial[blockIdx] = (sum a*b, sum c*d) over a grid-stride slice
-__global__ __launch_bounds__(kBlock) void dot2_partial(int n, const double *__restrict__ a,
-                                                       const double *__restrict__ b,
-                                                       const double *__restrict__ c,
-                                                       const double *__restrict__ d, double *__restrict__ part) {
+// Sums of (v0, v1) over the block's threads in a fixed tree, on every thread.
+__device__ __forceinline__ double2 block_sum(double v0, double v1) {
   __shared__ double s0[kBlock], s1[kBlock];
-  double x0 = 0, x1 = 0;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    x0 += a[i] * b[i];
-    x1 += c[i] * d[i];
-  }
-  s0[threadIdx.x] = x0;
-  s1[threadIdx.x] = x1;
+  s0[threadIdx.x] = v0;
+  s1[threadIdx.x] = v1;
   __syncthreads();
   for (int s = kBlock / 2; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) {
@@ -74,79 +74,45 @@ __global__ __launch_bounds__(kBlock) void dot2_partial(int n, const double *__re
     }
     __syncthreads();
   }
+  const double2 r = make_double2(s0[0], s1[0]);
+  __syncthreads();  // the arrays may be used again
+  return r;
+}
+
+__device__ __forceinline__ void put_partial(double *__restrict__ part, double2 d) {
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s0[0];
-    part[2 * blockIdx.x + 1] = s1[0];
+    part[2 * blockIdx.x] = d.x;
+    part[2 * blockIdx.x + 1] = d.y;
   }
+}
+
+// The dot products whose partials a kernel of as many blocks left, by every
+// block that uses them: at most kDotBlocks pairs from the cache, against a
+// launch of one block between producer and consumer (4.6 us each, four an
+// iteration; N=20,000).
+__device__ __forceinline__ double2 sum_partials(const double *__restrict__ part) {
+  double x0 = 0, x1 = 0;
+  for (int i = threadIdx.x; i < (int)gridDim.x; i += kBlock) {
+    x0 += part[2 * i];
+    x1 += part[2 * i + 1];
+  }
+  return block_sum(x0, x1);
+}
+
+// partial[block] = (sum a*b, sum a*c) over a grid-stride slice
+__global__ __launch_bounds__(kBlock) void dot2_partial(int n, const double *__restrict__ a,
+                                                       const double *__restrict__ b,
+                                                       const double *__restrict__ c, double *__restrict__ part) {
+  double x0 = 0, x1 = 0;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    x0 += a[i] * b[i];
+    x1 += a[i] * c[i];
+  }
+  put_partial(part, block_sum(x0, x1));
 }
 
 __device__ __forceinline__ bool below_tol(double rnorm, double bnorm, double tol) {
   return rnorm / (bnorm > 0.0 ? bnorm : 1.0) < tol;
-}
-
-// Reduces the partials and updates the scalars:
-//   op 0 (start):  bnorm = sqrt(d0)               [d0 = (b,b)]
-//   op 1 (rnorm):  rnorm = sqrt(d0)               [d0 = (r,r)], stop if below tol
-//   op 2 (alpha):  alpha = d0/d1, znomold = d0    [(s,r), (s,Ap)]
-//   op 3 (zeta):   zeta = d0/d1                   [(At,t), (At,At)]
-//   op 4 (beta):   beta = alpha/zeta*d0/znomold, rnorm = sqrt(d1), iters += 1,
-//                  stop if below tol              [(s,r), (r,r)]
-// Ops 2-4 do nothing once the stop word is set; a non-finite alpha, zeta,
-// beta or rnorm sets it to 2.
-__global__ __launch_bounds__(kBlock) void dot2_finish(int nblk, const double *__restrict__ part, int op,
-                                                      double tol, double *__restrict__ S) {
-  __shared__ double s0[kBlock], s1[kBlock];
-  if (op >= 2 && S[kStop] != 0.0) return;  // uniform over the block
-  double x0 = 0, x1 = 0;
-  for (int i = threadIdx.x; i < nblk; i += kBlock) {
-    x0 += part[2 * i];
-    x1 += part[2 * i + 1];
-  }
-  s0[threadIdx.x] = x0;
-  s1[threadIdx.x] = x1;
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      s0[threadIdx.x] += s0[threadIdx.x + s];
-      s1[threadIdx.x] += s1[threadIdx.x + s];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    const double d0 = s0[0], d1 = s1[0];
-    switch (op) {
-      case 0: S[kBnorm] = sqrt(d0); break;
-      case 1:
-        S[kRnorm] = sqrt(d0);
-        if (below_tol(S[kRnorm], S[kBnorm], tol)) S[kStop] = 1.0;
-        break;
-      case 2: {
-        const double al = d0 / d1;
-        S[kAlpha] = al;
-        S[kZnomOld] = d0;
-        if (!isfinite(al)) S[kStop] = 2.0;
-        break;
-      }
-      case 3: {
-        const double ze = d0 / d1;
-        S[kZeta] = ze;
-        if (!isfinite(ze)) S[kStop] = 2.0;
-        break;
-      }
-      default: {
-        const double be = S[kAlpha] / S[kZeta] * d0 / S[kZnomOld];
-        const double rn = sqrt(d1);
-        S[kBeta] = be;
-        S[kRnorm] = rn;
-        S[kIters] += 1.0;
-        if (below_tol(rn, S[kBnorm], tol))
-          S[kStop] = 1.0;  // the reference leaves the loop before beta is used
-        else if (!isfinite(rn) || !isfinite(be))
-          S[kStop] = 2.0;
-        break;
-      }
-    }
-  }
 }
 
 // S = 0 (a kernel rather than a memset, so that no memset node enters a
@@ -155,44 +121,123 @@ __global__ void bicg_scalars_zero(double *__restrict__ S) {
   if (threadIdx.x < kNumScalars) S[threadIdx.x] = 0.0;
 }
 
-// r = b - r (r holds A u on entry), shadow = r, p = 0, Ap = 0
+// r = b - r (r holds A u on entry), shadow = r; partials (b,b), (r,r)
 __global__ __launch_bounds__(kBlock) void bicg_init(int n, const double *__restrict__ b, double *__restrict__ r,
-                                                    double *__restrict__ sh, double *__restrict__ p,
-                                                    double *__restrict__ ap) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const double v = b[i] - r[i];
-  r[i] = v;
-  sh[i] = v;
-  p[i] = 0.0;
-  ap[i] = 0.0;
+                                                    double *__restrict__ sh, double *__restrict__ part) {
+  double x0 = 0, x1 = 0;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    const double v = b[i] - r[i];
+    r[i] = v;
+    sh[i] = v;
+    x0 += b[i] * b[i];
+    x1 += v * v;
+  }
+  put_partial(part, block_sum(x0, x1));
 }
 
-// p = r + beta*(p - zeta*Ap)
+// The state between two iterations, d = (b,b), (r,r) after the start or
+// (s,r), (r,r) after an update: residual norm, stop word, rho = (s,r), beta.
+struct Between {
+  double bnorm, rho, rnorm, beta, stop;
+};
+__device__ __forceinline__ Between between(double2 d, double tol, const double *__restrict__ S) {
+  Between w;
+  const bool first = S[kItersU] == 0.0;
+  w.bnorm = first ? sqrt(d.x) : S[kBnorm];
+  w.rho = first ? d.y : d.x;  // the shadow is the first r
+  w.rnorm = sqrt(d.y);
+  w.beta = first ? 0.0 : S[kAlpha] / S[kZeta] * w.rho / S[kRhoOld];
+  w.stop = below_tol(w.rnorm, w.bnorm, tol) ? 1.0  // the reference leaves the loop before beta is used
+           : !first && (!isfinite(w.rnorm) || !isfinite(w.beta)) ? 2.0
+                                                                 : 0.0;
+  return w;
+}
+
+// p = r + beta*(p - zeta*Ap); p = r in the first iteration
 __global__ __launch_bounds__(kBlock) void bicg_p(int n, const double *__restrict__ r, double *__restrict__ p,
-                                                 const double *__restrict__ ap, const double *__restrict__ S) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n || S[kStop] != 0.0) return;
-  p[i] = r[i] + S[kBeta] * (p[i] - S[kZeta] * ap[i]);
+                                                 const double *__restrict__ ap, const double *__restrict__ part,
+                                                 double tol, double *__restrict__ S) {
+  const bool first = S[kItersU] == 0.0, stopped = S[kStopU] != 0.0;  // uniform over the grid
+  Between w{};
+  if (!stopped) w = between(sum_partials(part), tol, S);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[kStopP] = stopped ? S[kStopU] : w.stop;
+    S[kItersP] = S[kItersU];
+    if (!stopped) {
+      S[kRho] = w.rho;
+      S[kRnorm] = w.rnorm;
+      if (first) S[kBnorm] = w.bnorm;
+    }
+  }
+  if (stopped || w.stop != 0.0) return;
+  const double ze = S[kZeta];
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+    p[i] = first ? r[i] : r[i] + w.beta * (p[i] - ze * ap[i]);
 }
 
-// t = r - alpha*Ap
+// The state for the host, as the next bicg_p would find it.
+__global__ __launch_bounds__(kBlock) void bicg_state(int nblk, const double *__restrict__ part, double tol,
+                                                     double *__restrict__ S) {
+  double x0 = 0, x1 = 0;
+  for (int i = threadIdx.x; i < nblk; i += kBlock) {  // sum_partials of the larger grid
+    x0 += part[2 * i];
+    x1 += part[2 * i + 1];
+  }
+  const double2 d = block_sum(x0, x1);
+  if (threadIdx.x != 0) return;
+  const bool stopped = S[kStopU] != 0.0;
+  const Between w = between(d, tol, S);
+  S[kOutStop] = stopped ? S[kStopU] : w.stop;
+  S[kOutIters] = S[kItersU];
+  S[kOutRnorm] = stopped ? S[kRnorm] : w.rnorm;
+  S[kOutBnorm] = stopped ? S[kBnorm] : w.bnorm;
+}
+
+// alpha = rho/(s,Ap); t = r - alpha*Ap
 __global__ __launch_bounds__(kBlock) void bicg_t(int n, const double *__restrict__ r, const double *__restrict__ ap,
-                                                 double *__restrict__ t, const double *__restrict__ S) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n || S[kStop] != 0.0) return;
-  t[i] = r[i] - S[kAlpha] * ap[i];
+                                                 double *__restrict__ t, const double *__restrict__ part,
+                                                 double *__restrict__ S) {
+  const bool stopped = S[kStopP] != 0.0;
+  const double rho = S[kRho], al = rho / sum_partials(part).x;
+  const double stop = stopped ? S[kStopP] : isfinite(al) ? 0.0 : 2.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[kStopT] = stop;
+    if (!stopped) {
+      S[kAlpha] = al;
+      S[kRhoOld] = rho;
+    }
+  }
+  if (stop != 0.0) return;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) t[i] = r[i] - al * ap[i];
 }
 
-// u += alpha*p + zeta*t ; r = t - zeta*At
+// zeta = (At,t)/(At,At); u += alpha*p + zeta*t ; r = t - zeta*At; partials
+// (s,r), (r,r)
 __global__ __launch_bounds__(kBlock) void bicg_update(int n, double *__restrict__ u, const double *__restrict__ p,
                                                       const double *__restrict__ t, const double *__restrict__ at,
-                                                      double *__restrict__ r, const double *__restrict__ S) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n || S[kStop] != 0.0) return;
-  const double al = S[kAlpha], ze = S[kZeta];
-  u[i] = u[i] + al * p[i] + ze * t[i];
-  r[i] = t[i] - ze * at[i];
+                                                      double *__restrict__ r, const double *__restrict__ sh,
+                                                      const double *__restrict__ part, double *__restrict__ part_r,
+                                                      double *__restrict__ S) {
+  const bool stopped = S[kStopT] != 0.0;
+  const double2 d = sum_partials(part);
+  const double ze = d.x / d.y;
+  const double stop = stopped ? S[kStopT] : isfinite(ze) ? 0.0 : 2.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[kStopU] = stop;
+    S[kItersU] = S[kItersP] + (stop == 0.0 ? 1.0 : 0.0);
+    if (!stopped) S[kZeta] = ze;
+  }
+  if (stop != 0.0) return;  // uniform over the grid
+  const double al = S[kAlpha];
+  double x0 = 0, x1 = 0;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    u[i] = u[i] + al * p[i] + ze * t[i];
+    const double v = t[i] - ze * at[i];
+    r[i] = v;
+    x0 += sh[i] * v;
+    x1 += v * v;
+  }
+  put_partial(part_r, block_sum(x0, x1));
 }
 
 // Device vectors and scalars of one solve: b and u are the caller's (or
@@ -204,41 +249,48 @@ struct Solver {
   hipStream_t st = nullptr;
   const double *b = nullptr;
   double *u = nullptr, *r = nullptr, *sh = nullptr, *p = nullptr, *ap = nullptr, *t = nullptr, *at = nullptr,
-         *part = nullptr, *S = nullptr;
-  int nblk() const { return std::min(kDotBlocks, (n + kBlock - 1) / kBlock); }
-  dim3 grid() const { return dim3((n + kBlock - 1) / kBlock); }
+         *part = nullptr, *part_r = nullptr, *S = nullptr;
+  // one grid for all kernels: a kernel sums as many partials as it has blocks
+  dim3 grid() const { return dim3(std::min(kDotBlocks, (n + kBlock - 1) / kBlock)); }
 
-  void dots(const double *a, const double *bb, const double *c, const double *d, int op) {
-    hipLaunchKernelGGL(dot2_partial, dim3(nblk()), dim3(kBlock), 0, st, n, a, bb, c, d, part);
-    hipLaunchKernelGGL(dot2_finish, dim3(1), dim3(kBlock), 0, st, nblk(), part, op, tol, S);
+  // Divides work space (6 n vectors, 2 arrays of partials, the scalars).
+  void place(double *w) {
+    const size_t m = (size_t)n;
+    r = w;
+    sh = w + m;
+    p = w + 2 * m;
+    ap = w + 3 * m;
+    t = w + 4 * m;
+    at = w + 5 * m;
+    part = w + 6 * m;
+    part_r = part + 2 * kDotBlocks;
+    S = part_r + 2 * kDotBlocks;
   }
-  // r = b - A u ; shadow = r ; p = Ap = 0 ; norms (m_HACApK_solve.f90:326-339)
+  // r = b - A u ; shadow = r ; norms (m_HACApK_solve.f90:326-339)
   int start() {
     hipLaunchKernelGGL(bicg_scalars_zero, dim3(1), dim3(64), 0, st, S);
-    dots(b, b, b, b, 0);
     int rc = hmvm_plan_apply(plan, u, r, 0, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(bicg_init, grid(), dim3(kBlock), 0, st, n, b, r, sh, p, ap);
-    dots(r, r, r, r, 1);
+    hipLaunchKernelGGL(bicg_init, grid(), dim3(kBlock), 0, st, n, b, r, sh, part_r);
     KRY_TRY(hipGetLastError());
     return HMVM_OK;
   }
   // one BiCGSTAB iteration (m_HACApK_solve.f90:341-372)
   int iterate() {
-    hipLaunchKernelGGL(bicg_p, grid(), dim3(kBlock), 0, st, n, r, p, ap, S);
+    hipLaunchKernelGGL(bicg_p, grid(), dim3(kBlock), 0, st, n, r, p, ap, part_r, tol, S);
     int rc = hmvm_plan_apply(plan, p, ap, 0, st);
     if (rc) return rc;
-    dots(sh, r, sh, ap, 2);
-    hipLaunchKernelGGL(bicg_t, grid(), dim3(kBlock), 0, st, n, r, ap, t, S);
+    hipLaunchKernelGGL(dot2_partial, grid(), dim3(kBlock), 0, st, n, sh, ap, ap, part);
+    hipLaunchKernelGGL(bicg_t, grid(), dim3(kBlock), 0, st, n, r, ap, t, part, S);
     rc = hmvm_plan_apply(plan, t, at, 0, st);
     if (rc) return rc;
-    dots(at, t, at, at, 3);
-    hipLaunchKernelGGL(bicg_update, grid(), dim3(kBlock), 0, st, n, u, p, t, at, r, S);
-    dots(sh, r, r, r, 4);
+    hipLaunchKernelGGL(dot2_partial, grid(), dim3(kBlock), 0, st, n, at, t, at, part);
+    hipLaunchKernelGGL(bicg_update, grid(), dim3(kBlock), 0, st, n, u, p, t, at, r, sh, part, part_r, S);
     KRY_TRY(hipGetLastError());
     return HMVM_OK;
   }
   int read_scalars(double *S_host) {
+    hipLaunchKernelGGL(bicg_state, dim3(1), dim3(kBlock), 0, st, (int)grid().x, part_r, tol, S);
     KRY_TRY(hipMemcpyAsync(S_host, S, sizeof(double) * kNumScalars, hipMemcpyDeviceToHost, st));
     KRY_TRY(hipStreamSynchronize(st));
     return HMVM_OK;
@@ -253,10 +305,12 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
   int rc = s.start();
   if (rc) return rc;
   double S0[kNumScalars];
-  if ((rc = s.read_scalars(S0))) return rc;
+  // the graph is made while the device works on the start (N=20,000: 60 us
+  // of the 100 to 150 us that capture and instantiation take); a start that
+  // is already converged leaves it unused
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
-  if (use_graph && S0[kStop] == 0.0 && max_iter > 0) {
+  if (use_graph && max_iter > 0) {
     KRY_TRY(hipStreamBeginCapture(s.st, hipStreamCaptureModeThreadLocal));
     rc = s.iterate();
     const hipError_t e = hipStreamEndCapture(s.st, &graph);
@@ -270,6 +324,16 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
       return hip_fail("hipGraphInstantiate", ei);
     }
   }
+  rc = s.read_scalars(S0);
+  if (!rc && S0[kOutStop] != 0.0 && gexec) {  // no iteration to launch
+    (void)hipGraphExecDestroy(gexec);
+    gexec = nullptr;
+  }
+  if (rc) {
+    if (gexec) (void)hipGraphExecDestroy(gexec);
+    if (graph) (void)hipGraphDestroy(graph);
+    return rc;
+  }
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (timed) {
     (void)hipEventCreate(&e0);
@@ -277,7 +341,7 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
     (void)hipEventRecord(e0, s.st);
   }
   int launched = 0;
-  while (launched < max_iter && S0[kStop] == 0.0) {
+  while (launched < max_iter && S0[kOutStop] == 0.0) {
     const int chunk = check_every > 0 ? std::min(check_every, max_iter - launched) : max_iter - launched;
     for (int c = 0; c < chunk && !rc; c++) {
       if (gexec) {
@@ -300,14 +364,14 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
   if (gexec) (void)hipGraphExecDestroy(gexec);
   if (graph) (void)hipGraphDestroy(graph);
   if (rc) return rc;
-  const double bnorm = S0[kBnorm] > 0 ? S0[kBnorm] : 1.0;
-  res->iters = (int)S0[kIters];
+  const double bnorm = S0[kOutBnorm] > 0 ? S0[kOutBnorm] : 1.0;
+  res->iters = (int)S0[kOutIters];
   res->hmvms = 2 * res->iters + 1;
-  res->relres = S0[kRnorm] / bnorm;
+  res->relres = S0[kOutRnorm] / bnorm;
   res->ms_loop = ms;
   res->ms_per_iter = launched > 0 ? ms / launched : 0.0;
   res->graph_used = gexec ? 1 : 0;
-  if (S0[kStop] == 2.0) {
+  if (S0[kOutStop] == 2.0) {
     char m[256];
     std::snprintf(m, sizeof m, "BiCGSTAB broke down after %d iterations (zero divisor or non-finite scalar)",
                   res->iters);
@@ -332,34 +396,24 @@ extern "C" int hmvm_bicgstab(hmvm_plan *plan, const double *b_host, double *u_ho
   s.tol = tol;
   s.plan = plan;
   const size_t nb = sizeof(double) * (size_t)s.n;
-  // b, u, the six work vectors, the dot partials and the scalars
+  // work space, b and u, in one allocation
   struct Buffers {
-    double *d[10] = {};
+    double *d = nullptr;
     hipStream_t st = nullptr;
     ~Buffers() {
       if (st) (void)hipStreamSynchronize(st);
-      for (double *q : d)
-        if (q) (void)hipFree(q);
+      if (d) (void)hipFree(d);
       if (st) (void)hipStreamDestroy(st);
     }
   } m;
   KRY_TRY(hipStreamCreate(&m.st));
-  for (int i = 0; i < 10; i++) {
-    const size_t bytes = i < 8 ? nb : i == 8 ? sizeof(double) * 2 * kDotBlocks : sizeof(double) * kNumScalars;
-    KRY_TRY(hipMalloc(&m.d[i], bytes));
-  }
+  const size_t work = 6 * (size_t)s.n + kScalarDoubles;
+  KRY_TRY(hipMalloc(&m.d, sizeof(double) * (work + 2 * (size_t)s.n)));
   s.st = m.st;
-  s.b = m.d[0];
-  s.u = m.d[1];
-  s.r = m.d[2];
-  s.sh = m.d[3];
-  s.p = m.d[4];
-  s.ap = m.d[5];
-  s.t = m.d[6];
-  s.at = m.d[7];
-  s.part = m.d[8];
-  s.S = m.d[9];
-  KRY_TRY(hipMemcpyAsync(m.d[0], b_host, nb, hipMemcpyHostToDevice, s.st));
+  s.place(m.d);
+  s.b = m.d + work;
+  s.u = m.d + work + s.n;
+  KRY_TRY(hipMemcpyAsync(m.d + work, b_host, nb, hipMemcpyHostToDevice, s.st));
   KRY_TRY(hipMemcpyAsync(s.u, u_host, nb, hipMemcpyHostToDevice, s.st));
   rc = solve(s, max_iter, use_graph, check_every, true, res);
   if (rc == HMVM_OK || rc == HMVM_ERR_BREAKDOWN) {
@@ -372,11 +426,11 @@ extern "C" int hmvm_bicgstab(hmvm_plan *plan, const double *b_host, double *u_ho
 // ---- the allocation-free variant ----------------------------------------------
 // Work space of hmvm_bicgstab_static: the six work vectors of a solve of at
 // most kStaticMaxN unknowns, the dot partials and the scalars, in one array
-// of the library's code object (48 MiB + 8 KiB; each device the library runs
+// of the library's code object (48 MiB + 16 KiB; each device the library runs
 // on holds its own copy until the process ends).  Every call on a device
 // uses that device's copy: calls that overlap on one device race.
 constexpr int kStaticMaxN = HMVM_BICGSTAB_STATIC_MAX_N;
-constexpr size_t kScratchDoubles = 6 * (size_t)kStaticMaxN + 2 * kDotBlocks + kNumScalars;
+constexpr size_t kScratchDoubles = 6 * (size_t)kStaticMaxN + kScalarDoubles;
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 namespace {
@@ -429,14 +483,6 @@ extern "C" int hmvm_bicgstab_static(hmvm_plan *plan, const double *d_b, double *
   s.st = (hipStream_t)stream;
   s.b = d_b;
   s.u = d_u;
-  const size_t n = (size_t)s.n;
-  s.r = w;
-  s.sh = w + n;
-  s.p = w + 2 * n;
-  s.ap = w + 3 * n;
-  s.t = w + 4 * n;
-  s.at = w + 5 * n;
-  s.part = w + 6 * n;
-  s.S = s.part + 2 * kDotBlocks;
+  s.place(w);
   return solve(s, max_iter, 0, check_every, false, res);
 }
