@@ -865,6 +865,18 @@ __global__ __launch_bounds__(256) void flush_kernel(double4 *__restrict__ dst, s
     dst[i] = double4{v, v, v, v};
 }
 
+// dst = src, n doubles (both 16-byte aligned), one of them in pinned host
+// memory: one load per thread, all in flight at once (the link's latency, not
+// its rate, is what vectors of this size cost).
+__global__ __launch_bounds__(256) void stage_copy_kernel(double *__restrict__ dst, const double *__restrict__ src,
+                                                         size_t n) {
+  const size_t i = 2 * (blockIdx.x * (size_t)blockDim.x + threadIdx.x);
+  if (i + 1 < n)
+    *reinterpret_cast<double2 *>(dst + i) = *reinterpret_cast<const double2 *>(src + i);
+  else if (i < n)
+    dst[i] = src[i];
+}
+
 // y sum: out[i] = (accumulate ? out[i] : 0) + ysum_entry(i) for the n rows.
 template <typename P>
 __global__ __launch_bounds__(256) void ysum_kernel(int n, const int2 *__restrict__ rng,

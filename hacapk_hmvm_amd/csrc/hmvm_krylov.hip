@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "hmvm_hip.h"
+#include "hmvm_stage.hpp"
 #include "hmvm_status.hpp"
 
 namespace {
@@ -54,10 +55,12 @@ enum {
   kBnorm = 0, kRho, kRnorm, kStopP, kItersP,  // bicg_p (kBnorm: the first one)
   kAlpha, kRhoOld, kStopT,                    // bicg_t
   kZeta, kStopU, kItersU,                     // bicg_update
-  kOutStop, kOutIters, kOutRnorm, kOutBnorm,  // bicg_state, for the host
   kNumScalars
 };
-static_assert(4 * kDotBlocks + kNumScalars <= kScalarDoubles, "work space of the scalars");
+// what bicg_state writes for the host
+enum { kOutStop = 0, kOutIters, kOutRnorm, kOutBnorm, kNumOut };
+static_assert(4 * kDotBlocks + kNumScalars + kNumOut <= kScalarDoubles && 2 + kNumOut <= hmvm::kStageTail,
+              "work space of the scalars");
 // stop words: 0 running, 1 converged, 2 breakdown; iterations counted once
 // they have updated u
 
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(kBlock) void bicg_p(int n, const double *__restrict
 
 // The state for the host, as the next bicg_p would find it.
 __global__ __launch_bounds__(kBlock) void bicg_state(int nblk, const double *__restrict__ part, double tol,
-                                                     double *__restrict__ S) {
+                                                     const double *__restrict__ S, double *__restrict__ out) {
   double x0 = 0, x1 = 0;
   for (int i = threadIdx.x; i < nblk; i += kBlock) {  // sum_partials of the larger grid
     x0 += part[2 * i];
@@ -187,10 +190,10 @@ __global__ __launch_bounds__(kBlock) void bicg_state(int nblk, const double *__r
   if (threadIdx.x != 0) return;
   const bool stopped = S[kStopU] != 0.0;
   const Between w = between(d, tol, S);
-  S[kOutStop] = stopped ? S[kStopU] : w.stop;
-  S[kOutIters] = S[kItersU];
-  S[kOutRnorm] = stopped ? S[kRnorm] : w.rnorm;
-  S[kOutBnorm] = stopped ? S[kBnorm] : w.bnorm;
+  out[kOutStop] = stopped ? S[kStopU] : w.stop;
+  out[kOutIters] = S[kItersU];
+  out[kOutRnorm] = stopped ? S[kRnorm] : w.rnorm;
+  out[kOutBnorm] = stopped ? S[kBnorm] : w.bnorm;
 }
 
 // alpha = rho/(s,Ap); t = r - alpha*Ap
@@ -250,6 +253,7 @@ struct Solver {
   const double *b = nullptr;
   double *u = nullptr, *r = nullptr, *sh = nullptr, *p = nullptr, *ap = nullptr, *t = nullptr, *at = nullptr,
          *part = nullptr, *part_r = nullptr, *S = nullptr;
+  double *host_out = nullptr;  // pinned: where bicg_state writes (else behind S, and copied)
   // one grid for all kernels: a kernel sums as many partials as it has blocks
   dim3 grid() const { return dim3(std::min(kDotBlocks, (n + kBlock - 1) / kBlock)); }
 
@@ -289,10 +293,13 @@ struct Solver {
     KRY_TRY(hipGetLastError());
     return HMVM_OK;
   }
-  int read_scalars(double *S_host) {
-    hipLaunchKernelGGL(bicg_state, dim3(1), dim3(kBlock), 0, st, (int)grid().x, part_r, tol, S);
-    KRY_TRY(hipMemcpyAsync(S_host, S, sizeof(double) * kNumScalars, hipMemcpyDeviceToHost, st));
+  int read_state(double *state) {
+    double *out = host_out ? host_out : S + kNumScalars;
+    hipLaunchKernelGGL(bicg_state, dim3(1), dim3(kBlock), 0, st, (int)grid().x, part_r, tol, S, out);
+    KRY_TRY(hipGetLastError());
+    if (!host_out) KRY_TRY(hipMemcpyAsync(state, out, sizeof(double) * kNumOut, hipMemcpyDeviceToHost, st));
     KRY_TRY(hipStreamSynchronize(st));
+    if (host_out) std::memcpy(state, host_out, sizeof(double) * kNumOut);
     return HMVM_OK;
   }
 };
@@ -304,7 +311,7 @@ struct Solver {
 int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, hmvm_krylov_result *res) {
   int rc = s.start();
   if (rc) return rc;
-  double S0[kNumScalars];
+  double S0[kNumOut];
   // the graph is made while the device works on the start (N=20,000: 60 us
   // of the 100 to 150 us that capture and instantiation take); a start that
   // is already converged leaves it unused
@@ -324,7 +331,7 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
       return hip_fail("hipGraphInstantiate", ei);
     }
   }
-  rc = s.read_scalars(S0);
+  rc = s.read_state(S0);
   if (!rc && S0[kOutStop] != 0.0 && gexec) {  // no iteration to launch
     (void)hipGraphExecDestroy(gexec);
     gexec = nullptr;
@@ -352,7 +359,7 @@ int solve(Solver &s, int max_iter, int use_graph, int check_every, bool timed, h
     }
     if (rc) break;
     launched += chunk;
-    if ((rc = s.read_scalars(S0))) break;
+    if ((rc = s.read_state(S0))) break;
   }
   float ms = 0;
   if (timed) {
@@ -396,28 +403,44 @@ extern "C" int hmvm_bicgstab(hmvm_plan *plan, const double *b_host, double *u_ho
   s.tol = tol;
   s.plan = plan;
   const size_t nb = sizeof(double) * (size_t)s.n;
-  // work space, b and u, in one allocation
+  // work space, b and u, in one allocation; the plan's stream
   struct Buffers {
     double *d = nullptr;
     hipStream_t st = nullptr;
     ~Buffers() {
-      if (st) (void)hipStreamSynchronize(st);
+      (void)hipStreamSynchronize(st);
       if (d) (void)hipFree(d);
-      if (st) (void)hipStreamDestroy(st);
     }
   } m;
-  KRY_TRY(hipStreamCreate(&m.st));
-  const size_t work = 6 * (size_t)s.n + kScalarDoubles;
-  KRY_TRY(hipMalloc(&m.d, sizeof(double) * (work + 2 * (size_t)s.n)));
+  m.st = hmvm::plan_stream(plan);
+  // b and u start on 16 bytes, on the device and in pinned memory: n rounded up to even
+  const size_t n = (size_t)s.n, ne = n + n % 2, work = 6 * ne + kScalarDoubles;
+  KRY_TRY(hipMalloc(&m.d, sizeof(double) * (work + 2 * ne)));
   s.st = m.st;
   s.place(m.d);
-  s.b = m.d + work;
-  s.u = m.d + work + s.n;
-  KRY_TRY(hipMemcpyAsync(m.d + work, b_host, nb, hipMemcpyHostToDevice, s.st));
-  KRY_TRY(hipMemcpyAsync(s.u, u_host, nb, hipMemcpyHostToDevice, s.st));
+  double *b = m.d + work;
+  s.b = b;
+  s.u = b + ne;
+  double *h = hmvm::plan_stage(plan);
+  if (h) {
+    std::memcpy(h, b_host, nb);
+    std::memcpy(h + ne, u_host, nb);
+    hmvm::stage_copy(b, h, ne + n, s.st);
+    s.host_out = h + 2 * ne;
+  } else {
+    KRY_TRY(hipMemcpyAsync(b, b_host, nb, hipMemcpyHostToDevice, s.st));
+    KRY_TRY(hipMemcpyAsync(s.u, u_host, nb, hipMemcpyHostToDevice, s.st));
+  }
   rc = solve(s, max_iter, use_graph, check_every, true, res);
   if (rc == HMVM_OK || rc == HMVM_ERR_BREAKDOWN) {
-    const hipError_t e = hipMemcpy(u_host, s.u, nb, hipMemcpyDeviceToHost);
+    hipError_t e;
+    if (h) {
+      hmvm::stage_copy(h + ne, s.u, n, s.st);
+      e = hipStreamSynchronize(s.st);
+      if (e == hipSuccess) std::memcpy(u_host, h + ne, nb);
+    } else {
+      e = hipMemcpy(u_host, s.u, nb, hipMemcpyDeviceToHost);
+    }
     if (e != hipSuccess) rc = hip_fail("hipMemcpy (u)", e);
   }
   return rc;
