@@ -6,8 +6,8 @@ profiles/ and the traffic record bench.py reads.
         --grid-a THREADS --grid-b THREADS [--md OUT.md] [--json OUT.json] [--cmd "..."]
     python -m hacapk_hmvm_amd.rocprof_summary --mfma DIR [--md OUT.md] [--cmd "..."]
 
-The two tile launches of one HMVM run the same kernel (tile_kernel, or
-tile_multi_kernel for several right-hand sides); they are told apart by
+The two large launches of one HMVM run the same kernel (tile_kernel, or
+multi_kernel for several right-hand sides); they are told apart by
 their grid size (threads = 256 * ceil(tiles / 4) with 256-thread workgroups).
 Counter values are KiB per dispatch; they are scaled by what the same counter
 reads for the bandwidth-probe kernels of bench.py, which read (probe_read) and
@@ -46,7 +46,7 @@ def trace_table(rows):
     by = {}
     for r in rows:
         k = short(r["Kernel_Name"])
-        key = (k, int(r["Grid_Size_X"]) if k.startswith(("tile_kernel", "tile_multi_kernel")) else 0)
+        key = (k, int(r["Grid_Size_X"]) if k.startswith(("tile_kernel", "tile_multi_kernel", "multi_kernel")) else 0)
         by.setdefault(key, []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
     return by
 
@@ -62,7 +62,7 @@ def counters(rows, counter):
 
 
 def mfma_table(d, nxcd=8, nsimd=1024):
-    """MFMA busy share and MFMA FLOPs of the tile_multi_kernel launches from a
+    """MFMA busy share and MFMA FLOPs of the multi_kernel launches from a
     --pmc run of SQ_VALU_MFMA_BUSY_CYCLES, SQ_INSTS_VALU_MFMA_MOPS_{F64,F32,
     BF16} and GRBM_GUI_ACTIVE: busy % = MFMA busy cycles summed over the SIMDs
     / (GRBM_GUI_ACTIVE per XCD x SIMDs); GRBM_GUI_ACTIVE is read summed over
@@ -70,7 +70,7 @@ def mfma_table(d, nxcd=8, nsimd=1024):
     by = {}
     for r in read_csv(d, "_counter_collection.csv"):
         k = short(r["Kernel_Name"])
-        if not k.startswith("tile_multi_kernel"):
+        if not k.startswith(("tile_multi_kernel", "multi_kernel")):
             continue
         by.setdefault((k, int(r["Grid_Size"])), {}).setdefault(r["Counter_Name"], []).append(float(r["Counter_Value"]))
     lines = ["| kernel | grid | MFMA busy % | MFMA GFLOP per launch |", "|---|---|---|---|"]
