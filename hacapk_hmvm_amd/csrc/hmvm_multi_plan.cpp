@@ -179,6 +179,10 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
       opt.cols1 < 1)
     return "bad multi-RHS options";
   Builder B(storage, M);
+  // (address space alone: what is not used is never touched)
+  M.slices.reserve((size_t)(P.nvals / (16 * B.KS)) + 64);
+  M.pack.reserve(4 * P.repack.size());
+  M.items.reserve(4 * P.repack.size());
   const int nw = opt.waves;
   const bool bf16 = storage == kBF16;
 
