@@ -160,7 +160,12 @@ struct GroupList {
 //   wave_cols  one wave a stack saves the sum over the waves, but a launch of
 //          a small matrix then lasts as long as its longest stack (N=4,096,
 //          FP64, 16 right-hand sides: 256 columns 0.038, 32 columns 0.025;
-//          N=101,250: 32 columns 0.548, 256 columns 0.542).
+//          N=101,250: 32 columns 0.548, 256 columns 0.542);
+//   cols1  stacks up to so many columns need no slots and no t sum; beyond
+//          2048 a launch lasts as long as its widest stacks (32 right-hand
+//          sides, 1024 / 2048 / 4096 / 8192 columns, us: N=20,011 FP32 120 /
+//          118 / 117 / 117, BF16 81 / 77 / 78 / 78; N=101,250 FP64 547 / 545 /
+//          545 / 614, BF16 with 16 164 / 161 / 163 / 192).
 MultiOptions multi_options(const Plan &P) {
   MultiOptions o;
   o.rows = P.nd >= 16384 ? 64 : P.nd >= 2048 ? 32 : 16;

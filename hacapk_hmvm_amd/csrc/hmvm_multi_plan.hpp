@@ -122,7 +122,7 @@ struct MultiOptions {
   int rows = kMultiRows;    // most rows of a row group
   int rows_a = kMultiRows;  // most rank rows of a stage-1 group
   int waves = 4;            // waves per workgroup
-  int cols1 = 1024;         // most columns of a stage-1 group
+  int cols1 = 2048;         // most columns of a stage-1 group
   int wave_cols = 256;      // stage-1 stacks of at most so many columns are one wave's
 };
 
