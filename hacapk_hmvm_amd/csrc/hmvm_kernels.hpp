@@ -1,8 +1,9 @@
 // hmvm_kernels.hpp -- gfx950 device code of the HMVM (included by the runtime).
 //
 // Kernel roles (one HMVM = four launches on one stream; three when no leaf
-// reads a materialised t, t_mode 0):
-//   tile_kernel (launch A)  stage-1 slots = stacked a1 panels x x-slices,
+// reads a materialised t, t_mode 0, or the stage-1 tiles write t: t_mode 3 and
+// the default of small matrices):
+//   tile_kernel (launch A)  stage-1 slots (or t) = stacked a1 panels x x-slices,
 //                           dense slots   = transposed dense leaves x x-slices
 //   [tsum_kernel            t = sum of stage-1 slots            (fixed order)]
 //   tile_kernel (launch B)  stage-2 slots = a2 panels x t (the materialised t,

@@ -6,13 +6,13 @@
 // the residual norm, the stop state and the iteration count) stays in device
 // memory, so one iteration is a fixed sequence of launches with no host
 // synchronisation; with use_graph the iteration is captured once into a
-// hipGraph and replayed.  Dot products are two-pass (per-block partials, then
-// one block) and therefore deterministic: the eager and the graph-replayed
-// solve give the same bits.
+// hipGraph and replayed.  A dot product is per-block partials, summed in one
+// fixed tree by every block of the kernel that needs it, and therefore
+// deterministic: the eager and the graph-replayed solve give the same bits.
 //
 // Stopping: the reference leaves its loop at the top of the first iteration
 // whose ||r||/||b|| is below eps (m_HACApK_solve.f90:342).  Here the kernel
-// that computes ||r|| sets a device stop word instead, and every later update
+// that finds ||r|| sets a device stop word instead, and every later update
 // kernel and scalar update returns at once, so the host may launch whole
 // chunks of iterations between its read-backs and still get the reference's
 // iterate and iteration count.  A zero divisor or a non-finite scalar sets

@@ -1066,8 +1066,8 @@ void launch_segsum(hmvm_plan *p, int phase, double *y, int accumulate, hipStream
 }
 
 // Launch `phase` of one HMVM: 0 = tiles A (stage 1 + dense), 1 = t segment sum
-// (only when some leaf's rank rows straddle two row groups), 2 = tiles B
-// (stage 2), 3 = y segment sum.
+// (none where launch A writes t or launch B sums the slots itself), 2 = tiles
+// B (stage 2), 3 = y segment sum.
 void launch_phase(hmvm_plan *p, int phase, const double *x, double *y, int accumulate, hipStream_t st) {
   if (phase == 0 || phase == 2) {
     const int which = phase == 0 ? 0 : 1;
