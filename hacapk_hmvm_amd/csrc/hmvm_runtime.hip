@@ -477,8 +477,8 @@ const LaunchDefaults &launch_defaults(int storage) {
 // tiles, which end early), then 7168.  Launch B has about a third of the
 // elements and takes 6144 tiles of all elements, two per three of its slots;
 // tiles of 64 (FP64) or 96 (FP32) rows make as many of them from the large
-// clusters; BF16 tiles stay longer (two-byte values: no gain below 84 million
-// elements).  Measured on 14 matrices of 1 to 241 million elements against
+// clusters; BF16's take launch A's width up to 126 million elements (shorter
+// ones lost 2.5 to 4% on matrices of leaf size 16).  Measured on 14 matrices of 1 to 241 million elements against
 // one tile per slot throughout and the large matrices' rows: FP64 1.085,
 // FP32 1.070, BF16 1.021 times faster (geometric means; none slower by more
 // than 0.6%), ms per product: N=20,000 sphere FP64 0.071 -> 0.062, N=30,011
@@ -486,7 +486,7 @@ const LaunchDefaults &launch_defaults(int storage) {
 // cube FP64 0.186 -> 0.165 and FP32 0.113 -> 0.094, N=60,013 (leaf 64) BF16
 // 0.087 -> 0.075.
 constexpr int64_t kKneeA[3] = {8192, 8192, 20480};  // FP64, FP32, BF16
-constexpr int64_t kBandLen[3] = {200000000, 64000000, 64000000};  // see plan_options
+constexpr int64_t kBandLen[3] = {200000000, 64000000, 40000000};  // see plan_options
 struct FitWidths {
   int64_t a, b;  // stage-1 and dense tiles, stage-2 tiles
   int rows_b;    // rows of a stage-2 tile
@@ -495,7 +495,7 @@ FitWidths fit_widths(int storage, int64_t len, int rows_b) {
   const int64_t fit = std::max<int64_t>(1024, len / 4096);
   FitWidths w;
   w.a = std::min(fit, std::max(kKneeA[storage], len / 7168));
-  w.b = storage == kBF16 ? std::min(fit, std::max<int64_t>(10240, len / 6144)) : std::max<int64_t>(1024, len / 6144);
+  w.b = storage == kBF16 ? std::min(fit, std::max(kKneeA[storage], len / 6144)) : std::max<int64_t>(1024, len / 6144);
   w.rows_b = len >= 200000000 || storage == kBF16 ? rows_b : storage == kF64 ? 64 : 96;
   return w;
 }
@@ -532,10 +532,12 @@ PlanOptions plan_options(const hmvm_options *o, int64_t len) {
   // Chunks -> bands, us per product: N=1,000 FP64 16.3 -> 13.9, N=4,096 FP64
   // 23.4 -> 18.8 / FP32 22.1 -> 18.8 / BF16 24.4 -> 20.8, N=10,007 cube FP64
   // 41.5 -> 36.0, N=20,011 (52 million elements) 89.7 -> 82.0 / 56.1 -> 53.1 /
-  // 44.7 -> 40.6, N=35,003 (83 million) 138 -> 129 / 75.5 -> 77.0 / 51.9 ->
-  // 59.9, N=60,013 (141 million) 208 -> 204 / 113 -> 116 / 74 -> 83, N=101,250
-  // 327 -> 329 / 177 -> 196 / 117 -> 147.  (Summing t inside launch B instead
-  // repeats the sums in every row tile: N=4,096 FP64 23.2 -> 30.8.)
+  // 44.7 -> 40.6 (BF16 on cubes of 53 and 58 million elements 39.2 -> 41.6 and
+  // 45.1 -> 47.7: its line lies at 40 million), N=35,003 (83 million) 138 -> 129
+  // / 75.5 -> 77.0 / 51.9 -> 59.9, N=60,013 (141 million) 208 -> 204 / 113 -> 116
+  // / 74 -> 83, N=101,250 327 -> 329 / 177 -> 196 / 117 -> 147.  (Summing t inside
+  // launch B instead repeats the sums in every row tile: N=4,096 FP64 23.2 ->
+  // 30.8.)
   po.t_mode = o->t_mode >= 0 ? o->t_mode : 1;
   po.bands = o->t_mode < 0 && len < kBandLen[storage];
   // A BF16 product with several right-hand sides rounds t to BF16, so its
