@@ -901,14 +901,14 @@ __global__ __launch_bounds__(256) void tsum_kernel(int n, const int2 *__restrict
 }
 
 // tsum_kernel for nrhs right-hand sides (rows of nrhs in buf and out) over
-// the n entries listed in desc (entry = d.z): a thread sums W consecutive
-// right-hand sides with 16-byte loads (W = 2 for FP64 slots, 4 for FP32).
-template <bool kScaled, typename P, typename O>
+// the n entries listed in desc (entry = d.z): a thread sums two consecutive
+// right-hand sides with 16-byte loads.
+template <bool kScaled, typename O>
 __global__ __launch_bounds__(256) void tsum_multi_kernel(int n, int nrhs, const int4 *__restrict__ desc,
-                                                         const P *__restrict__ buf,
+                                                         const double *__restrict__ buf,
                                                          const int32_t *__restrict__ factor_of,
                                                          const float *__restrict__ scales, O *__restrict__ out) {
-  constexpr int W = 16 / sizeof(P);
+  constexpr int W = 2;
   const int nw = nrhs / W;
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= (int64_t)n * nw) return;

@@ -6,8 +6,7 @@ namespace hmvm {
 namespace {
 template <typename S, int NB, bool kOrdered>
 void launch(const MultiArgs &a, int ngroups, int waves, hipStream_t st) {
-  constexpr size_t lds = multi_lds_wave<S, NB, kOrdered>();
-  hipLaunchKernelGGL((multi_kernel<S, NB, kOrdered>), dim3(ngroups), dim3(64 * waves), lds * waves, st, a);
+  hipLaunchKernelGGL((multi_kernel<S, NB, kOrdered>), dim3(ngroups), dim3(64 * waves), (size_t)kMultiLdsWave * waves, st, a);
 }
 template <typename S, bool kOrdered>
 void launch_nb(int nrhs, const MultiArgs &a, int ngroups, int waves, hipStream_t st) {

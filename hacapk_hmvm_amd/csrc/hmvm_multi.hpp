@@ -326,17 +326,14 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
 }
 
 // MFMA tiles whose sums of all waves are added at once: 8 KiB of LDS a wave.
-template <typename S, bool kOrdered>
-using LdsOf = typename std::conditional<kOrdered, double, typename SlotOf<S>::T>::type;
-template <typename S, int NB, bool kOrdered>
+// LDS words and slots are FP64 in all storages: a wave's share of a group's
+// columns may add up to more than FLT_MAX where the rows of y, or t scaled by
+// its leaf's factors, are finite numbers.
+template <int NB>
 constexpr int multi_piece() {
-  constexpr int n = 8192 / (256 * NB * (int)sizeof(LdsOf<S, kOrdered>));
-  return n < 1 ? 1 : n;
+  return 4 / NB;
 }
-template <typename S, int NB, bool kOrdered>
-constexpr int multi_lds_wave() {
-  return multi_piece<S, NB, kOrdered>() * 256 * NB * (int)sizeof(LdsOf<S, kOrdered>);
-}
+constexpr int kMultiLdsWave = 8192;  // bytes
 
 // W right-hand sides c.. of the t row that entry m of the row map names
 // (BF16: times both factor scales of its leaf).
@@ -356,12 +353,11 @@ __device__ __forceinline__ void store_t(const MultiArgs &a, int m, int c, double
 // t slot.
 template <typename S, int NB, int NT, bool kOrdered>
 __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it, int lane,
-                                           LdsOf<S, kOrdered> *lds) {
+                                           double *lds) {
   using M = Mfma<S>;
-  using Slot = typename SlotOf<S>::T;
   constexpr int nrhs = 16 * NB;
-  constexpr int PT = multi_piece<S, NB, kOrdered>() < NT ? multi_piece<S, NB, kOrdered>() : NT;
-  constexpr int W = 16 / (int)sizeof(*lds);  // right-hand sides a thread adds (16 bytes)
+  constexpr int PT = multi_piece<NB>() < NT ? multi_piece<NB>() : NT;
+  constexpr int W = 2;  // right-hand sides a thread adds (16 bytes)
   using Sum = MultiSum<S, NB, kOrdered>;
   Sum acc[NT][NB];
 #pragma unroll
@@ -380,14 +376,14 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
 #pragma unroll
         for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[t][cb][v];
         if (it.kind == kItemSlot)
-          store_n<NB>((Slot *)a.slots + ((int64_t)it.out + row) * nrhs + NB * (lane & 15), r);
+          store_n<NB>(a.slots + ((int64_t)it.out + row) * nrhs + NB * (lane & 15), r);
         else
           store_t<S, NB>(a, it.out + row, NB * (lane & 15), r);
       }
     return;
   }
   const int nthreads = (int)blockDim.x, nw = nthreads >> 6, w = (int)(threadIdx.x >> 6);
-  LdsOf<S, kOrdered> *mine = lds + w * PT * 256 * NB;
+  double *mine = lds + w * PT * 256 * NB;
 #pragma unroll
   for (int t0 = 0; t0 < NT; t0 += PT) {
     __syncthreads();  // the previous piece is read, and this workgroup's slots are written
@@ -420,7 +416,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
         const int2 rg = a.yrng[y];
         for (int l = rg.x; l < rg.y; ++l) {
           double r[W];
-          load_n<W>((const Slot *)a.slots + (a.ylist[l] + y) * nrhs + c, r);
+          load_n<W>(a.slots + (a.ylist[l] + y) * nrhs + c, r);
 #pragma unroll
           for (int k = 0; k < W; ++k) s[k] += r[k];
         }
@@ -440,12 +436,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
       } else if (grp.kind == kMultiT) {
         store_t<S, NB>(a, grp.out + row, c, s);
       } else {
-        store_n<W>((Slot *)a.slots + ((int64_t)grp.out + row) * nrhs + c, s);
-        if constexpr (kOrdered) {
-#pragma unroll
-          for (int k = 0; k < W; ++k) s[k] -= (double)(Slot)s[k];
-          store_n<W>((Slot *)a.slots + ((int64_t)grp.out + grp.nrows + row) * nrhs + c, s);
-        }
+        store_n<W>(a.slots + ((int64_t)grp.out + row) * nrhs + c, s);
       }
     }
   }
@@ -454,7 +445,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
 // multi_item for the row tiles that `rows` rows take.
 template <typename S, int NB, bool kOrdered>
 __device__ __forceinline__ void multi_item_rows(const MultiArgs &a, const MultiGroup &grp, const MultiItem &it,
-                                                int lane, LdsOf<S, kOrdered> *lds) {
+                                                int lane, double *lds) {
   static_assert(kMultiRows <= 64 && kOrderedRows <= 32, "row tiles");
   if (it.nrows <= 16)
     multi_item<S, NB, 1, kOrdered>(a, grp, it, lane, lds);
@@ -474,7 +465,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void m
   const MultiGroup grp = a.groups[blockIdx.x];
   const MultiWave wv = a.waves[(int)blockIdx.x * (int)(blockDim.x >> 6) + w];
   for (int i = 0; i < wv.nitems; ++i)
-    multi_item_rows<S, NB, kOrdered>(a, grp, a.items[wv.item0 + i], lane, (LdsOf<S, kOrdered> *)multi_lds);
+    multi_item_rows<S, NB, kOrdered>(a, grp, a.items[wv.item0 + i], lane, multi_lds);
 }
 
 // Packs the values of one record per workgroup (MultiPack); one thread a row

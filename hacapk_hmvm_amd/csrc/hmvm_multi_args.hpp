@@ -20,7 +20,7 @@ struct MultiArgs {
   const void *__restrict__ X;
   const void *T;             // t (written by launch A, read by launch B)
   const void *__restrict__ zero;  // kMultiZeroBytes of zeros: what columns and batches past the last one read
-  void *slots;
+  double *slots;
   void *t_out;
   const int32_t *__restrict__ tmap;
   const double *__restrict__ mscale;  // BF16: both factor scales of every tmap row's leaf

@@ -343,13 +343,13 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
             else
               add_group(A, direct ? kMultiT : kMultiTSlot, direct ? map : M.n_slots, s.col0 + c0, b, nr, none, idle,
                         unit);
-            if (!direct) M.n_slots += 2 * nr;
+            if (!direct) M.n_slots += nr;
             if (M.n_slots > INT32_MAX) return "slots exceed int32";
           }
           if (direct)
             M.tmap.insert(M.tmap.end(), trow.begin() + r0, trow.begin() + r0 + nr);
           else
-            for (int r = 0; r < nr; r++) M.tsum.push_back({(int32_t)(slot0 + r), 2 * groups, nr, trow[(size_t)r0 + r]});
+            for (int r = 0; r < nr; r++) M.tsum.push_back({(int32_t)(slot0 + r), groups, nr, trow[(size_t)r0 + r]});
         }
         g0 += n;
       }
@@ -685,9 +685,6 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
           if (e < 0 || e >= M.n_t || t_seen[(size_t)e]++) return "t row out of range or written twice";
         } else if (g.kind == kMultiTSlot && list == 0) {
           if ((int64_t)g.out + r >= M.n_slots || slot_seen[(size_t)g.out + r]++) return "t slot";
-          if (storage != kBF16) continue;
-          const int64_t low = (int64_t)g.out + g.nrows + r;  // what the FP32 slot leaves
-          if (low >= M.n_slots || slot_seen[(size_t)low]++) return "t slot";
         } else if (g.kind == kMultiY && list == 1) {
           if ((int64_t)g.out + r >= P.nd || y_seen[(size_t)g.out + r]++) return "y row out of range or written twice";
         } else {

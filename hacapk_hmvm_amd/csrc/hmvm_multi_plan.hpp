@@ -69,8 +69,7 @@ constexpr int kSliceT = 1 << 8;
 // in groups of at most Plan::chunk_rows that end with a leaf, a group's columns
 // in chunks (chunk_cols), a chunk one FP32 sum in steps of 16 columns
 // (v_mfma_f32_16x16x16_bf16), and the chunks added in FP64, in registers, over
-// the waves, and over a stack's groups (a group's slots are the FP32 rounding
-// of its rows, then of what that leaves).  A batch is two steps of 16 columns:
+// the waves, and over a stack's groups.  A batch is two steps of 16 columns:
 // its slice s takes columns 4s + 0..3 and, as its second half, those + 16; info
 // holds the columns in use of each half (bits 0..3, 4..7) and whether the batch
 // ends a chunk.

@@ -168,7 +168,7 @@ struct hmvm_plan {
   int32_t *d_pptr_a = nullptr, *d_pptr_b = nullptr;       // wave w's tiles: [ptr[w], ptr[w+1])
   // several right-hand sides: buffers sized for multi_cap columns
   int multi_cap = 0;
-  void *d_mslots = nullptr;  // slot_bytes(storage) per slot
+  double *d_mslots = nullptr;
   void *d_mt = nullptr;      // t: vec_bytes(storage) per entry
   void *d_mXc = nullptr;     // X in the operand type (FP32 and BF16 storage)
   std::vector<int> nstrtl, nstrtt;  // first row and column of every leaf, for the schedule below
@@ -1186,12 +1186,11 @@ int multi_buffers(hmvm_plan *p, int nrhs) {
   void *bufs[5] = {p->d_mslots, p->d_mt, p->d_mX, p->d_mY, p->d_mXc};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
-  p->d_mslots = p->d_mt = nullptr;
-  p->d_mX = p->d_mY = nullptr;
-  p->d_mXc = nullptr;
+  p->d_mslots = p->d_mX = p->d_mY = nullptr;
+  p->d_mt = p->d_mXc = nullptr;
   p->multi_cap = 0;
   int rc;
-  if ((rc = dalloc_bytes(&p->d_mslots, slot_bytes(p->storage) * (size_t)p->n_mslots * nrhs)) ||
+  if ((rc = dalloc(&p->d_mslots, (size_t)p->n_mslots * nrhs)) ||
       (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)p->n_mt * nrhs)) ||
       (rc = dalloc(&p->d_mX, (size_t)P.nd * nrhs)) || (rc = dalloc(&p->d_mY, (size_t)P.nd * nrhs)))
     return rc;
@@ -1254,22 +1253,21 @@ void launch_multi_part(hmvm_plan *p, int which, const void *X, double *Y, int nr
   }
 }
 
-// Multi-RHS t sum over slots of type P.
-template <typename P>
 void launch_tsum_multi(hmvm_plan *p, int nrhs, hipStream_t st) {
   const int n = p->n_mtsum;
   if (n == 0) return;
-  const P *slots = (const P *)p->d_mslots;
   // 16-byte loads and stores (slots and t are the plan's own allocations); t
   // in the multi-RHS operand type (VecOf: FP64, FP32 or BF16 bits)
-  const int64_t tw = (int64_t)n * (nrhs / (16 / (int)sizeof(P)));
-  const dim3 grid((unsigned)((tw + 255) / 256));
-  if (p->storage == kBF16)
-    hipLaunchKernelGGL((tsum_multi_kernel<true, P, uint16_t>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, slots,
-                       p->d_mtfac, p->d_scales, (uint16_t *)p->d_mt);
+  const dim3 grid((unsigned)(((int64_t)n * (nrhs / 2) + 255) / 256));
+  if (p->storage == kF64)
+    hipLaunchKernelGGL((tsum_multi_kernel<false, double>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, p->d_mslots,
+                       (const int32_t *)nullptr, (const float *)nullptr, (double *)p->d_mt);
+  else if (p->storage == kF32)
+    hipLaunchKernelGGL((tsum_multi_kernel<false, float>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, p->d_mslots,
+                       (const int32_t *)nullptr, (const float *)nullptr, (float *)p->d_mt);
   else
-    hipLaunchKernelGGL((tsum_multi_kernel<false, P, P>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, slots,
-                       (const int32_t *)nullptr, (const float *)nullptr, (P *)p->d_mt);
+    hipLaunchKernelGGL((tsum_multi_kernel<true, uint16_t>), grid, dim3(256), 0, st, n, nrhs, p->d_mtsum, p->d_mslots,
+                       p->d_mtfac, p->d_scales, (uint16_t *)p->d_mt);
 }
 
 // Phase 0: the operand copy of X (FP32 and BF16 storage) and launch A, 1: the
@@ -1277,13 +1275,7 @@ void launch_tsum_multi(hmvm_plan *p, int nrhs, hipStream_t st) {
 void launch_multi_phase(hmvm_plan *p, int phase, const double *X, double *Y, int nrhs, int accumulate,
                         hipStream_t st) {
   const Plan &P = p->plan;
-  if (phase == 1) {
-    if (p->storage == kF64)
-      launch_tsum_multi<double>(p, nrhs, st);
-    else
-      launch_tsum_multi<float>(p, nrhs, st);
-    return;
-  }
+  if (phase == 1) return launch_tsum_multi(p, nrhs, st);
   if (phase == 3) return;
   if (phase == 0 && p->storage != kF64) {
     // the groups read X and t in the operand type
