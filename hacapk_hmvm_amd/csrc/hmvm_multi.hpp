@@ -167,14 +167,20 @@ constexpr bool multi_tail() {
   return sizeof(S) == 4 || (sizeof(S) == 2 && NB == 4);
 }
 
-// Whether the MFMA sums of a few batches are folded into sums of their own:
-// FP32 storage (FP64 sums up to 32 right-hand sides, FP32 for 64: no registers
-// for more), and FP64 storage with 16 right-hand sides, the only case with
-// registers for it.
 // An even share of a group's columns is a longer chain of roundings than a
-// tile of the one-vector launches: without, the error against 64 bits was
-// 2.6e-7 instead of 1.1e-7 at N=4,096 and 5.1e-7 instead of 3.4e-7 at
-// N=101,250; with, FP64 1.1e-7 and 1.3e-7, at 3% of the time.
+// tile of the one-vector launches, so the MFMA sums of a few batches are
+// folded into sums of their own (FP64; FP32 storage with 64 right-hand sides
+// FP32): for FP32 storage the error against 64 bits was 2.6e-7 without instead
+// of 1.1e-7 at N=4,096 and 5.1e-7 instead of 3.4e-7 at N=101,250; with, 1.1e-7
+// and 1.3e-7, at 3% of the time.
+// multi_fold: whether a second set of sums for all tiles does that, every
+// multi_depth batches; FP64 storage has the registers for it with 16 right-hand
+// sides only (with 32, 540 -> 650 us at N=101,250) and otherwise folds each
+// batch of each MFMA tile: error at N=12,007 / 101,250 6.9e-16 / 1.02e-15 ->
+// 2.4e-16 / 3.3e-16 (the tile launches 4.0e-16 / 7.1e-16), us with 32 right-hand
+// sides 93 / 540 -> 95 / 538, with 64 146 / 811 -> 163 / 854.  Without the
+// barriers between the tiles the compiler keeps several sums and spills (32:
+// 100 / 560, 64: 165 / 928).
 // BF16 stage 1 (kOrdered) folds a chunk at its end, into FP64 sums.
 template <typename S, int NB, bool kOrdered>
 constexpr bool multi_fold() {
@@ -266,17 +272,25 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       }
       if constexpr (kOrdered)
         if (__builtin_amdgcn_readfirstlane(l.end)) fold();
-    } else {
+    } else if constexpr (multi_fold<S, NB, kOrdered>()) {
 #pragma unroll
       for (int q = 0; q < KS; ++q)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int cb = 0; cb < NB; ++cb)
-            if constexpr (multi_fold<S, NB, kOrdered>())
-              part[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], part[t][cb]);
-            else
-              out[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], out[t][cb]);
+          for (int cb = 0; cb < NB; ++cb) part[t][cb] = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], part[t][cb]);
+    } else {  // one MFMA tile after the other, so that one sum of the batch is live at a time
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) {
+          typename M::Acc sum{0, 0, 0, 0};
+#pragma unroll
+          for (int q = 0; q < KS; ++q) sum = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], sum);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) out[t][cb][v] += sum[v];
+          __builtin_amdgcn_sched_barrier(0);
+        }
     }
   };
   constexpr int D = multi_depth<S, NB>();

@@ -83,3 +83,36 @@ def test_rows_of_y_above_the_fp32_range(gpu, H, O, tmp_path, storage, nrhs):
     for c in (0, nrhs - 1):
         ref = O.seq_2(h, np.ascontiguousarray(X[:, c]))
         assert np.linalg.norm(Y[:, c] * 1e-30 - ref * 1e-30) <= TOL[storage] * np.linalg.norm(ref * 1e-30)
+
+
+def long_sums(H, path, big, nrhs, stage1):
+    """64 leaves of 64 columns side by side, all ones, X one but for `big` in
+    the first row.  Dense leaves (64 rows taller than a group and 20 rows that
+    are part of one), or one stack of rank 32 of which y is the first row."""
+    leaves = [(2, m, 64, r, 1 + 64 * q, 0) for m, r in ((64, 1), (20, 101)) for q in range(64)]
+    if stage1:
+        leaves = [(1, 64, 4096, 1, 1, 32), (1, 20, 4096, 101, 1, 32)]
+    write_format1(path, ND, leaves, np.random.default_rng(1))
+    h = H.loadHmatrix(path)
+    a = h.arrays()
+    for v in (a["rowmat"], a["rowmat_t"]):
+        v[:] = 1.0
+    if stage1:
+        for i, (_, m, _, _, _, k) in enumerate(leaves):
+            a["rowmat"][a["a2"][i] + m:a["a2"][i] + m * k] = 0.0
+    X = np.ones((ND, nrhs))
+    X[0] = big
+    return h, X
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nrhs", [16, 32, 64])
+@pytest.mark.parametrize("storage,big,stage1", [("f64", 2.0**53, False), ("f64", 2.0**53, True)])
+def test_chains_of_roundings_stay_short(gpu, H, tmp_path, storage, big, stage1, nrhs):
+    """Ones added to a number of which one is half the last bit are lost, and
+    kept in sums of their own: of 4,096 columns no more than the 64 of a leaf
+    may be added in the same chain as the first."""
+    h, X = long_sums(H, str(tmp_path / "l.bin"), big, nrhs, stage1)
+    Y = product(H, h, storage, X)
+    for r, m in ((0, 64), (100, 20)):
+        assert np.abs(Y[r:r + m] - big - 4095).max() <= 64, np.unique(Y[r:r + m] - big)
