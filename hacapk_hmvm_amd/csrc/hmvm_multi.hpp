@@ -181,14 +181,18 @@ constexpr bool multi_tail() {
 // sides 93 / 540 -> 95 / 538, with 64 146 / 811 -> 163 / 854.  Without the
 // barriers between the tiles the compiler keeps several sums and spills (32:
 // 100 / 560, 64: 165 / 928).
-// BF16 stage 1 (kOrdered) folds a chunk at its end, into FP64 sums.
+// BF16 stage 1 (kOrdered) folds a chunk at its end; BF16 rows of y fold into
+// FP64 sums (64 right-hand sides as FP64 storage does): with one FP32 chain a
+// wave lost its 1,023 ones next to 2^30, and sums above FLT_MAX were infinite.
+// us without / with, 64 right-hand sides: N=12,007 52 / 57, 50,021 163 / 177,
+// 101,250 242 / 254; 32: 39 / 40, 119 / 127, 187 / 188 (the registers of FP64
+// sums).
 template <typename S, int NB, bool kOrdered>
 constexpr bool multi_fold() {
-  return kOrdered || sizeof(S) == 4 || (sizeof(S) == 8 && NB == 1);
+  return kOrdered || sizeof(S) == 4 || NB == 1 || (sizeof(S) == 2 && NB == 2);
 }
 template <typename S, int NB, bool kOrdered>
-using MultiSum =
-    typename std::conditional<kOrdered || (sizeof(S) == 4 && NB <= 2), mf_d4, typename Mfma<S>::Acc>::type;
+using MultiSum = typename std::conditional<sizeof(S) == 4 && NB == 4, typename Mfma<S>::Acc, mf_d4>::type;
 
 // out += the item's columns: D batches of loads in flight, and the slices of
 // the D after those.  kOrdered (BF16 stage 1): a batch is two steps of 16
@@ -234,14 +238,16 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
 #pragma unroll
       for (int cb = 0; cb < NB; ++cb) part[t][cb] = typename M::Acc{0, 0, 0, 0};
   };
+  auto add = [](MultiSum<S, NB, kOrdered> &o, const typename M::Acc &p) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] += p[v];
+  };
   auto fold = [&]() {
     if constexpr (multi_fold<S, NB, kOrdered>()) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) out[t][cb][v] += part[t][cb][v];
+        for (int cb = 0; cb < NB; ++cb) add(out[t][cb], part[t][cb]);
       clear();
     }
   };
@@ -267,7 +273,14 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
             }
         } else {
 #pragma unroll
-          for (int t = 0; t < NT; ++t) out[t][cb] = mfma_step(l.a[t][0], b.v, out[t][cb]);
+          for (int t = 0; t < NT; ++t) {
+            if constexpr (multi_fold<S, NB, kOrdered>()) {
+              part[t][cb] = mfma_step(l.a[t][0], b.v, part[t][cb]);
+            } else {
+              add(out[t][cb], mfma_step(l.a[t][0], b.v, typename M::Acc{0, 0, 0, 0}));
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
         }
       }
       if constexpr (kOrdered)
@@ -287,8 +300,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
           typename M::Acc sum{0, 0, 0, 0};
 #pragma unroll
           for (int q = 0; q < KS; ++q) sum = mfma_step(l.a[t][q / E][q % E], l.x[q].v[cb], sum);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) out[t][cb][v] += sum[v];
+          add(out[t][cb], sum);
           __builtin_amdgcn_sched_barrier(0);
         }
     }
