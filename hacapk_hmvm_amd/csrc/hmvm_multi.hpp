@@ -168,38 +168,33 @@ constexpr bool multi_tail() {
 }
 
 // An even share of a group's columns is a longer chain of roundings than a
-// tile of the one-vector launches, so the MFMA sums of a few batches are
-// folded into sums of their own (FP64; FP32 storage with 64 right-hand sides
-// FP32): for FP32 storage the error against 64 bits was 2.6e-7 without instead
-// of 1.1e-7 at N=4,096 and 5.1e-7 instead of 3.4e-7 at N=101,250; with, 1.1e-7
-// and 1.3e-7, at 3% of the time.
-// multi_fold: whether a second set of sums for all tiles does that, every
-// multi_depth batches; FP64 storage has the registers for it with 16 right-hand
-// sides only (with 32, 540 -> 650 us at N=101,250) and otherwise folds each
-// batch of each MFMA tile: error at N=12,007 / 101,250 6.9e-16 / 1.02e-15 ->
-// 2.4e-16 / 3.3e-16 (the tile launches 4.0e-16 / 7.1e-16), us with 32 right-hand
-// sides 93 / 540 -> 95 / 538, with 64 146 / 811 -> 163 / 854.  Without the
-// barriers between the tiles the compiler keeps several sums and spills (32:
-// 100 / 560, 64: 165 / 928).
-// BF16 stage 1 (kOrdered) folds a chunk at its end; BF16 rows of y fold into
-// FP64 sums (64 right-hand sides as FP64 storage does): with one FP32 chain a
-// wave lost its 1,023 ones next to 2^30, and sums above FLT_MAX were infinite.
-// us without / with, 64 right-hand sides: N=12,007 52 / 57, 50,021 163 / 177,
-// 101,250 242 / 254; 32: 39 / 40, 119 / 127, 187 / 188 (the registers of FP64
-// sums).
+// tile of the one-vector launches, so the MFMA sums of a few columns are folded
+// into FP64 sums.  Error against 80 bits, one chain / folded / the tile
+// launches: FP64 (32 right-hand sides) N=12,007 6.9e-16 / 2.4e-16 / 4.0e-16,
+// N=101,250 1.02e-15 / 3.3e-16 / 7.1e-16; FP32 N=101,250 5.1e-7 / 1.35e-7 / 3.6e-7,
+// 64 right-hand sides 1.0e-7 (1.8e-7 with FP32 sums).  BF16: the operands' 2.2e-3
+// in all three, but one chain lost 1,023 ones next to 2^30, and made shares above
+// FLT_MAX infinite.
+// multi_fold: whether a second set of sums for all MFMA tiles takes multi_depth
+// batches, where the registers hold it; else each batch of each tile is folded
+// (FP64, 32 right-hand sides: a second set 540 -> 650 us at N=101,250).  Without
+// the barriers between the tiles the compiler keeps several sums and spills
+// (N=101,250: FP64 32 538 -> 560, 64 830 -> 928; FP32 64 542 -> 593).
+// us, one chain / folded: FP64 32 right-hand sides N=12,007 93 / 94, N=101,250
+// 535 / 532, 64 145 / 162 and 804 / 831; FP32 64 118 / 109, 550 / 542 (FP32 sums
+// before); BF16 32 39 / 40, N=50,021 119 / 127, 64 52 / 57, 163 / 177.
+// BF16 stage 1 (kOrdered) folds a chunk at its end.
 template <typename S, int NB, bool kOrdered>
 constexpr bool multi_fold() {
-  return kOrdered || sizeof(S) == 4 || NB == 1 || (sizeof(S) == 2 && NB == 2);
+  return kOrdered || NB == 1 || (sizeof(S) < 8 && NB == 2);
 }
-template <typename S, int NB, bool kOrdered>
-using MultiSum = typename std::conditional<sizeof(S) == 4 && NB == 4, typename Mfma<S>::Acc, mf_d4>::type;
 
 // out += the item's columns: D batches of loads in flight, and the slices of
 // the D after those.  kOrdered (BF16 stage 1): a batch is two steps of 16
 // columns, one after the other (ordered_column).
 template <typename S, int NB, int NT, bool kOrdered>
 __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiItem &it, int lane,
-                                              MultiSum<S, NB, kOrdered> (&out)[NT][NB]) {
+                                              mf_d4 (&out)[NT][NB]) {
   using M = Mfma<S>;
   using V = typename VecOf<S>::T;
   constexpr int KS = M::KS, E = M::E, H = M::H, nrhs = 16 * NB;
@@ -238,7 +233,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
 #pragma unroll
       for (int cb = 0; cb < NB; ++cb) part[t][cb] = typename M::Acc{0, 0, 0, 0};
   };
-  auto add = [](MultiSum<S, NB, kOrdered> &o, const typename M::Acc &p) {
+  auto add = [](mf_d4 &o, const typename M::Acc &p) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) o[v] += p[v];
   };
@@ -385,12 +380,11 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
   constexpr int PT = multi_piece<NB>() < NT ? multi_piece<NB>() : NT;
   constexpr int W = 4;  // right-hand sides a thread adds: with two, twice the rounds of dependent slot loads (BF16,
                         // 64 right-hand sides, N=50,021: 174 -> 163 us a product)
-  using Sum = MultiSum<S, NB, kOrdered>;
-  Sum acc[NT][NB];
+  mf_d4 acc[NT][NB];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int cb = 0; cb < NB; ++cb) acc[t][cb] = Sum{0, 0, 0, 0};
+    for (int cb = 0; cb < NB; ++cb) acc[t][cb] = mf_d4{0, 0, 0, 0};
   multi_columns<S, NB, NT, kOrdered>(a, it, lane, acc);
   if (it.kind != kItemKept) {
 #pragma unroll
@@ -401,7 +395,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
         if (row >= it.nrows) continue;
         double r[NB];
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[t][cb][v];
+        for (int cb = 0; cb < NB; ++cb) r[cb] = acc[t][cb][v];
         if (it.kind == kItemSlot)
           store_n<NB>(a.slots + ((int64_t)it.out + row) * nrhs + NB * (lane & 15), r);
         else
@@ -420,7 +414,7 @@ __device__ __forceinline__ void multi_item(const MultiArgs &a, const MultiGroup 
       for (int v = 0; v < 4; ++v) {
         double r[NB];
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb) r[cb] = (double)acc[t][cb][v];
+        for (int cb = 0; cb < NB; ++cb) r[cb] = acc[t][cb][v];
         store_n<NB>(mine + ((t - t0) * 16 + M::row(lane, v)) * nrhs + NB * (lane & 15), r);
       }
     __syncthreads();

@@ -204,10 +204,9 @@ int hmvm_plan_reset_launch(hmvm_plan *plan);
 
 /* Several right-hand sides on the matrix cores: Y (+)= A X with X, Y of
  * nd x nrhs doubles, row-major (X[i*nrhs + c]); nrhs = 16, 32 or 64.  FP64
- * storage runs v_mfma_f64_16x16x4, FP32 v_mfma_f32_16x16x4 (FP32 sums of a
- * few columns, folded into FP64 sums, FP32 ones for 64 right-hand sides; FP64
- * across waves), BF16 v_mfma_f32_16x16x32_bf16 with the vector entries rounded
- * to BF16 (FP32 and BF16 storage read a copy of X in their own type that the
+ * storage runs v_mfma_f64_16x16x4, FP32 v_mfma_f32_16x16x4, BF16
+ * v_mfma_f32_16x16x32_bf16 with the vector entries rounded to BF16; the sums of
+ * a few columns are added in FP64 (FP32 and BF16 storage read a copy of X in their own type that the
  * apply makes on the device).  hmvm_plan_reserve_multi builds the multi-RHS
  * schedule, packs a copy of the plan's values in its order (about the size of
  * the plan's own; where the device lacks that memory, a smaller window that

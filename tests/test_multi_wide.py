@@ -69,7 +69,7 @@ def test_bf16_t_above_the_fp32_range_before_its_scales(gpu, H, O, tmp_path, nrhs
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("storage,nrhs", [("f32", 16), ("f32", 32), ("bf16", 16), ("bf16", 32), ("bf16", 64)])
+@pytest.mark.parametrize("storage,nrhs", [("f32", 16), ("f32", 32), ("f32", 64), ("bf16", 16), ("bf16", 32), ("bf16", 64)])
 def test_rows_of_y_above_the_fp32_range(gpu, H, O, tmp_path, storage, nrhs):
     """12 dense leaves of 400 columns side by side, X around 1e36: the sum of a
     leaf is below FLT_MAX, that of a wave's share of the columns (1,200) and y
@@ -108,7 +108,8 @@ def long_sums(H, path, big, nrhs, stage1):
 @pytest.mark.gpu
 @pytest.mark.parametrize("nrhs", [16, 32, 64])
 @pytest.mark.parametrize("storage,big,stage1", [("f64", 2.0**53, False), ("f64", 2.0**53, True),
-                                                ("bf16", 2.0**30, False)])
+                                                ("bf16", 2.0**30, False), ("f32", 2.0**28, False),
+                                                ("f32", 2.0**28, True)])
 def test_chains_of_roundings_stay_short(gpu, H, tmp_path, storage, big, stage1, nrhs):
     """Ones added to a number of which one is half the last bit or less are lost, and
     kept in sums of their own: of 4,096 columns no more than the 64 of a leaf
