@@ -839,7 +839,7 @@ __global__ __launch_bounds__(256) void probe_copy_kernel(const double4 *__restri
     dst[i] = src[i];
 }
 
-// dst[i] = src[i] in the multi-RHS operand type O (FP32, or the BF16 bits of
+// dst[i] = src[i] in the multi-RHS operand type O (FP64, FP32, or the BF16 bits of
 // the FP32-rounded value) for n elements, W at a time (W = 2: src 16-byte
 // aligned, n even), grid-stride: the operand copy of a multi-RHS X.
 template <int W, typename O>

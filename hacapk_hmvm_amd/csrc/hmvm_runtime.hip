@@ -1270,30 +1270,34 @@ void launch_tsum_multi(hmvm_plan *p, int nrhs, hipStream_t st) {
                        p->d_mtfac, p->d_scales, (uint16_t *)p->d_mt);
 }
 
-// Phase 0: the operand copy of X (FP32 and BF16 storage) and launch A, 1: the
-// t sum, 2: launch B.
+// Phase 0: the copy of X, if any, and launch A, 1: the t sum, 2: launch B.
 void launch_multi_phase(hmvm_plan *p, int phase, const double *X, double *Y, int nrhs, int accumulate,
                         hipStream_t st) {
   const Plan &P = p->plan;
   if (phase == 1) return launch_tsum_multi(p, nrhs, st);
   if (phase == 3) return;
-  if (phase == 0 && p->storage != kF64) {
-    // the groups read X and t in the operand type
-    const size_t n = (size_t)P.nd * nrhs;
-    const unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 8192);
+  const size_t n = (size_t)P.nd * nrhs;
+  // the groups read X and t in the operand type; launch B reads X while it
+  // writes Y, so an FP64 X that overlaps Y is copied too
+  const bool copy = p->storage != kF64 || ((uintptr_t)X < (uintptr_t)(Y + n) && (uintptr_t)Y < (uintptr_t)(X + n));
+  void *Xc = p->storage == kF64 ? (void *)p->d_mX : p->d_mXc;
+  if (phase == 0 && copy) {
     const bool a16 = ((uintptr_t)X & 15) == 0;
-    if (p->storage == kF32 && a16)
-      hipLaunchKernelGGL((to_vec_kernel<2, float>), dim3(blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
+    const dim3 grid((unsigned)std::min<size_t>((n / 2 + 255) / 256, 8192) * (a16 ? 1 : 2));
+    if (p->storage == kF64 && a16)
+      hipLaunchKernelGGL((to_vec_kernel<2, double>), grid, dim3(256), 0, st, X, (double *)Xc, n);
+    else if (p->storage == kF64)
+      hipLaunchKernelGGL((to_vec_kernel<1, double>), grid, dim3(256), 0, st, X, (double *)Xc, n);
+    else if (p->storage == kF32 && a16)
+      hipLaunchKernelGGL((to_vec_kernel<2, float>), grid, dim3(256), 0, st, X, (float *)Xc, n);
     else if (p->storage == kF32)
-      hipLaunchKernelGGL((to_vec_kernel<1, float>), dim3(2 * blocks), dim3(256), 0, st, X, (float *)p->d_mXc, n);
+      hipLaunchKernelGGL((to_vec_kernel<1, float>), grid, dim3(256), 0, st, X, (float *)Xc, n);
     else if (a16)
-      hipLaunchKernelGGL((to_vec_kernel<2, uint16_t>), dim3(blocks), dim3(256), 0, st, X, (uint16_t *)p->d_mXc, n);
+      hipLaunchKernelGGL((to_vec_kernel<2, uint16_t>), grid, dim3(256), 0, st, X, (uint16_t *)Xc, n);
     else
-      hipLaunchKernelGGL((to_vec_kernel<1, uint16_t>), dim3(2 * blocks), dim3(256), 0, st, X, (uint16_t *)p->d_mXc,
-                         n);
+      hipLaunchKernelGGL((to_vec_kernel<1, uint16_t>), grid, dim3(256), 0, st, X, (uint16_t *)Xc, n);
   }
-  launch_multi_part(p, phase == 2, p->storage == kF64 ? (const void *)X : (const void *)p->d_mXc, Y, nrhs, accumulate,
-                    st);
+  launch_multi_part(p, phase == 2, copy ? Xc : (const void *)X, Y, nrhs, accumulate, st);
 }
 
 int apply_multi(hmvm_plan *p, const double *X, double *Y, int nrhs, int accumulate, hipStream_t st) {

@@ -212,8 +212,8 @@ int hmvm_plan_reset_launch(hmvm_plan *plan);
  * the plan's own; where the device lacks that memory, a smaller window that
  * every apply fills part by part) and allocates the work buffers for up to
  * nrhs columns; the apply itself allocates nothing.  The host form reserves by
- * itself.  d_X and d_Y need 8-byte alignment; a 16-byte-aligned d_Y gets
- * 16-byte stores. */
+ * itself.  d_X and d_Y need 8-byte alignment (a 16-byte-aligned d_Y gets
+ * 16-byte stores) and may overlap: FP64 storage then copies d_X first. */
 int hmvm_plan_reserve_multi(hmvm_plan *plan, int nrhs);
 int hmvm_plan_apply_multi(hmvm_plan *plan, const double *d_X, double *d_Y, int nrhs, int accumulate, void *stream);
 int hmvm_plan_apply_multi_host(hmvm_plan *plan, const double *X, double *Y, int nrhs, int accumulate);
