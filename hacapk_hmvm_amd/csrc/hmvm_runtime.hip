@@ -181,7 +181,7 @@ struct hmvm_plan {
   MultiItem *d_mitems = nullptr;
   MultiSlice *d_mslices = nullptr;
   void *d_mvals = nullptr;      // values packed for the multi-RHS kernels, or one window of them
-  int64_t multi_elems = 0;      // packed values
+  size_t multi_bytes = 0, multi_work_bytes = 0;  // schedule and packed values; work buffers for multi_cap columns
   std::vector<MultiWindow> multi_windows;  // empty: all values are packed
   MultiPack *d_mpack = nullptr;
   int4 *d_mtsum = nullptr;      // {first, (nch << 16) | stride, entry, 0}
@@ -1112,6 +1112,12 @@ void multi_free(hmvm_plan *p) {
   p->d_mvals = nullptr;
   p->multi_ready = false;
   p->multi_windows.clear();
+  p->multi_bytes = 0;
+}
+
+template <typename... T>
+size_t vector_bytes(const std::vector<T> &...v) {
+  return ((sizeof(T) * v.size()) + ... + size_t(0));
 }
 
 // Builds, checks and uploads the multi-RHS schedule and packs its values.
@@ -1144,8 +1150,8 @@ int multi_schedule(hmvm_plan *p, int64_t window) {
       hipLaunchKernelGGL(map_scale_kernel, dim3((unsigned)((M.tmap.size() + 255) / 256)), dim3(256), 0, p->stream,
                          (int)M.tmap.size(), p->d_mtmap, p->d_mtfac, (const float *)p->d_scales, p->d_mscale_m);
   }
-  if ((rc = dalloc_bytes(&p->d_mvals, (size_t)elem_bytes(p->storage) * (size_t)(window > 0 ? window : M.nvals))))
-    return rc;
+  const size_t values = (size_t)elem_bytes(p->storage) * (size_t)(window > 0 ? window : M.nvals);
+  if ((rc = dalloc_bytes(&p->d_mvals, values))) return rc;
   if (window == 0) {
     launch_multi_pack(p->storage, (int)M.pack.size(), p->d_mpack, p->d_vals, p->d_scales, p->d_mvals, p->stream);
     HIP_TRY(hipStreamSynchronize(p->stream));
@@ -1160,7 +1166,10 @@ int multi_schedule(hmvm_plan *p, int64_t window) {
   p->n_mtsum = (int)ts.size();
   p->n_mt = M.n_t;
   p->n_mslots = M.n_slots;
-  p->multi_elems = M.nvals;
+  p->multi_bytes = vector_bytes(M.groups_a, M.groups_b, M.waves_a, M.waves_b, M.items, M.slices, M.tmap, ts, rng,
+                                M.ylist) +
+                   kMultiZeroBytes + (p->d_mpack ? vector_bytes(M.pack) : 0) +
+                   (p->storage == kBF16 ? vector_bytes(M.t_factor) + 8 * M.tmap.size() : 0) + values;
   p->multi_ready = true;
   return HMVM_OK;
 }
@@ -1189,6 +1198,7 @@ int multi_buffers(hmvm_plan *p, int nrhs) {
   p->d_mslots = p->d_mX = p->d_mY = nullptr;
   p->d_mt = p->d_mXc = nullptr;
   p->multi_cap = 0;
+  p->multi_work_bytes = 0;
   int rc;
   if ((rc = dalloc(&p->d_mslots, (size_t)p->n_mslots * nrhs)) ||
       (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)p->n_mt * nrhs)) ||
@@ -1196,6 +1206,8 @@ int multi_buffers(hmvm_plan *p, int nrhs) {
     return rc;
   if (p->storage != kF64 && (rc = dalloc_bytes(&p->d_mXc, vec_bytes(p->storage) * (size_t)P.nd * nrhs))) return rc;
   p->multi_cap = nrhs;
+  p->multi_work_bytes = (8 * (size_t)(p->n_mslots + 2 * P.nd) + vec_bytes(p->storage) * (size_t)p->n_mt +
+                         (p->storage != kF64 ? vec_bytes(p->storage) * (size_t)P.nd : 0)) * nrhs;
   return HMVM_OK;
 }
 
@@ -1525,7 +1537,7 @@ void fill_info(const hmvm_plan *p, const Plan &P, int storage, hmvm_plan_info *i
   info->vec_reads_a = P.vec_a;
   info->vec_reads_b = P.vec_b;
   info->algorithmic_bytes = (long long)info->elem_bytes * P.len + 16LL * P.nd;
-  info->device_bytes = p ? (long long)p->device_bytes : 0;
+  info->device_bytes = p ? (long long)(p->device_bytes + p->multi_bytes + p->multi_work_bytes) : 0;
   info->mode = !p ? 0 : persistent_ok(p) ? 1 : overlap_ok(p) ? 2 : 0;
   info->t_direct = P.t_direct ? 1 : 0;
 }
