@@ -1087,10 +1087,12 @@ void launch_phase(hmvm_plan *p, int phase, const double *x, double *y, int accum
 }
 
 // ---- several right-hand sides -------------------------------------------------
-// Elements of the multi-RHS value window: the value of HMVM_MULTI_WINDOW when
-// set (>= 1), else 0 (all values packed once, in windows only if memory lacks).
-int64_t multi_window_elems() {
-  const char *e = std::getenv("HMVM_MULTI_WINDOW");
+// HMVM_MULTI_WINDOW: elements of the multi-RHS value window (else 0: all values
+// packed once, in windows only if memory lacks).  HMVM_MULTI_LIMIT: bytes that
+// the multi-RHS schedule, packed values and work buffers of a plan may take
+// (else 0: what the device has).
+int64_t env_number(const char *name) {
+  const char *e = std::getenv(name);
   return e && *e ? std::max(0LL, std::atoll(e)) : 0;
 }
 
@@ -1120,10 +1122,41 @@ size_t vector_bytes(const std::vector<T> &...v) {
   return ((sizeof(T) * v.size()) + ... + size_t(0));
 }
 
-// Builds, checks and uploads the multi-RHS schedule and packs its values.
-// window: 0 packs all values into a copy of their own; else a buffer of so
-// many elements, which every apply fills and uses window by window.
-int multi_schedule(hmvm_plan *p, int64_t window) {
+void multi_free_buffers(hmvm_plan *p) {
+  void *bufs[5] = {p->d_mslots, p->d_mt, p->d_mX, p->d_mY, p->d_mXc};
+  for (void *b : bufs)
+    if (b) (void)hipFree(b);
+  p->d_mslots = p->d_mX = p->d_mY = nullptr;
+  p->d_mt = p->d_mXc = nullptr;
+  p->multi_cap = 0;
+  p->multi_work_bytes = 0;
+}
+
+// Work buffers for nrhs columns beside `held` bytes of schedule and values.
+int multi_buffers(hmvm_plan *p, int nrhs, size_t held) {
+  const Plan &P = p->plan;
+  multi_free_buffers(p);
+  const size_t work = (8 * (size_t)(p->n_mslots + 2 * P.nd) + vec_bytes(p->storage) * (size_t)p->n_mt +
+                       (p->storage != kF64 ? vec_bytes(p->storage) * (size_t)P.nd : 0)) * nrhs;
+  const size_t limit = (size_t)env_number("HMVM_MULTI_LIMIT");
+  if (limit > 0 && held + work > limit)
+    return set_error(HMVM_ERR_HIP, "multi-RHS schedule: %zu bytes exceed HMVM_MULTI_LIMIT", held + work);
+  int rc;
+  if ((rc = dalloc(&p->d_mslots, (size_t)p->n_mslots * nrhs)) ||
+      (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)p->n_mt * nrhs)) ||
+      (rc = dalloc(&p->d_mX, (size_t)P.nd * nrhs)) || (rc = dalloc(&p->d_mY, (size_t)P.nd * nrhs)))
+    return rc;
+  if (p->storage != kF64 && (rc = dalloc_bytes(&p->d_mXc, vec_bytes(p->storage) * (size_t)P.nd * nrhs))) return rc;
+  p->multi_cap = nrhs;
+  p->multi_work_bytes = work;
+  return HMVM_OK;
+}
+
+// Builds, checks and uploads the multi-RHS schedule, with work buffers for nrhs
+// columns, and packs its values.  window: 0 packs all values into a copy of
+// their own; else a buffer of so many elements, which every apply fills and
+// uses window by window.
+int multi_schedule(hmvm_plan *p, int64_t window, int nrhs) {
   MultiPlan M;
   MultiOptions opt = multi_options(p->plan);
   if (window > 0) opt.wave_cols = 0;
@@ -1150,13 +1183,19 @@ int multi_schedule(hmvm_plan *p, int64_t window) {
       hipLaunchKernelGGL(map_scale_kernel, dim3((unsigned)((M.tmap.size() + 255) / 256)), dim3(256), 0, p->stream,
                          (int)M.tmap.size(), p->d_mtmap, p->d_mtfac, (const float *)p->d_scales, p->d_mscale_m);
   }
+  p->n_mt = M.n_t;
+  p->n_mslots = M.n_slots;
   const size_t values = (size_t)elem_bytes(p->storage) * (size_t)(window > 0 ? window : M.nvals);
-  if ((rc = dalloc_bytes(&p->d_mvals, values))) return rc;
+  p->multi_bytes = vector_bytes(M.groups_a, M.groups_b, M.waves_a, M.waves_b, M.items, M.slices, M.tmap, ts, rng,
+                                M.ylist, M.pack) +
+                   kMultiZeroBytes + (p->storage == kBF16 ? vector_bytes(M.t_factor) + 8 * M.tmap.size() : 0) + values;
+  if ((rc = multi_buffers(p, nrhs, p->multi_bytes)) || (rc = dalloc_bytes(&p->d_mvals, values))) return rc;
   if (window == 0) {
     launch_multi_pack(p->storage, (int)M.pack.size(), p->d_mpack, p->d_vals, p->d_scales, p->d_mvals, p->stream);
     HIP_TRY(hipStreamSynchronize(p->stream));
     (void)hipFree(p->d_mpack);
     p->d_mpack = nullptr;
+    p->multi_bytes -= vector_bytes(M.pack);
   }
   HIP_TRY(hipStreamSynchronize(p->stream));
   HIP_TRY(hipGetLastError());
@@ -1164,66 +1203,36 @@ int multi_schedule(hmvm_plan *p, int64_t window) {
   p->n_mgroups_a = (int)M.groups_a.size();
   p->n_mgroups_b = (int)M.groups_b.size();
   p->n_mtsum = (int)ts.size();
-  p->n_mt = M.n_t;
-  p->n_mslots = M.n_slots;
-  p->multi_bytes = vector_bytes(M.groups_a, M.groups_b, M.waves_a, M.waves_b, M.items, M.slices, M.tmap, ts, rng,
-                                M.ylist) +
-                   kMultiZeroBytes + (p->d_mpack ? vector_bytes(M.pack) : 0) +
-                   (p->storage == kBF16 ? vector_bytes(M.t_factor) + 8 * M.tmap.size() : 0) + values;
   p->multi_ready = true;
   return HMVM_OK;
 }
 
-// The schedule with all values packed, or, where the device has no memory for
-// that, with a window of half, a quarter, ... of them.
-int multi_schedule_fit(hmvm_plan *p, bool whole) {
-  int64_t window = multi_window_elems();
-  if (window == 0 && !whole) window = std::max<int64_t>(1, p->plan.nvals / 2);
-  for (;;) {
-    multi_free(p);
-    const int rc = multi_schedule(p, window);
-    if (rc == HMVM_OK) return rc;
-    (void)hipGetLastError();
-    multi_free(p);
-    if (rc != HMVM_ERR_HIP || window == 1) return rc;
-    window = window > 0 ? (window + 1) / 2 : std::max<int64_t>(1, p->plan.nvals / 2);
-  }
-}
-
-int multi_buffers(hmvm_plan *p, int nrhs) {
-  const Plan &P = p->plan;
-  void *bufs[5] = {p->d_mslots, p->d_mt, p->d_mX, p->d_mY, p->d_mXc};
-  for (void *b : bufs)
-    if (b) (void)hipFree(b);
-  p->d_mslots = p->d_mX = p->d_mY = nullptr;
-  p->d_mt = p->d_mXc = nullptr;
-  p->multi_cap = 0;
-  p->multi_work_bytes = 0;
-  int rc;
-  if ((rc = dalloc(&p->d_mslots, (size_t)p->n_mslots * nrhs)) ||
-      (rc = dalloc_bytes(&p->d_mt, vec_bytes(p->storage) * (size_t)p->n_mt * nrhs)) ||
-      (rc = dalloc(&p->d_mX, (size_t)P.nd * nrhs)) || (rc = dalloc(&p->d_mY, (size_t)P.nd * nrhs)))
-    return rc;
-  if (p->storage != kF64 && (rc = dalloc_bytes(&p->d_mXc, vec_bytes(p->storage) * (size_t)P.nd * nrhs))) return rc;
-  p->multi_cap = nrhs;
-  p->multi_work_bytes = (8 * (size_t)(p->n_mslots + 2 * P.nd) + vec_bytes(p->storage) * (size_t)p->n_mt +
-                         (p->storage != kF64 ? vec_bytes(p->storage) * (size_t)P.nd : 0)) * nrhs;
-  return HMVM_OK;
-}
-
+// Schedule and work buffers for nrhs columns; where the device has no memory
+// for them beside all packed values, with a window of half, a quarter, ... of
+// these, down to the values of one group.
 int reserve_multi(hmvm_plan *p, int nrhs) {
   if (nrhs != 16 && nrhs != 32 && nrhs != 64) return set_error(HMVM_ERR_ARG, "nrhs must be 16, 32 or 64");
-  int rc;
-  if (!p->multi_ready && (rc = multi_schedule_fit(p, true))) return rc;
   if (p->multi_cap >= nrhs) return HMVM_OK;
-  rc = multi_buffers(p, nrhs);
-  if (rc == HMVM_ERR_HIP && p->multi_windows.empty()) {
-    // the packed values took the memory of the work buffers: pack them in windows
-    (void)hipGetLastError();
-    if ((rc = multi_schedule_fit(p, false))) return rc;
-    rc = multi_buffers(p, nrhs);
+  if (p->multi_ready) {
+    const int rc = multi_buffers(p, nrhs, p->multi_bytes);
+    if (rc != HMVM_ERR_HIP) return rc;
   }
-  return rc;
+  int64_t window = env_number("HMVM_MULTI_WINDOW");
+  std::string no_memory;
+  for (;;) {
+    (void)hipGetLastError();
+    multi_free(p);
+    const int rc = multi_schedule(p, window, nrhs);
+    if (rc == HMVM_OK) return rc;
+    multi_free(p);
+    multi_free_buffers(p);
+    // a window below one group's values ends the search: the memory was short
+    if (rc == HMVM_ERR_UNSUPPORTED && !no_memory.empty()) return set_error(HMVM_ERR_HIP, "%s", no_memory.c_str());
+    if (rc != HMVM_ERR_HIP) return rc;
+    no_memory = hmvm_hip_last_error_message();
+    window = window > 0 ? (window + 1) / 2 : std::max<int64_t>(1, p->plan.nvals / 2);
+    if (window <= 1) return rc;
+  }
 }
 
 // which: 0 launch A (stage 1 to t and t slots), 1 launch B (rows of y); X in
