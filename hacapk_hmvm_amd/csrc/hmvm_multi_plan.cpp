@@ -221,7 +221,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
       if (f.t) {
         t_idx[leaf] = (int)M.n_t;
         M.n_t += r.cols;
-        if (M.n_t > INT32_MAX) return "t exceeds int32";
+        if (M.n_t > INT32_MAX) return kMultiTooLarge;
       }
       f.v = f.t ? t_idx[leaf] : nstrtt[leaf] - 1;
       clusters.back().factors.push_back(f);
@@ -344,7 +344,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
               add_group(A, direct ? kMultiT : kMultiTSlot, direct ? map : M.n_slots, s.col0 + c0, b, nr, none, idle,
                         unit);
             if (!direct) M.n_slots += nr;
-            if (M.n_slots > INT32_MAX) return "slots exceed int32";
+            if (M.n_slots > INT32_MAX) return kMultiTooLarge;
           }
           if (direct)
             M.tmap.insert(M.tmap.end(), trow.begin() + r0, trow.begin() + r0 + nr);
@@ -379,14 +379,14 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
           M.tmap.insert(M.tmap.end(), trow.begin() + r0, trow.begin() + r0 + nr);
         else
           M.n_slots += nr;
-        if (M.n_slots > INT32_MAX) return "slots exceed int32";
+        if (M.n_slots > INT32_MAX) return kMultiTooLarge;
       }
       if (!direct)
         for (int r = 0; r < nr; r++)
           M.tsum.push_back({(int32_t)(slot0 + r), chunks, nr, trow[(size_t)r0 + r]});
     }
   }
-  if (M.tmap.size() > (size_t)INT32_MAX) return "t map exceeds int32";
+  if (M.tmap.size() > (size_t)INT32_MAX) return kMultiTooLarge;
   // one-wave stacks of like cost share a workgroup
   std::stable_sort(single.begin(), single.end(), [](const Single &x, const Single &y) {
     return x.it.nbatch * batch_cost(x.it.nrows) > y.it.nbatch * batch_cost(y.it.nrows);
@@ -509,7 +509,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
                          (int32_t)M.n_slots, kItemSlot, 0});
         lo_of.push_back(lo);
         M.n_slots += n;
-        if (M.n_slots > INT32_MAX) return "slots exceed int32";
+        if (M.n_slots > INT32_MAX) return kMultiTooLarge;
       }
     }
     // y lists: rows between two ends of partial items add the same slots
@@ -531,7 +531,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
           M.yptr[2 * ((size_t)r0 + r) + 1] = (int32_t)M.ylist.size();
         }
       }
-      if (M.ylist.size() > (size_t)INT32_MAX) return "y lists exceed int32";
+      if (M.ylist.size() > (size_t)INT32_MAX) return kMultiTooLarge;
     }
     // partial items to the waves, largest first to the least loaded
     std::vector<int> ord(small.size());
@@ -549,7 +549,7 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
     }
     add_group(Bl, kMultiY, r0, r0, B.place(col, nr), nr, own, load);
   }
-  if (M.slices.size() > (size_t)INT32_MAX || M.items.size() > (size_t)INT32_MAX) return "multi-RHS schedule too large";
+  if (M.slices.size() > (size_t)INT32_MAX || M.items.size() > (size_t)INT32_MAX) return kMultiTooLarge;
   A.finish(nw, &M.groups_a, &M.waves_a);
   Bl.finish(nw, &M.groups_b, &M.waves_b);
   return "";
@@ -608,6 +608,20 @@ std::string window_multi_plan(int storage, int64_t cap, MultiPlan *Mp, std::vect
     wl.swap(nwv);
   }
   if (rec != M.pack.size()) return "pack records outside the windows";
+  // what the kernels of a window address lies inside its buffer
+  for (const MultiWindow &w : *out) {
+    auto outside = [&](int64_t a, int64_t n) { return a < w.a0 || a + n > w.a0 + cap; };
+    for (int32_t i = w.pack0; i < w.pack0 + w.npack; i++) {
+      const MultiPack &r = M.pack[(size_t)i];
+      if (outside(r.dst, ((r.cols + KS - 1) / KS + r.pad) * (int64_t)r.nrows * KS)) return "pack record outside its window";
+    }
+    const std::vector<MultiWave> &wl = w.launch == 0 ? M.waves_a : M.waves_b;
+    for (size_t k = (size_t)w.group0 * nw; k < (size_t)(w.group0 + w.ngroups) * nw; k++)
+      for (int i = wl[k].item0; i < wl[k].item0 + wl[k].nitems; i++) {
+        const MultiItem &it = M.items[(size_t)i];
+        if (it.nbatch > 0 && outside(it.a0, (int64_t)it.nbatch * kMultiBatch * it.nrows * KS)) return "item outside its window";
+      }
+  }
   return "";
 }
 
@@ -615,18 +629,51 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
   const int KS = multi_slice_cols(storage);
   const int64_t nslice = (int64_t)M.slices.size();
   // packing: sources inside the values, each element once
-  int64_t packed = 0, written = 0;
+  int64_t packed = 0;
   for (const MultiPack &r : M.pack) {
     if (r.rows < 1 || r.cols < 1 || r.row0 < 0 || r.row0 + r.rows > r.nrows || r.pad < 0) return "pack record shape";
     if (r.src < 0 || r.ld < 1 || r.src + r.rows - 1 + (int64_t)(r.cols - 1) * r.ld >= P.nvals)
       return "pack source outside the values";
-    const int64_t ns = (r.cols + KS - 1) / KS + r.pad;
-    if (r.dst < 0 || r.dst + ns * r.nrows * KS > M.nvals) return "pack destination outside the packed values";
     if (r.factor >= P.nfactors) return "pack factor";
     packed += (int64_t)r.rows * r.cols;
-    written += ns * r.rows * KS;
   }
-  if (packed != P.len || written != M.nvals) return "packing does not cover the leaves";
+  if (packed != P.len) return "packing does not cover the leaves";
+  // the records of the same slices cover the item's rows, one after the
+  // other, and the slices follow each other up to the last value
+  std::vector<int32_t> order(M.pack.size());
+  for (size_t i = 0; i < order.size(); i++) order[i] = (int32_t)i;
+  auto before = [&](int32_t x, int32_t y) {
+    const MultiPack &p = M.pack[(size_t)x], &q = M.pack[(size_t)y];
+    return p.dst != q.dst ? p.dst < q.dst : p.row0 < q.row0;
+  };
+  if (!std::is_sorted(order.begin(), order.end(), before)) std::sort(order.begin(), order.end(), before);
+  int64_t end = 0;
+  for (size_t i = 0; i < order.size();) {
+    const MultiPack &f = M.pack[(size_t)order[i]];
+    const int64_t ns = (f.cols + KS - 1) / KS + f.pad;
+    int row = 0;
+    if (f.dst != end) return "packed values overlap or have gaps";
+    for (; i < order.size() && M.pack[(size_t)order[i]].dst == f.dst; i++) {
+      const MultiPack &r = M.pack[(size_t)order[i]];
+      if (r.row0 != row || r.nrows != f.nrows || (r.cols + KS - 1) / KS + r.pad != ns)
+        return "pack records of the same slices disagree";
+      row += r.rows;
+    }
+    if (row != f.nrows) return "packed rows missing";
+    end += ns * f.nrows * KS;
+  }
+  if (end != M.nvals) return "packing does not cover the packed values";
+  // every packed element is read by one item: the items' values follow each other
+  std::vector<std::pair<int64_t, int64_t>> read;
+  for (const MultiItem &it : M.items)
+    if (it.nbatch > 0) read.push_back({it.a0, it.a0 + (int64_t)it.nbatch * kMultiBatch * it.nrows * KS});
+  std::sort(read.begin(), read.end());
+  end = 0;
+  for (const auto &r : read) {
+    if (r.first != end) return "items overlap or leave packed values out";
+    end = r.second;
+  }
+  if (end != M.nvals) return "items leave packed values out";
   int64_t covered = 0;
   std::vector<char> t_seen((size_t)M.n_t, 0), y_seen((size_t)P.nd, 0), slot_seen((size_t)M.n_slots, 0);
   for (int list = 0; list < 2; list++) {
@@ -715,6 +762,111 @@ std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M) {
       if (s < 0 || s >= M.n_slots || !slot_seen[(size_t)s]) return "y list slot";
     }
   }
+  return "";
+}
+
+std::string verify_multi_values(const Plan &P, int storage, const int *nstrtl, const int *nstrtt, const MultiPlan &M) {
+  const int KS = multi_slice_cols(storage);
+  // the repack record of every element of the value layout, and its first
+  // rank row or column in the factor
+  std::vector<int32_t> owner((size_t)P.nvals, -1);
+  std::vector<int> first(P.repack.size(), 0), kdone(P.nlf, 0);
+  for (size_t i = 0; i < P.repack.size(); i++) {
+    const RepackDesc &r = P.repack[i];
+    if (r.rows == 0 || r.cols == 0) continue;
+    if (r.factor % 2 == 0) {
+      first[i] = kdone[r.factor / 2];
+      kdone[r.factor / 2] += r.rows;
+    }
+    for (int c = 0; c < r.cols; c++)
+      for (int k = 0; k < r.rows; k++) owner[(size_t)(r.dst_off + k + (int64_t)c * r.dst_cs)] = (int32_t)i;
+  }
+  std::vector<int> t_idx(P.nlf, -1);
+  for (int64_t e = M.n_t; e-- > 0;) t_idx[(size_t)M.t_factor[(size_t)e] / 2] = (int)e;
+  // where the rows of every item go: a row of t (launch A) or of y
+  struct Read {
+    int64_t a0, end;
+    int32_t item, row0;  // row0: first row of y or index in t_of
+    int list;
+  };
+  std::vector<int32_t> t_of(M.tmap), slot_t((size_t)M.n_slots, -1);
+  for (const MultiPlan::TSum &t : M.tsum)
+    for (int c = 0; c < t.nch; c++) slot_t[(size_t)t.first + (size_t)c * t.stride] = t.entry;
+  std::vector<int32_t> slot_y((size_t)M.n_slots, -1);
+  std::vector<char> added((size_t)M.n_slots, 0);
+  for (int r = 0; r < P.nd; r++)
+    for (int i = M.yptr[2 * (size_t)r]; i < M.yptr[2 * (size_t)r + 1]; i++) {
+      const size_t q = (size_t)M.ylist[(size_t)i] + r;
+      if (added[q]++) return "slot added to y twice";
+      slot_y[q] = r;
+    }
+  std::vector<Read> read;
+  for (int list = 0; list < 2; list++) {
+    const std::vector<MultiGroup> &gl = list == 0 ? M.groups_a : M.groups_b;
+    const std::vector<MultiWave> &wl = list == 0 ? M.waves_a : M.waves_b;
+    for (size_t k = 0; k < wl.size(); k++)
+      for (int i = wl[k].item0; i < wl[k].item0 + wl[k].nitems; i++) {
+        const MultiItem &it = M.items[(size_t)i];
+        const MultiGroup &g = gl[k / (size_t)M.waves];
+        if (it.nbatch == 0) continue;
+        Read r{it.a0, it.a0 + (int64_t)it.nbatch * kMultiBatch * it.nrows * KS, i, 0, list};
+        const bool slots = it.kind == kItemSlot || (it.kind == kItemKept && g.kind == kMultiTSlot);
+        const int out = it.kind == kItemKept ? g.out : it.out;
+        if (list == 0 && !slots) {
+          r.row0 = out;
+        } else if (list == 0) {
+          r.row0 = (int32_t)t_of.size();
+          for (int q = 0; q < it.nrows; q++) t_of.push_back(slot_t[(size_t)out + q]);
+        } else if (slots) {
+          r.row0 = slot_y[(size_t)out];
+          for (int q = 0; q < it.nrows; q++)
+            if (slot_y[(size_t)out + q] != r.row0 + q || r.row0 < 0) return "slot added to another row of y";
+        } else {
+          r.row0 = out;
+        }
+        read.push_back(r);
+      }
+  }
+  std::sort(read.begin(), read.end(), [](const Read &x, const Read &y) { return x.a0 < y.a0; });
+  for (const MultiPack &r : M.pack) {
+    const int64_t step = (int64_t)r.nrows * KS;  // of a slice
+    for (int s = 0; s < (r.cols + KS - 1) / KS + r.pad; s++) {
+      const int64_t at = r.dst + s * step;
+      auto rd = std::upper_bound(read.begin(), read.end(), at, [](int64_t a, const Read &x) { return a < x.a0; });
+      if (rd == read.begin()) return "packed slice without an item";
+      --rd;
+      const MultiItem &it = M.items[(size_t)rd->item];
+      if (at >= rd->end || it.nrows != r.nrows || (at - rd->a0) % step) return "packed slice beside its item";
+      const MultiSlice &q = M.slices[(size_t)it.slice0 + (size_t)((at - rd->a0) / step)];
+      const bool ordered = storage == kBF16 && rd->list == 0;
+      if (ordered != (r.ordered != 0)) return "order of a pack record";
+      const int n1 = q.info & 15, n2 = ordered ? (q.info >> 4) & 15 : 0;
+      for (int j = 0; j < KS; j++) {
+        const int c = ordered ? ordered_column(s, j) : s * KS + j;
+        const bool in_use = ordered && j >= kHalf ? j - kHalf < n2 : j < n1;
+        if (in_use != (c < r.cols)) return "columns of a slice in use";
+        if (!in_use) continue;
+        const int v = q.v + (ordered && j >= kHalf ? kStep + j - kHalf : j);
+        for (int k = 0; k < r.rows; k++) {
+          const int64_t p = r.src + k + (int64_t)c * r.ld;
+          const int32_t o = owner[(size_t)p];
+          if (o < 0) return "element packed twice, or none";
+          owner[(size_t)p] = -1;
+          const RepackDesc &d = P.repack[(size_t)o];
+          const int leaf = d.factor / 2, row = (int)((p - d.dst_off) % d.dst_cs), col = (int)((p - d.dst_off) / d.dst_cs);
+          const bool a1 = d.factor % 2 == 0, a2 = !a1 && kdone[(size_t)leaf] > 0;
+          if (a1 != (rd->list == 0) || a2 != ((q.info & kSliceT) != 0)) return "factor in the wrong launch";
+          if (v != (a2 ? t_idx[(size_t)leaf] : nstrtt[leaf] - 1) + col) return "element meets another vector entry";
+          const int out = a1 ? t_of[(size_t)rd->row0 + r.row0 + k] : rd->row0 + r.row0 + k;
+          if (out != (a1 ? t_idx[(size_t)leaf] + first[(size_t)o] : nstrtl[leaf] - 1) + row) return "element goes to another row";
+          if (r.factor >= 0 && r.factor != d.factor) return "scale of another factor";
+          if (storage == kBF16 && !a1 && !a2 && r.factor < 0) return "dense leaf without its scale";
+        }
+      }
+    }
+  }
+  for (int32_t o : owner)
+    if (o >= 0) return "element never packed";
   return "";
 }
 

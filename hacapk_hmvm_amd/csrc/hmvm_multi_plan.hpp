@@ -142,15 +142,22 @@ struct MultiPlan {
   std::vector<int32_t> ylist;
 };
 
+constexpr const char *kMultiTooLarge = "the matrix is too large for the multi-RHS schedule";
+
 // P: the plan whose value layout (repack records) is read; nstrtl, nstrtt:
-// first row and column of every leaf (1-based).  "" or an error message.
+// first row and column of every leaf (1-based).  "" or an error message
+// (kMultiTooLarge: offsets exceed int32).
 std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, const int *nstrtt,
                              const MultiOptions &opt, MultiPlan *out);
 
-// Every element of every leaf packed once, every packed element written once
-// and read by one item, every t row and y row written once, every address a
-// kernel forms inside its buffer.
+// Every packed element written once and read by one item, every t row and y row
+// written once, every address a kernel forms inside its buffer.
 std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M);
+
+// For a plan that passed verify_multi_plan, element by element (4 bytes of host
+// memory each): every element of every leaf packed once, against its vector
+// entry, into its row.
+std::string verify_multi_values(const Plan &P, int storage, const int *nstrtl, const int *nstrtt, const MultiPlan &M);
 
 // Sizes by matrix order, see the definition.
 MultiOptions multi_options(const Plan &P);

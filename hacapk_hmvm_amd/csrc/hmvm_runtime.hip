@@ -1161,8 +1161,8 @@ int multi_schedule(hmvm_plan *p, int64_t window, int nrhs) {
   MultiOptions opt = multi_options(p->plan);
   if (window > 0) opt.wave_cols = 0;
   std::string err = build_multi_plan(p->plan, p->storage, p->nstrtl.data(), p->nstrtt.data(), opt, &M);
-  if (err.empty()) err = verify_multi_plan(p->plan, p->storage, M);
   if (err.empty() && window > 0) err = window_multi_plan(p->storage, window, &M, &p->multi_windows);
+  if (err.empty()) err = verify_multi_plan(p->plan, p->storage, M);
   if (!err.empty()) return set_error(HMVM_ERR_UNSUPPORTED, "multi-RHS schedule: %s", err.c_str());
   std::vector<int4> ts;
   for (const MultiPlan::TSum &t : M.tsum)
@@ -2012,10 +2012,13 @@ int hmvm_plan_check(const matrix2 *mat2, const hmvm_options *opt, hmvm_plan_info
   if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "%s", err.c_str());
   err = verify_plan(P, s.la);
   if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "schedule check failed: %s", err.c_str());
-  MultiPlan M;  // the schedule of several right-hand sides (a matrix too large for it keeps the other)
-  if (build_multi_plan(P, po.storage, s.la.nstrtl, s.la.nstrtt, multi_options(P), &M).empty())
-    err = verify_multi_plan(P, po.storage, M);
-  if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "multi-RHS schedule check failed: %s", err.c_str());
+  MultiPlan M;  // the schedule of several right-hand sides, where the matrix is not too large for it
+  err = build_multi_plan(P, po.storage, s.la.nstrtl, s.la.nstrtt, multi_options(P), &M);
+  if (err != kMultiTooLarge) {
+    if (err.empty()) err = verify_multi_plan(P, po.storage, M);
+    if (err.empty()) err = verify_multi_values(P, po.storage, s.la.nstrtl, s.la.nstrtt, M);
+    if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "multi-RHS schedule check failed: %s", err.c_str());
+  }
   if (info) fill_info(nullptr, P, po.storage, info);
   return HMVM_OK;
 }
