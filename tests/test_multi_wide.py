@@ -118,3 +118,37 @@ def test_chains_of_roundings_stay_short(gpu, H, tmp_path, storage, big, stage1, 
     Y = product(H, h, storage, X)
     for r, m in ((0, 64), (100, 20)):
         assert np.abs(Y[r:r + m] - big - 4095).max() <= 64, np.unique(Y[r:r + m] - big)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nrhs", [16, 32, 64])
+@pytest.mark.parametrize("storage", ["f64", "f32", "bf16"])
+def test_wide_stacks_match_oracle(gpu, H, O, tmp_path, storage, nrhs, monkeypatch):
+    """Random factors, at once and in windows; BF16 (whose t is rounded to BF16)
+    keeps its bits under other layouts of the one-vector launches."""
+    write_format1(str(tmp_path / "r.bin"), ND, WIDE + [(2, 33, 65, 900, 1, 0), (2, 17, 9, 950, 20, 0)],
+                  np.random.default_rng(5))
+    h = H.loadHmatrix(str(tmp_path / "r.bin"))
+    X = np.random.default_rng(nrhs).uniform(-1, 1, (ND, nrhs))
+    ref = {c: O.seq_2(h, np.ascontiguousarray(X[:, c])) for c in (0, 5, nrhs - 1)}
+
+    def check(**kw):
+        p = H.Plan(h, storage=storage, **kw)
+        one = p.info()["device_bytes"]
+        Y = p.apply_multi_host(X)
+        held.append(p.info()["device_bytes"] - one)
+        p.close()
+        for c, r in ref.items():
+            assert np.linalg.norm(Y[:, c] - r) <= TOL[storage] * np.linalg.norm(r), c
+        return Y
+
+    held = []
+    Y = check()
+    for kw in ({"t_mode": 1}, {"t_mode": 0}, {"t_mode": 2}, {"w2": 500, "w3": 700, "max_rows_b": 40}):
+        Z = check(**kw)
+        assert storage != "bf16" or np.array_equal(Z, Y), kw
+    # in windows: a quarter of the values' bytes less than all takes
+    monkeypatch.setenv("HMVM_MULTI_LIMIT", str(held[0] - h.mat2.len * {"f64": 8, "f32": 4, "bf16": 2}[storage] // 4))
+    Z = check()
+    assert held[-1] < held[0]
+    assert storage != "bf16" or np.array_equal(Z, Y)
