@@ -123,19 +123,17 @@ struct TileOut {
   const int32_t *tmap;
   void *tout;  // t: double
   const double *mscale;
-  int via_slot;  // t gets what the t sum would read from the slot: the row in the slots' type
 };
 
 template <typename S, bool kScaled>
 __device__ __forceinline__ void store_row(const TileDesc &td, int row, double v, const TileOut &o,
                                           const float *__restrict__ scales) {
-  using Slot = typename SlotOf<S>::T;
   if (td.map_off < 0) {
+    using Slot = typename SlotOf<S>::T;
     static_cast<Slot *>(o.out)[td.out_off + row] = (Slot)v;
     return;
   }
   const int e = o.tmap[td.map_off + row];
-  if (o.via_slot) v = (double)(Slot)v;
   if constexpr (kScaled) v *= o.mscale[td.map_off + row];
   static_cast<double *>(o.tout)[e] = v;
 }
@@ -755,7 +753,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(S) =
   const int nwg = (int)gridDim.x;
   extern __shared__ double tile_lds[];
   double *lds = tile_lds + (threadIdx.x >> 6) * lds_wave_doubles<S>();
-  const TileOut o{slots, tmap, t, mscale, 0};  // stage-1 rows with a map go to t
+  const TileOut o{slots, tmap, t, mscale};  // stage-1 rows with a map go to t
   // join: count this workgroup on its XCD (XCC_ID register), then learn how
   // many workgroups each XCD holds once all have joined
   __shared__ int xcd_info[3];  // XCD, its workgroups, XCDs in use

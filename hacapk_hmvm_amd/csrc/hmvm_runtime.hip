@@ -769,9 +769,9 @@ int upload_values(hmvm_plan *p, const Source &src) {
   return rc;
 }
 
-// The tiles of launch `which` as its launches take them: in a plan with bands
-// the stage-1 tiles write t through their maps (the persistent launch takes
-// the plan's own, which write the slots that its t sum stage reads).
+// A launch's tiles as the device takes them: in a plan with bands the stage-1
+// tiles write t through their maps, FP64 (an FP32 slot between a band's sum
+// and its leaf's factor scales made sums above FLT_MAX infinite).
 std::vector<TileDesc> launch_list(const Plan &P, const std::vector<TileDesc> &tiles) {
   std::vector<TileDesc> l = tiles;
   if (P.t_bands)
@@ -932,7 +932,7 @@ int create_plan(Source &src, const hmvm_options *opt, hmvm_plan **out) {
 // Where the tiles of one launch store their rows: the slots, and for
 // stage-1 tiles with a row map the plan's t.
 TileOut tile_out(const hmvm_plan *p, void *out, void *tout) {
-  return TileOut{out, p->d_tmap, tout, p->d_mscale, p->plan.t_bands ? 1 : 0};
+  return TileOut{out, p->d_tmap, tout, p->d_mscale};
 }
 
 // kind: unused by the one-wave-per-tile launch (kept so every launch names
@@ -1428,7 +1428,7 @@ int persist_prepare(hmvm_plan *p) {
   p->persist_key = -1;
   std::vector<TileDesc> ta, tb;
   std::vector<int32_t> pa, pb;
-  deal_tiles(p->plan.tiles_a, tile_costs(p, 0), nw, &ta, &pa);
+  deal_tiles(launch_list(p->plan, p->plan.tiles_a), tile_costs(p, 0), nw, &ta, &pa);
   deal_tiles(p->plan.tiles_b, tile_costs(p, 1), nw, &tb, &pb);
   int rc;
   if ((rc = upload(&p->d_ptiles_a, ta)) || (rc = upload(&p->d_ptiles_b, tb)) || (rc = upload(&p->d_pptr_a, pa)) ||
@@ -1447,7 +1447,7 @@ template <typename S, bool kScaled, int kVar>
 void launch_persistent_v(hmvm_plan *p, const double *x, double *y, int accumulate, hipStream_t st) {
   const Plan &P = p->plan;
   const size_t lds = sizeof(double) * (p->block_threads / 64) * lds_wave_doubles<S>();
-  const int n_t = P.t_fused || P.t_direct ? 0 : p->n_tsum;
+  const int n_t = P.t_fused || P.t_direct || P.t_bands ? 0 : p->n_tsum;
   hipLaunchKernelGGL((persistent_fn<S, kScaled, kVar>()), dim3(p->persist_blocks), dim3(p->block_threads), lds, st,
                      p->d_ptiles_a, p->d_pptr_a, p->d_ptiles_b, p->d_pptr_b, p->d_panels, (const S *)p->d_vals, x,
                      p->d_t, (typename SlotOf<S>::T *)p->d_slots, (const float *)p->d_scales, p->d_tmap, p->d_mscale, p->d_tfac,
