@@ -152,10 +152,11 @@ struct MultiLoads {
 // Batches whose loads are in flight at once: two (three and four cost
 // registers and instruction cache and were slower, FP64 0.56 -> 0.65 and BF16
 // 0.188 -> 0.217 ms at N=101,250 with 32 right-hand sides), one where the sums
-// leave no registers for a second.
-template <typename S, int NB>
+// leave no registers for a second (BF16 rows of y, 64 right-hand sides, four
+// row tiles: two spill 108 bytes a lane, N=50,021 143 -> 137 us with one).
+template <typename S, int NB, int NT, bool kOrdered>
 constexpr int multi_depth() {
-  return sizeof(S) >= 4 && NB == 4 ? 1 : 2;
+  return NB == 4 && (sizeof(S) >= 4 || (!kOrdered && NT == 4)) ? 1 : 2;
 }
 // How a column loop ends when its batches are not a multiple of the depth:
 // with a tail (more code), or with batches of zeros read from the zero page
@@ -184,9 +185,9 @@ constexpr bool multi_tail() {
 // 535 / 532, 64 145 / 162 and 804 / 831; FP32 64 118 / 109, 550 / 542 (FP32 sums
 // before); BF16 32 39 / 40, N=50,021 119 / 127, 64 52 / 57, 163 / 177.
 // BF16 stage 1 (kOrdered) folds a chunk at its end.
-template <typename S, int NB, bool kOrdered>
+template <typename S, int NB, int NT, bool kOrdered>
 constexpr bool multi_fold() {
-  return kOrdered || NB == 1 || (sizeof(S) < 8 && NB == 2);
+  return kOrdered || NB == 1 || (sizeof(S) < 8 && NB == 2) || (sizeof(S) != 4 && NB == 4 && NT <= 2);
 }
 
 // out += the item's columns: D batches of loads in flight, and the slices of
@@ -226,7 +227,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       xr += nrhs;
     }
   };
-  typename M::Acc part[multi_fold<S, NB, kOrdered>() ? NT : 1][NB];
+  typename M::Acc part[multi_fold<S, NB, NT, kOrdered>() ? NT : 1][NB];
   auto clear = [&]() {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -238,7 +239,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
     for (int v = 0; v < 4; ++v) o[v] += p[v];
   };
   auto fold = [&]() {
-    if constexpr (multi_fold<S, NB, kOrdered>()) {
+    if constexpr (multi_fold<S, NB, NT, kOrdered>()) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -246,7 +247,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       clear();
     }
   };
-  if constexpr (multi_fold<S, NB, kOrdered>()) clear();
+  if constexpr (multi_fold<S, NB, NT, kOrdered>()) clear();
   auto fold_all = [&]() {  // after D batches, where chunks do not say
     if constexpr (!kOrdered) fold();
   };
@@ -269,7 +270,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         } else {
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            if constexpr (multi_fold<S, NB, kOrdered>()) {
+            if constexpr (multi_fold<S, NB, NT, kOrdered>()) {
               part[t][cb] = mfma_step(l.a[t][0], b.v, part[t][cb]);
             } else {
               add(out[t][cb], mfma_step(l.a[t][0], b.v, typename M::Acc{0, 0, 0, 0}));
@@ -280,7 +281,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
       }
       if constexpr (kOrdered)
         if (__builtin_amdgcn_readfirstlane(l.end)) fold();
-    } else if constexpr (multi_fold<S, NB, kOrdered>()) {
+    } else if constexpr (multi_fold<S, NB, NT, kOrdered>()) {
 #pragma unroll
       for (int q = 0; q < KS; ++q)
 #pragma unroll
@@ -300,7 +301,7 @@ __device__ __forceinline__ void multi_columns(const MultiArgs &a, const MultiIte
         }
     }
   };
-  constexpr int D = multi_depth<S, NB>();
+  constexpr int D = multi_depth<S, NB, NT, kOrdered>();
   MultiLoads<S, NB, NT> l[D];
   MultiSlice s[D];
 #pragma unroll
