@@ -13,7 +13,8 @@ namespace hmvm {
 // type.  A lane-per-row tile's FP32 sum is stored exactly; a column-split
 // tile adds its groups' FP32 partials in FP64 and stores that sum rounded
 // once to FP32.  The segment sums that add slots into t and y accumulate in
-// FP64.  FP32 and BF16 storage thus move half the slot bytes of FP64.
+// FP64.  FP32 and BF16 storage thus move half the slot bytes of FP64.  (The
+// slots of the multi-RHS groups are FP64 in all storages.)
 template <typename S>
 struct SlotOf { using T = float; };
 template <>

@@ -182,8 +182,9 @@ constexpr bool multi_tail() {
 // the barriers between the tiles the compiler keeps several sums and spills
 // (N=101,250: FP64 32 538 -> 560, 64 830 -> 928; FP32 64 542 -> 593).
 // us, one chain / folded: FP64 32 right-hand sides N=12,007 93 / 94, N=101,250
-// 535 / 532, 64 145 / 162 and 804 / 831; FP32 64 118 / 109, 550 / 542 (FP32 sums
-// before); BF16 32 39 / 40, N=50,021 119 / 127, 64 52 / 57, 163 / 177.
+// 535 / 534, 64 146 / 157 and 809 / 838 (each fold waits for its MFMA: 18 cycles);
+// FP32 64 119 / 109, 551 / 543 (FP32 sums before); BF16 32 39 / 40, N=50,021 (leaf
+// 16) 120 / 127, 64 52 / 52, 164 / 171 (fewer waves beside FP64 sums).
 // BF16 stage 1 (kOrdered) folds a chunk at its end.
 template <typename S, int NB, int NT, bool kOrdered>
 constexpr bool multi_fold() {

@@ -154,9 +154,16 @@ struct GroupList {
 //          0.073; N=1,000: 32 rows 0.019, 16 rows 0.014; N=30,011: 32 rows
 //          0.172, 64 rows 0.167);
 //   waves  more waves a group shorten the chain of batches of each (N=1,000: 2
-//          waves 0.021, 8 waves 0.014); from 81,920 rows on there are groups
-//          enough, and fewer waves start and end less often (N=101,250: 4
-//          waves 0.552, 2 waves 0.542);
+//          waves 0.021, 8 waves 0.014); from about 80,000 rows on there are
+//          groups enough, and fewer waves start and end less often (2 / 4
+//          waves, us, 16 and 64 right-hand sides: N=60,013 FP64 272 / 261 and
+//          610 / 489, FP32 168 / 152 and 371 / 313, BF16 113 / 111 and 159 / 152;
+//          N=70,003 302 / 293 and 595 / 540, 178 / 177 and 377 / 347, 105 / 110
+//          and 171 / 177; N=82,007 337 / 331 and 627 / 605, 198 / 200 and 408 /
+//          384, 129 / 129 and 187 / 203; N=101,250 454 / 456 and 860 / 843, 267 /
+//          274 and 556 / 542, 160 / 173 and 258 / 289; N=160,003 783 / 810 and
+//          1437 / 1408, 446 / 461 and 911 / 894, 256 / 272 and 387 / 411: BF16
+//          and 16 right-hand sides gain, 64 in FP64 and FP32 lose 2 to 4%);
 //   wave_cols  one wave a stack saves the sum over the waves, but a launch of
 //          a small matrix then lasts as long as its longest stack (N=4,096,
 //          FP64, 16 right-hand sides: 256 columns 0.038, 32 columns 0.025;

@@ -32,11 +32,12 @@
 //   a0 + (s*H + q/E)*nrows*E + r*E + q%E,   E = 16 bytes, H = KS/E,
 // so a lane's KS columns of its row are one or two 16-byte words, 16 lanes
 // read 256 consecutive bytes, and a wave one contiguous stream.  Reading the
-// one-vector layout instead (columns of a whole cluster apart) fetched 1.5 to
-// 2.6 times the bytes in partly used lines, and BF16 spent more time on
-// bringing a row's columns together than on the products (N=101,250 cube, 32
-// right-hand sides: rows of y 413 / 310 / 131 us for FP64 / FP32 / BF16; with
-// the matrix loads served by the cache 274 / 227 / 77).
+// one-vector layout instead (columns of a whole cluster apart) left lines
+// partly used, and BF16 spent more time on bringing a row's columns together
+// than on the products (N=101,250 cube, 32 right-hand sides: rows of y 413 / 310
+// / 131 us for FP64 / FP32 / BF16, packed 370 / 206 / 98; HBM bytes of the packed
+// launches 1.33 and 1.48 (FP64), 1.26 and 1.38 (FP32), 1.41 and 1.43 (BF16) times
+// the matrix they read).
 #pragma once
 
 #include <cstdint>

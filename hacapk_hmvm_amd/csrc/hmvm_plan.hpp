@@ -82,9 +82,9 @@ struct TileDesc {         // 64 bytes (one scalar load)
   int32_t flags = 0;      // kTileRowPerLane: lane-per-row path even when lanes per column <= 32
   int32_t ncols = 0;      // columns of all the tile's panels together
   // >= 0: row r may go straight to t[tmap[map_off_multi + r]] (a stage-1 tile
-  // of a row group of one column chunk; the launches write its slots, which
-  // the t sum adds, or t if all stage-1 tiles are such, Plan::t_bands);
-  // map_off under t_mode 3
+  // of a row group of one column chunk): where all stage-1 tiles are such
+  // (Plan::t_bands) every launch writes t so, else its slots, which the t sum
+  // adds; map_off under t_mode 3
   int32_t map_off_multi = -1;
   // a copy of panels[panel0]: the tile's first matrix loads need nothing but
   // this descriptor

@@ -478,13 +478,15 @@ const LaunchDefaults &launch_defaults(int storage) {
 // elements and takes 6144 tiles of all elements, two per three of its slots;
 // tiles of 64 (FP64) or 96 (FP32) rows make as many of them from the large
 // clusters; BF16's take launch A's width up to 126 million elements (shorter
-// ones lost 2.5 to 4% on matrices of leaf size 16).  Measured on 14 matrices of 1 to 241 million elements against
-// one tile per slot throughout and the large matrices' rows: FP64 1.085,
-// FP32 1.070, BF16 1.021 times faster (geometric means; none slower by more
-// than 0.6%), ms per product: N=20,000 sphere FP64 0.071 -> 0.062, N=30,011
-// (leaf 64, eps 1e-6) FP64 0.159 -> 0.134 and FP32 0.089 -> 0.078, N=50,021
-// cube FP64 0.186 -> 0.165 and FP32 0.113 -> 0.094, N=60,013 (leaf 64) BF16
-// 0.087 -> 0.075.
+// ones lost 2.5 to 4% on matrices of leaf size 16).  Measured on 14 matrices of
+// 1 to 241 million elements against one tile per slot throughout and the large
+// matrices' rows, products back to back on one stream: FP64 1.085, FP32 1.070,
+// BF16 1.021 times faster (geometric means; none slower by more than 1%, BF16
+// equal below 84 million elements), us per product: N=20,000 sphere FP64 71 -> 62,
+// N=30,011 (leaf 64, eps 1e-6) FP64 144 -> 123 and FP32 89 -> 78, N=50,021 cube FP64
+// 171 -> 159, FP32 115 -> 96 and BF16 68 -> 63, N=60,013 (leaf 64) BF16 87 -> 75.
+// Products on several streams in turn hide most of a launch's end (there the
+// last is 55.6 -> 55.1).
 constexpr int64_t kKneeA[3] = {8192, 8192, 20480};  // FP64, FP32, BF16
 constexpr int64_t kBandLen[3] = {200000000, 64000000, 40000000};  // see plan_options
 struct FitWidths {
@@ -1484,7 +1486,7 @@ int launch_persistent(hmvm_plan *p, const double *x, double *y, int accumulate, 
 }
 
 // Mode 1 runs the persistent launch (any t_mode: it sums t itself when the
-// plan materialises t).
+// plan materialises t and has no bands).
 bool persistent_ok(const hmvm_plan *p) { return p->mode == 1; }
 
 // Dense tiles depend only on x and write their own output slots, so in mode 2

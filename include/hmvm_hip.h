@@ -209,15 +209,17 @@ int hmvm_plan_reset_launch(hmvm_plan *plan);
  * v_mfma_f32_16x16x32_bf16 with the vector entries rounded to BF16; the sums of
  * a few columns are added in FP64 (FP32 and BF16 storage read a copy of X in
  * their own type that the apply makes on the device).
- * hmvm_plan_reserve_multi builds the multi-RHS schedule, packs a copy of the plan's values in its order and allocates the
- * work buffers for up to nrhs columns; the apply itself allocates nothing.  The
- * copy and its schedule take 1.03 to 1.15 times the bytes of the matrix (BF16
- * storage 1.1 to 1.4 times, below 10 million elements up to 2 times, and 4 times
- * for small matrices of ranks in the hundreds); where the device lacks that
- * memory (or HMVM_MULTI_LIMIT in the environment allows the schedule, copy and
- * work buffers fewer bytes), a smaller window that every apply fills part by
- * part.  The host form reserves by itself.  d_X and d_Y need 8-byte alignment (a 16-byte-aligned d_Y
- * gets 16-byte stores) and may overlap: FP64 storage then copies d_X first. */
+ * hmvm_plan_reserve_multi builds the multi-RHS schedule, packs a copy of the
+ * plan's values in its order and allocates the work buffers for up to nrhs
+ * columns; the apply itself allocates nothing.  The copy and its schedule take
+ * 1.03 to 1.15 times the bytes of the matrix (BF16 storage 1.1 to 1.4 times,
+ * below 10 million elements up to 2 times, and 4 times for small matrices of
+ * ranks in the hundreds); where the device lacks that memory (or
+ * HMVM_MULTI_LIMIT in the environment allows the schedule, copy and work
+ * buffers fewer bytes), a smaller window that every apply fills part by part.
+ * The host form reserves by itself.  d_X and d_Y need 8-byte alignment (a
+ * 16-byte-aligned d_Y gets 16-byte stores) and may overlap: FP64 storage then
+ * copies d_X first. */
 int hmvm_plan_reserve_multi(hmvm_plan *plan, int nrhs);
 int hmvm_plan_apply_multi(hmvm_plan *plan, const double *d_X, double *d_Y, int nrhs, int accumulate, void *stream);
 int hmvm_plan_apply_multi_host(hmvm_plan *plan, const double *X, double *Y, int nrhs, int accumulate);
