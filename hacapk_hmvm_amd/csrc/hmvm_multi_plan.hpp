@@ -156,8 +156,9 @@ std::string build_multi_plan(const Plan &P, int storage, const int *nstrtl, cons
 std::string verify_multi_plan(const Plan &P, int storage, const MultiPlan &M);
 
 // For a plan that passed verify_multi_plan, element by element (4 bytes of host
-// memory each): every element of every leaf packed once, against its vector
-// entry, into its row.
+// memory each; hmvm_plan_check does it up to kMultiCheckValues): every element
+// of every leaf packed once, against its vector entry, into its row.
+constexpr int64_t kMultiCheckValues = int64_t(1) << 28;
 std::string verify_multi_values(const Plan &P, int storage, const int *nstrtl, const int *nstrtt, const MultiPlan &M);
 
 // Sizes by matrix order, see the definition.

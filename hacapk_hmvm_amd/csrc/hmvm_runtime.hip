@@ -2018,7 +2018,8 @@ int hmvm_plan_check(const matrix2 *mat2, const hmvm_options *opt, hmvm_plan_info
   err = build_multi_plan(P, po.storage, s.la.nstrtl, s.la.nstrtt, multi_options(P), &M);
   if (err != kMultiTooLarge) {
     if (err.empty()) err = verify_multi_plan(P, po.storage, M);
-    if (err.empty()) err = verify_multi_values(P, po.storage, s.la.nstrtl, s.la.nstrtt, M);
+    if (err.empty() && P.nvals <= kMultiCheckValues)
+      err = verify_multi_values(P, po.storage, s.la.nstrtl, s.la.nstrtt, M);
     if (!err.empty()) return set_error(HMVM_ERR_MATRIX, "multi-RHS schedule check failed: %s", err.c_str());
   }
   if (info) fill_info(nullptr, P, po.storage, info);
